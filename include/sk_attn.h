@@ -41,7 +41,7 @@ extern "C" {
 #define SK_API
 #endif
 
-#define SK_ABI_VERSION 7
+#define SK_ABI_VERSION 8
 
 /* Element type codes. */
 #define SK_F32 0
@@ -78,6 +78,31 @@ SK_API int sk_attn_fwd(int dtype, const void* q, const void* k, const void* v, v
                 const int64_t* q_strides, const int64_t* k_strides,
                 const int64_t* v_strides, const int64_t* o_strides,
                 int is_causal, float sm_scale, void* stream);
+
+/*
+ * Forward attention with optional key splits and rotation.
+ *
+ * sk_attn_fwd_ws is sk_attn_fwd (rope_cos and rope_sin NULL) or
+ * sk_attn_fwd_rope (both given) with scratch: where the query blocks of a call
+ * leave part of the chip idle (chunked prefill of a few rows against a long
+ * cache, short prompts of few heads) each block's keys are split over several
+ * workgroups, whose fp32 partials, normalised per split and carrying their
+ * LSE, a second kernel merges.  num_splits 0 takes the table's count when
+ * workspace_bytes holds its partials (sk_attn_fwd_workspace reports them; 0
+ * bytes: the table runs that shape unsplit) and one split otherwise; a count
+ * given explicitly needs num_splits * B*Hq*Sq * (D + 1) * 4 bytes
+ * (SK_EWORKSPACE otherwise).  workspace: device memory, 16-byte aligned, any
+ * contents.
+ */
+SK_API int sk_attn_fwd_workspace(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D,
+                          int is_causal, size_t* bytes);
+SK_API int sk_attn_fwd_ws(int dtype, const void* q, const void* k, const void* v, void* o,
+                   float* lse, void* workspace, size_t workspace_bytes, int num_splits, int B,
+                   int Hq, int Hkv, int Sq, int Sk, int D, const int64_t* q_strides,
+                   const int64_t* k_strides, const int64_t* v_strides, const int64_t* o_strides,
+                   int is_causal, const void* rope_cos, const void* rope_sin, int rope_dtype,
+                   int rope_rows, int64_t rope_stride, const int32_t* rope_pos, int rope_start,
+                   float sm_scale, void* stream);
 
 /*
  * Most bytes of dS tiles one sk_attn_bwd call uses (2 GiB), whatever the
@@ -421,16 +446,16 @@ SK_API int sk_kv_cache_update_paged_rope(int dtype, const void* k, const void* v
 #define SK_VARIANT_ROPE 2
 #define SK_VARIANT_VARLEN 4  /* decode with per-row cache lengths (the paged pool implies it) */
 
-#define SK_CFG_GRID 0           /* workgroups per launch                        */
+#define SK_CFG_GRID 0           /* workgroups per launch (forward: per key split) */
 #define SK_CFG_THREADS 1        /* threads per workgroup (64 per wavefront)     */
 #define SK_CFG_BLOCK_M 2        /* query rows per workgroup (decode: query heads) */
 #define SK_CFG_BLOCK_N 3        /* keys per tile (dK/dV: keys per workgroup)    */
 #define SK_CFG_STAGES 4         /* tile ring depth; 0 = staged in registers     */
 #define SK_CFG_HEAD_DIM 5       /* padded head dim the kernel is compiled for   */
-#define SK_CFG_SPLITS 6         /* decode key splits (1 otherwise)              */
+#define SK_CFG_SPLITS 6         /* decode, forward: key splits (1 otherwise)    */
 #define SK_CFG_PAIRED 7         /* forward: causal query blocks paired per workgroup */
 #define SK_CFG_WORKSPACE 8      /* scratch bytes the call needs                 */
-#define SK_CFG_KEYS_PER_SPLIT 9 /* decode                                       */
+#define SK_CFG_KEYS_PER_SPLIT 9 /* decode, split forward                        */
 #define SK_CFG_LDS_BYTES 10     /* device-reported, or -1                       */
 #define SK_CFG_VGPRS 11         /* device-reported registers per lane, or -1    */
 #define SK_CFG_WG_PER_CU 12     /* device-reported resident workgroups per CU, or -1 */

@@ -26,6 +26,10 @@ from stackkernels_amd._core.attention._common import (
     stream_of,
 )
 from stackkernels_amd._core.attention.layout import validate_attention_layout
+from stackkernels_amd._core.attention.workspace import fwd_workspace
+
+
+_NO_ROPE = (None, None, 0, 0, 0, None, 0)
 
 
 def flash_attn_fwd(q, k, v, is_causal: bool = False, sm_scale: float | None = None,
@@ -40,15 +44,20 @@ def flash_attn_fwd(q, k, v, is_causal: bool = False, sm_scale: float | None = No
     out = torch.empty((b, hq, sq, dk), dtype=q.dtype, device=dev)
     lse = torch.empty((b, hq, sq), dtype=torch.float32, device=dev)
     lib = _lib.load()
-    args = (_lib.dtype_code(q.dtype), qk.data_ptr(), kk.data_ptr(), vk.data_ptr(),
-            out.data_ptr(), lse.data_ptr(), b, hq, hkv, sq, sk, dk,
-            _lib.strides3(qk), _lib.strides3(kk), _lib.strides3(vk), _lib.strides3(out),
-            int(bool(is_causal)))
+    code = _lib.dtype_code(q.dtype)
+    ws = fwd_workspace(code, b, hq, hkv, sq, sk, dk, is_causal, dev)
+    ptrs = (code, qk.data_ptr(), kk.data_ptr(), vk.data_ptr(), out.data_ptr(), lse.data_ptr())
+    shape = (b, hq, hkv, sq, sk, dk, _lib.strides3(qk), _lib.strides3(kk), _lib.strides3(vk),
+             _lib.strides3(out), int(bool(is_causal)))
     with torch.cuda.device(dev):
-        if rope is None:
-            rc = lib.sk_attn_fwd(*args, scale, stream_of(dev))
+        if ws is not None:
+            rc = lib.sk_attn_fwd_ws(*ptrs, ws.data_ptr(), ws.numel(), 0, *shape,
+                                    *(_NO_ROPE if rope is None else rope.args), scale,
+                                    stream_of(dev))
+        elif rope is None:
+            rc = lib.sk_attn_fwd(*ptrs, *shape, scale, stream_of(dev))
         else:
-            rc = lib.sk_attn_fwd_rope(*args, *rope.args, scale, stream_of(dev))
+            rc = lib.sk_attn_fwd_rope(*ptrs, *shape, *rope.args, scale, stream_of(dev))
     _lib.check(rc, "flash_attn_fwd")
     if dk != d:
         out = out[..., :d].contiguous()

@@ -3,7 +3,7 @@
 The reference allocates its scratch in the launchers
 (``src/stackkernels/_opt/memory/workspace.py:6-46``: LSE, delta and the
 split-KV partials as separate float32 tensors).  Here the library sizes one
-byte buffer per call (``sk_attn_bwd_workspace``, ``sk_decode_plan`` /
+byte buffer per call (``sk_attn_fwd_workspace``, ``sk_attn_bwd_workspace``, ``sk_decode_plan`` /
 ``sk_decode_workspace``) and never allocates; these helpers take that buffer
 from torch's caching allocator.  The launchers use them, and callers that bind
 the library directly can too.
@@ -12,10 +12,34 @@ the library directly can too.
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import torch
 
 from stackkernels_amd._core.attention import _lib
+
+
+@functools.lru_cache(maxsize=512)
+def _fwd_workspace_bytes(code: int, B: int, Hq: int, Hkv: int, Sq: int, Sk: int, D: int,
+                         is_causal: bool) -> int:
+    nb = ctypes.c_size_t(0)
+    _lib.check(_lib.load().sk_attn_fwd_workspace(code, B, Hq, Hkv, Sq, Sk, D, int(is_causal),
+                                                 ctypes.byref(nb)), "flash_attn_fwd")
+    return nb.value
+
+
+def fwd_workspace(code: int, B: int, Hq: int, Hkv: int, Sq: int, Sk: int, D: int,
+                  is_causal: bool, device) -> torch.Tensor | None:
+    """uint8 scratch for ``sk_attn_fwd_ws`` (code: the library's dtype code, D:
+    the kernel head dim), or None where the forward runs unsplit: the table's choice for the shape, or no
+    room for the partials (the same call, slower)."""
+    nb = _fwd_workspace_bytes(code, B, Hq, Hkv, Sq, Sk, D, is_causal)
+    if nb == 0:
+        return None
+    try:
+        return torch.empty(nb, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
 
 
 def bwd_workspace(dtype: torch.dtype, B: int, Hq: int, Hkv: int, Sq: int, Sk: int, D: int,
@@ -63,4 +87,4 @@ def decode_workspace(dtype: torch.dtype, B: int, Hq: int, Hkv: int, Sk: int, D: 
     return torch.empty(max(nb.value, 16), dtype=torch.uint8, device=device), int(num_splits)
 
 
-__all__ = ["bwd_workspace", "decode_workspace"]
+__all__ = ["fwd_workspace", "bwd_workspace", "decode_workspace"]

@@ -157,6 +157,9 @@ def pick(
         kernels.append(k)
         config = _public(k)
         config["paired_causal_blocks"] = bool(k["paired"])
+        # key splits of a small grid, each with a grid of its own; its scratch
+        config["SPLIT_KV"] = k["splits"]
+        config["workspace_bytes"] = k["workspace_bytes"]
     elif op_name in _BWD_OPS:
         dkv = kernel_config(_OP_BWD_DKV, code, prob, 0, 0, query)
         dq = kernel_config(_OP_BWD_DQ, code, prob, 0, 0, query)

@@ -192,7 +192,23 @@ static int fwd_shape(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D, i
                   (int64_t)((p->n_mblocks + 1) / 2) * B * Hq >=
                       sk::fwd_pair_min(dtype, D, (int64_t)B * Hq, Sq, Sk, is_causal != 0);
   p->n_items = p->pair_items ? (p->n_mblocks + 1) / 2 : p->n_mblocks;
+  p->n_splits = 1;
   return SK_OK;
+}
+
+// Bytes of the split forward's partials (per split and query row, D fp32
+// values and an LSE), 0 for one split.
+static size_t fwd_ws_bytes(int B, int Hq, int Sq, int D, int splits) {
+  if (splits <= 1) return 0;
+  return (size_t)splits * B * Hq * Sq * (D + 1) * sizeof(float);
+}
+
+// Splits a forward call runs with: the table's where the workspace holds
+// their partials, else one.
+static int fwd_splits(int dtype, int B, int Hq, int Sq, int Sk, int D, bool causal,
+                      size_t workspace_bytes) {
+  const int ns = sk::fwd_key_splits(dtype, D, (int64_t)B * Hq, Sq, Sk, causal);
+  return fwd_ws_bytes(B, Hq, Sq, D, ns) <= workspace_bytes ? ns : 1;
 }
 
 // Split count and keys per split of a decode call (num_splits 0: the gfx950
@@ -209,8 +225,9 @@ static int decode_splits(int dtype, int B, int Hq, int Hkv, int Sk, int D, bool 
   return SK_OK;
 }
 
-// sk_attn_fwd and sk_attn_fwd_rope.
+// sk_attn_fwd, sk_attn_fwd_rope (no workspace: one split) and sk_attn_fwd_ws.
 static int fwd_impl(int dtype, const void* q, const void* k, const void* v, void* o, float* lse,
+                    void* workspace, size_t workspace_bytes, int num_splits,
                     int B, int Hq, int Hkv, int Sq, int Sk, int D, const int64_t* q_strides,
                     const int64_t* k_strides, const int64_t* v_strides,
                     const int64_t* o_strides, int is_causal, const sk::RopeParams& rope,
@@ -224,6 +241,7 @@ static int fwd_impl(int dtype, const void* q, const void* k, const void* v, void
   if ((rc = check_ptr("q", q)) || (rc = check_ptr("o", o)) || (rc = check_ptr("lse", lse)))
     return rc;
   if (Sk > 0 && ((rc = check_ptr("k", k)) || (rc = check_ptr("v", v)))) return rc;
+  if (workspace_bytes > 0 && (rc = check_ptr("workspace", workspace))) return rc;
 
   sk::FwdParams p{};
   p.q = q;
@@ -240,6 +258,29 @@ static int fwd_impl(int dtype, const void* q, const void* k, const void* v, void
   const bool neg = sm_scale < 0.f;
   if ((rc = fwd_shape(dtype, B, Hq, Hkv, Sq, Sk, D, is_causal, &p))) return rc;
   p.rope = rope;
+  int splits = num_splits;
+  if (splits == 0) {
+    splits = fwd_splits(dtype, B, Hq, Sq, Sk, D, is_causal != 0, workspace_bytes);
+  } else if (splits > 1) {
+    if (dtype == SK_F32) splits = 1;
+    const int keys = sk::fwd_split_keys(Sk, splits);
+    splits = keys > 0 ? (Sk + keys - 1) / keys : 1;
+    const size_t need = fwd_ws_bytes(B, Hq, Sq, D, splits);
+    if (need > workspace_bytes)
+      return fail(SK_EWORKSPACE, "workspace of %zu bytes given, %zu needed", workspace_bytes, need);
+  }
+  if (splits > 1) {
+    // One query block per workgroup and split (pairing evens out the causal
+    // triangle on full grids only).
+    p.pair_items = 0;
+    p.n_items = p.n_mblocks;
+    p.n_splits = splits;
+    p.split_keys = sk::fwd_split_keys(Sk, splits);
+    p.part_o = (float*)workspace;
+    p.part_lse = p.part_o + (size_t)splits * B * Hq * Sq * D;
+    if ((int64_t)p.n_items * B * Hq * splits > 0x7fffffffLL)
+      return fail(SK_EINVAL, "grid too large");
+  }
   hipStream_t s = (hipStream_t)stream;
   hipError_t e;
   if (dtype == SK_F32) {
@@ -249,6 +290,7 @@ static int fwd_impl(int dtype, const void* q, const void* k, const void* v, void
     p.q_sign = neg ? 0x80008000u : 0u;
     e = sk::launch_fwd_mfma(dtype, p, is_causal != 0, s);
   }
+  if (e == hipSuccess && p.n_splits > 1) e = sk::launch_fwd_combine(dtype, p, s);
   if (e != hipSuccess) return hip_fail(e, "sk_attn_fwd launch");
   return SK_OK;
 }
@@ -260,8 +302,40 @@ int sk_attn_fwd(int dtype, const void* q, const void* k, const void* v, void* o,
                 const int64_t* k_strides, const int64_t* v_strides, const int64_t* o_strides,
                 int is_causal, float sm_scale, void* stream) {
   g_err[0] = 0;
-  return fwd_impl(dtype, q, k, v, o, lse, B, Hq, Hkv, Sq, Sk, D, q_strides, k_strides, v_strides,
-                  o_strides, is_causal, sk::RopeParams{}, sm_scale, stream);
+  return fwd_impl(dtype, q, k, v, o, lse, nullptr, 0, 1, B, Hq, Hkv, Sq, Sk, D, q_strides,
+                  k_strides, v_strides, o_strides, is_causal, sk::RopeParams{}, sm_scale, stream);
+}
+
+int sk_attn_fwd_workspace(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D, int is_causal,
+                          size_t* bytes) {
+  g_err[0] = 0;
+  int rc = check_dims(dtype, B, Hq, Hkv, Sq, Sk, D);
+  if (rc) return rc;
+  if (!bytes) return fail(SK_EINVAL, "bytes pointer is NULL");
+  *bytes = fwd_ws_bytes(B, Hq, Sq, D,
+                        sk::fwd_key_splits(dtype, D, (int64_t)B * Hq, Sq, Sk, is_causal != 0));
+  return SK_OK;
+}
+
+int sk_attn_fwd_ws(int dtype, const void* q, const void* k, const void* v, void* o, float* lse,
+                   void* workspace, size_t workspace_bytes, int num_splits, int B, int Hq,
+                   int Hkv, int Sq, int Sk, int D, const int64_t* q_strides,
+                   const int64_t* k_strides, const int64_t* v_strides, const int64_t* o_strides,
+                   int is_causal, const void* rope_cos, const void* rope_sin, int rope_dtype,
+                   int rope_rows, int64_t rope_stride, const int32_t* rope_pos, int rope_start,
+                   float sm_scale, void* stream) {
+  g_err[0] = 0;
+  if (num_splits < 0 || num_splits > 1024)
+    return fail(SK_EINVAL, "num_splits=%d outside [0, 1024]", num_splits);
+  sk::RopeParams r{};
+  if (rope_cos || rope_sin) {
+    const int rc = make_rope(rope_cos, rope_sin, rope_dtype, rope_rows, rope_stride, rope_pos,
+                             rope_start, D, (int64_t)B * Hq > 0 ? Sq : 0, &r);
+    if (rc) return rc;
+  }
+  return fwd_impl(dtype, q, k, v, o, lse, workspace, workspace_bytes, num_splits, B, Hq, Hkv, Sq,
+                  Sk, D, q_strides, k_strides, v_strides, o_strides, is_causal, r, sm_scale,
+                  stream);
 }
 
 int sk_attn_fwd_rope(int dtype, const void* q, const void* k, const void* v, void* o, float* lse,
@@ -275,8 +349,8 @@ int sk_attn_fwd_rope(int dtype, const void* q, const void* k, const void* v, voi
   const int rc = make_rope(rope_cos, rope_sin, rope_dtype, rope_rows, rope_stride, rope_pos,
                            rope_start, D, (int64_t)B * Hq > 0 ? Sq : 0, &r);
   if (rc) return rc;
-  return fwd_impl(dtype, q, k, v, o, lse, B, Hq, Hkv, Sq, Sk, D, q_strides, k_strides, v_strides,
-                  o_strides, is_causal, r, sm_scale, stream);
+  return fwd_impl(dtype, q, k, v, o, lse, nullptr, 0, 1, B, Hq, Hkv, Sq, Sk, D, q_strides,
+                  k_strides, v_strides, o_strides, is_causal, r, sm_scale, stream);
 }
 
 int sk_attn_bwd_workspace(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D, int is_causal,
@@ -883,7 +957,13 @@ int sk_kernel_config(int op, int dtype, int B, int Hq, int Hkv, int Sq, int Sk, 
     k = dtype == SK_F32 ? sk::plan_fwd_f32(p, !decode && is_causal)
                         : sk::plan_fwd_mfma(dtype, p, is_causal != 0);
     paired = p.pair_items;
-    if (decode) ws = decode_ws_bytes(dtype, B, Hq, D, 1);
+    if (decode) {
+      ws = decode_ws_bytes(dtype, B, Hq, D, 1);
+    } else {
+      splits = sk::fwd_key_splits(dtype, D, (int64_t)B * Hq, Sq, Sk, is_causal != 0);
+      if (splits > 1) kps = sk::fwd_split_keys(Sk, (int)splits);
+      ws = fwd_ws_bytes(B, Hq, Sq, D, (int)splits);
+    }
   } else if (op == SK_OP_BWD_DKV || op == SK_OP_BWD_DQ) {
     sk::BwdParams p{};
     p.B = B, p.Hq = Hq, p.Hkv = Hkv, p.Sq = Sq, p.Sk = Sk, p.D = D, p.group = Hq / Hkv;

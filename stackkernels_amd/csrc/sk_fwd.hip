@@ -54,6 +54,7 @@
 //   workgroup runs query blocks j and n-1-j back to back when the grid
 //   stays at two or more workgroups per CU, which evens out the work per
 //   workgroup and halves the per-item fixed cost.
+#include <algorithm>
 #include <type_traits>
 
 #include "sk_common.h"
@@ -134,16 +135,27 @@ __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
   // pairs them (causal), blocks j and n_mblocks-1-j run back to back, so every
   // workgroup carries the same causal work and the per-item fixed cost is
   // paid half as often.
+  // With key splits the item's splits are neighbours, so the query blocks of a
+  // head that read one key range run side by side.
   const int w = xcd_work_index(blockIdx.x, gridDim.x);
-  const int bh = w / p.n_items;
-  const int item = w - bh * p.n_items;
+  const int ns = max(1, p.n_splits);
+  const int iw = w / ns;
+  const int split = w - iw * ns;
+  const int bh = iw / p.n_items;
+  const int item = iw - bh * p.n_items;
   const int b = bh / p.Hq;
   const int hq = bh % p.Hq;
   const int hkv = hq / p.group;
-  const int diag = p.Sk - p.Sq;  // causal offset
+  // The split's keys: sk of them from n_lo, numbered from 0 below (so query i
+  // sees key j of them iff j <= i + diag).
+  const int n_lo = split * p.split_keys;
+  const int sk = ns > 1 ? min(p.split_keys, p.Sk - n_lo) : p.Sk;
+  const int diag = p.Sk - p.Sq - n_lo;
 
-  const uint16_t* kbase = (const uint16_t*)p.k + b * p.k_sb + hkv * p.k_sh;
-  const uint16_t* vbase = (const uint16_t*)p.v + b * p.v_sb + hkv * p.v_sh;
+  const uint16_t* kbase =
+      (const uint16_t*)p.k + b * p.k_sb + hkv * p.k_sh + (int64_t)n_lo * p.k_ss;
+  const uint16_t* vbase =
+      (const uint16_t*)p.v + b * p.v_sb + hkv * p.v_sh + (int64_t)n_lo * p.v_ss;
   const uint32_t lds0 = lds_addr(smem);
 
   // Per-lane global byte offsets of the chunks this lane loads (tile-relative).
@@ -181,8 +193,8 @@ __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
   const int m0 = mblk * BM;
   const int mw = m0 + wave * 32;
   const int row = mw + l32;
-  int n_end = p.Sk;
-  if (CAUSAL) n_end = min(p.Sk, m0 + BM + diag);
+  int n_end = sk;
+  if (CAUSAL) n_end = min(sk, m0 + BM + diag);
   const int n_tiles = n_end > 0 ? (n_end + BN - 1) / BN : 0;
 
   // Q^T operand: lane holds q[row][16*s + 8*hl .. +7] (zero past S_q and D).
@@ -224,7 +236,7 @@ __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
   const uint16_t* iss_k = kbase;
   const uint16_t* iss_v = vbase;
   auto issue_k = [&](int stg) {
-    const int bytes = tile_bytes(max(0, min(BN, p.Sk - k_n0)), p.k_ss, p.D);
+    const int bytes = tile_bytes(max(0, min(BN, sk - k_n0)), p.k_ss, p.D);
     const i32x4 kr = make_rsrc_words(iss_k, bytes);
 #pragma unroll
     for (int j = 0; j < LK; ++j)
@@ -233,7 +245,7 @@ __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
     iss_k += (int64_t)BN * p.k_ss;
   };
   auto issue_v = [&](int stg) {
-    const int bytes = tile_bytes(max(0, min(BN, p.Sk - v_n0)), p.v_ss, p.D);
+    const int bytes = tile_bytes(max(0, min(BN, sk - v_n0)), p.v_ss, p.D);
     const i32x4 vr = make_rsrc_words(iss_v, bytes);
 #pragma unroll
     for (int j = 0; j < LK; ++j)
@@ -286,10 +298,10 @@ __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
   // Mask tile t's scores where needed; returns the tile's row maximum.
   auto mask_max = [&](int t, f32x16 (&sc)[KB]) {
     const int n0 = t * BN;
-    const bool tail = n0 + BN > p.Sk;
+    const bool tail = n0 + BN > sk;
     const bool straddle = CAUSAL && (n0 + BN - 1 > mw + diag);
     if (tail || straddle) {
-      int lim = p.Sk - 1;
+      int lim = sk - 1;
       if (CAUSAL) lim = min(lim, row + diag);
       // Element offset o (32*kb + 8*(r/4) + r%4) is masked iff o > lim - n0 - 4*hl.
       // keep = all-ones iff visible; one bitfield insert per element selects
@@ -452,7 +464,7 @@ __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
   f32x16 s0[KB], s1[KB];
   auto masked = [&](int t) {
     const int n0 = t * BN;
-    return n0 + BN > p.Sk || (CAUSAL && (n0 + BN - 1 > mw + diag));
+    return n0 + BN > sk || (CAUSAL && (n0 + BN - 1 > mw + diag));
   };
   auto barrier_issue = [&](int k, int u_k) {  // before body k; u_k = k % 4
     if constexpr (kSync == 2) {
@@ -554,7 +566,32 @@ __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
   }
 
   const float l_tot = xhalf_sum(l_run);
-  if (row < p.Sq) {
+  if (ns > 1) {
+    // A split's partial: a row that saw no key leaves its output unwritten
+    // (the combine skips it); a NaN row keeps its NaN.
+    if (row < p.Sq) {
+      const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+      const int64_t rows = (int64_t)p.B * p.Hq * p.Sq;
+      const int64_t r = split * rows + (int64_t)bh * p.Sq + row;
+      if (l_tot != 0.f) {
+        float* po = p.part_o + r * p.D;
+#pragma unroll
+        for (int c = 0; c < DB; ++c)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int d = 32 * c + 8 * i + 4 * hl;
+            if (d < p.D)
+              *reinterpret_cast<f32x4*>(po + d) =
+                  f32x4{oacc[c][4 * i] * inv, oacc[c][4 * i + 1] * inv, oacc[c][4 * i + 2] * inv,
+                        oacc[c][4 * i + 3] * inv};
+          }
+      }
+      if (hl == 0)
+        p.part_lse[r] = l_tot > 0.f    ? m_run * p.scale + __logf(l_tot)
+                        : l_tot == 0.f ? kNegInf
+                                       : l_tot;
+    }
+  } else if (row < p.Sq) {
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     uint16_t* ob = (uint16_t*)p.o + b * p.o_sb + hq * p.o_sh + (int64_t)row * p.o_ss;
 #pragma unroll
@@ -582,6 +619,60 @@ __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
     __syncthreads();  // every wave is done with the LDS ring before it is refilled
     run_item(second);
   }
+}
+
+// Merge of the key splits' partials: O = sum_s w_s O_s / sum_s w_s with
+// w_s = exp(LSE_s - max LSE), LSE = max + log(sum_s w_s).  LPR lanes per query
+// row, four head-dim values each (DQ quads per lane at D > 128), so a row's
+// loads are whole lines; a split without a key for the row (LSE -inf) is not
+// read.  Bound by the partials' HBM / L2 traffic: 33.5 MB of 4 splits at
+// B*Hq*Sq = 16,384 rows of D = 128.
+template <class T>
+__device__ __forceinline__ void store_quad(void* o, int64_t at, f32x4 v) {
+  if constexpr (__is_same(T, float)) {
+    *reinterpret_cast<f32x4*>((float*)o + at) = v;
+  } else {
+    *reinterpret_cast<u32x2*>((uint16_t*)o + at) =
+        u32x2{pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
+  }
+}
+
+template <class T, int LPR, int DQ>
+__global__ void __launch_bounds__(256) fwd_combine_kernel(FwdParams p) {
+  constexpr bool kF32 = __is_same(T, float);
+  const int64_t rows = (int64_t)p.B * p.Hq * p.Sq;
+  const int64_t r = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
+  if (r >= rows) return;
+  const int j = threadIdx.x % LPR;
+  const float* lse = p.part_lse + r;
+  float mx = kNegInf;
+  for (int s = 0; s < p.n_splits; ++s) mx = __builtin_elementwise_maximum(mx, lse[s * rows]);
+  f32x4 acc[DQ];
+#pragma unroll
+  for (int q = 0; q < DQ; ++q) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float den = 0.f;
+#pragma unroll 4
+  for (int s = 0; s < p.n_splits; ++s) {
+    const float l = lse[s * rows];
+    if (l == kNegInf) continue;
+    const float w = kF32 ? expf(l - mx) : __expf(l - mx);
+    den += w;
+#pragma unroll
+    for (int q = 0; q < DQ; ++q) {
+      const int d = 4 * (j + q * LPR);
+      if (d < p.D) acc[q] += w * *reinterpret_cast<const f32x4*>(p.part_o + (s * rows + r) * p.D + d);
+    }
+  }
+  const float inv = den > 0.f ? 1.f / den : 0.f;
+  const int bh = (int)(r / p.Sq);
+  const int row = (int)(r - (int64_t)bh * p.Sq);
+  const int64_t o0 = (bh / p.Hq) * p.o_sb + (bh % p.Hq) * p.o_sh + (int64_t)row * p.o_ss;
+#pragma unroll
+  for (int q = 0; q < DQ; ++q) {
+    const int d = 4 * (j + q * LPR);
+    if (d < p.D) store_quad<T>(p.o, o0 + d, acc[q] * inv);
+  }
+  if (j == 0) p.lse[r] = den > 0.f ? mx + (kF32 ? logf(den) : __logf(den)) : kNegInf;
 }
 
 // gfx950 tile table for the forward kernel, by head dim (padded to 64, 128
@@ -678,6 +769,50 @@ int fwd_pair_min(int dtype, int d, int64_t bh, int sq, int sk, bool causal) {
   return 256 * fwd_config(d, bh, sq, sk, causal).occ * SK_FWD_PAIR_ROUNDS;
 }
 
+// Key splits of a forward whose query blocks leave CUs idle (chunked prefill,
+// a few query rows against a long cache).  The count minimises a model of the
+// call's microseconds fitted to sweeps of 1 to 32 splits: the most loaded
+// CU's workgroups (ceil(items * splits / 256)), each its share of the key
+// tiles plus two tiles' worth of prologue and epilogue, and, when split, the
+// merge (a second launch and the partials' traffic).  A tile (128 query rows
+// x BN keys) takes about 1 us at D = 128, 0.5 at D <= 64, 1.15 at D = 256 (BN
+// = 32), 5% less with two workgroups on a CU.  Measured, D = 128 bf16, H_q =
+// 32, H_kv = 8, causal, S_q x S_k, one split against the table's: 512 x
+// 16,000 236 -> 134 us (4 splits), 128 x 16,000 237 -> 50 (8), 16 x 4,096 61
+// -> 20 (8); unsplit stays at 512 x 1,024 (21 us, 27 with 2) and 1,024 x
+// 8,000 (138 us, 132 with 2), where the grid or the merge leaves no gain.
+// A predicted gain under 15% is left alone (causal squares, whose blocks
+// differ: 1,000 x 1,000 at 8 heads 20 us either way), and from 384 query
+// blocks on (1.5 per CU) nothing is split.
+int fwd_split_keys(int sk, int splits) {
+  const int per = (sk + splits - 1) / splits;
+  return (per + 63) / 64 * 64;
+}
+
+int fwd_key_splits(int dtype, int d, int64_t bh, int sq, int sk, bool causal) {
+  if (dtype != BF16::code && dtype != F16::code) return 1;
+  if (sq <= 0 || sk <= 0 || bh <= 0) return 1;
+  const FwdConfig c = fwd_config(d, bh, sq, sk, causal);
+  const int64_t items = (sq + 32 * c.nw - 1) / (32 * c.nw) * bh;
+  if (items >= 384) return 1;
+  const double tile_us = d <= 64 ? 0.5 : d <= 128 ? 1.0 : 1.15;
+  const double tiles = (double)sk / c.bn;
+  const double merge_us = (double)bh * sq * d * 8 / 1.2e7;  // per split
+  int best = 1;
+  double best_us = 0, one_us = 0;
+  for (int ns = 1; ns <= 32; ++ns) {
+    if (ns > 1 && sk < ns * 256) break;
+    const int64_t load = (items * ns + 255) / 256;
+    const double eff = load > 1 && c.occ > 1 ? 0.95 : 1.0;
+    const double us = load * eff * (tiles / ns + 2) * tile_us + (ns > 1 ? 8 + ns * merge_us : 0);
+    if (ns == 1) one_us = us;
+    if (ns == 1 || us < best_us) best = ns, best_us = us;
+  }
+  if (best_us > 0.85 * one_us) return 1;
+  const int keys = fwd_split_keys(sk, best);
+  return (sk + keys - 1) / keys;
+}
+
 template <class T, int DP, int BN, int NW, int OCC, int STAGES = 4>
 static KernelPlan plan_fwd_t(const FwdParams& p, bool causal) {
   KernelPlan k;
@@ -690,7 +825,7 @@ static KernelPlan plan_fwd_t(const FwdParams& p, bool causal) {
     k.fn = (const void*)fwd_mfma_kernel<T, DP, BN, NW, STAGES, OCC, true, true>;
   else
     k.fn = (const void*)fwd_mfma_kernel<T, DP, BN, NW, STAGES, OCC, false, true>;
-  k.grid = dim3((unsigned)(p.n_items * p.B * p.Hq));
+  k.grid = dim3((unsigned)(p.n_items * p.B * p.Hq * std::max(1, p.n_splits)));
   k.block = dim3(NW * 64);
   k.kernel = "fwd_mfma_kernel";
   k.elem = T::code;
@@ -735,6 +870,33 @@ hipError_t launch_fwd_mfma(int dtype, const FwdParams& p, bool causal, hipStream
   const KernelPlan k = plan_fwd_mfma(dtype, p, causal);
   if (!k.fn) return hipErrorInvalidValue;
   return run_plan(k, &p, s);
+}
+
+template <class T>
+static const void* combine_fn(int d) {
+  if (d <= 64) return (const void*)fwd_combine_kernel<T, 16, 1>;
+  if (d <= 128) return (const void*)fwd_combine_kernel<T, 32, 1>;
+  return (const void*)fwd_combine_kernel<T, 32, 2>;
+}
+
+KernelPlan plan_fwd_combine(int dtype, const FwdParams& p) {
+  KernelPlan k;
+  k.fn = dtype == BF16::code  ? combine_fn<BF16>(p.D)
+         : dtype == F16::code ? combine_fn<F16>(p.D)
+         : dtype == 0         ? combine_fn<float>(p.D)
+                              : nullptr;
+  const int rows_per = p.D <= 64 ? 16 : 8;
+  k.grid = dim3((unsigned)(((int64_t)p.B * p.Hq * p.Sq + rows_per - 1) / rows_per));
+  k.block = dim3(256);
+  k.kernel = "fwd_combine_kernel";
+  k.elem = dtype;
+  k.head_dim = padded_head_dim(p.D);
+  k.block_m = rows_per;
+  return k;
+}
+
+hipError_t launch_fwd_combine(int dtype, const FwdParams& p, hipStream_t s) {
+  return run_plan(plan_fwd_combine(dtype, p), &p, s);
 }
 
 hipError_t run_plan(const KernelPlan& k, const void* params, hipStream_t s) {

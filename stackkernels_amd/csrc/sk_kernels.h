@@ -59,6 +59,15 @@ struct FwdParams {
   float scale;       // |sm_scale|
   float scale_log2;  // |sm_scale| * log2(e)
   uint32_t q_sign;   // 0, or the sign-bit mask that negates q when sm_scale < 0
+  // Key splits (MFMA kernels): split s of a work item covers keys
+  // [s * split_keys, (s + 1) * split_keys), split_keys a multiple of 64.  With
+  // one split (0 and 1 both mean that) the kernel writes O and LSE; with more
+  // it writes each split's normalised output and its LSE in fp32 for
+  // fwd_combine_kernel: part_o [n_splits][B*Hq*Sq][D] (rows of a split that
+  // sees no key are not written), part_lse [n_splits][B*Hq*Sq] (-inf there).
+  int n_splits, split_keys;
+  float* part_o;
+  float* part_lse;
   // Decode only (fp32 path, non-causal): null, or per-batch-row key counts;
   // row b sees keys [0, clamp(seqlens[b], 0, Sk)).
   const int* seqlens;
@@ -239,6 +248,7 @@ hipError_t run_plan(const KernelPlan& k, const void* params, hipStream_t s);
 
 KernelPlan plan_fwd_mfma(int dtype, const FwdParams& p, bool causal);
 KernelPlan plan_fwd_f32(const FwdParams& p, bool causal);
+KernelPlan plan_fwd_combine(int dtype, const FwdParams& p);
 // Query rows per workgroup of the fp32 forward for head dim d and sq queries.
 int fwd_f32_rows_per_block(int d, int sq);
 KernelPlan plan_decode_mfma(int dtype, const DecParams& p);
@@ -256,6 +266,7 @@ KernelPlan plan_bwd_dq_f32(BwdParams& p, bool causal);
 // Launchers: return hipSuccess or the launch error.  dtype is SK_F32/F16/BF16.
 hipError_t launch_fwd_mfma(int dtype, const FwdParams& p, bool causal, hipStream_t s);
 hipError_t launch_fwd_f32(const FwdParams& p, bool causal, hipStream_t s);
+hipError_t launch_fwd_combine(int dtype, const FwdParams& p, hipStream_t s);
 hipError_t launch_decode_mfma(int dtype, const DecParams& p, hipStream_t s);
 hipError_t launch_decode_combine(int dtype, const DecParams& p, hipStream_t s);
 hipError_t launch_bwd_prep(int dtype, const BwdParams& p, hipStream_t s);
@@ -270,6 +281,10 @@ int fwd_rows_per_block(int dtype, int d, int64_t bh, int sq, int sk, bool causal
 // Fewest paired workgroups for which a causal forward of that shape pairs
 // its query blocks.
 int fwd_pair_min(int dtype, int d, int64_t bh, int sq, int sk, bool causal);
+// Key splits the forward's table takes for that shape (1: unsplit), and the
+// keys each covers.
+int fwd_key_splits(int dtype, int d, int64_t bh, int sq, int sk, bool causal);
+int fwd_split_keys(int sk, int splits);
 // Padded head dim the kernels are compiled for (64, 96, 128 or 256), or 0.
 int padded_head_dim(int d);
 
