@@ -31,9 +31,9 @@ def _fwd_workspace_bytes(code: int, B: int, Hq: int, Hkv: int, Sq: int, Sk: int,
 def fwd_workspace(code: int, B: int, Hq: int, Hkv: int, Sq: int, Sk: int, D: int,
                   is_causal: bool, device) -> torch.Tensor | None:
     """uint8 scratch for ``sk_attn_fwd_ws`` (code: the library's dtype code, D:
-    the kernel head dim), or None where the forward runs unsplit: the table's choice for the shape, or no
-    room for the partials (the same call, slower)."""
-    nb = _fwd_workspace_bytes(code, B, Hq, Hkv, Sq, Sk, D, is_causal)
+    the kernel head dim), or None where the forward runs unsplit: the table's
+    choice for the shape, or no room for the partials (the same call, slower)."""
+    nb = _fwd_workspace_bytes(code, B, Hq, Hkv, Sq, Sk, D, bool(is_causal))
     if nb == 0:
         return None
     try:

@@ -121,6 +121,23 @@ __device__ __forceinline__ int xcd_work_index(int bid, int n) {
   return xcd * per + min(xcd, rem) + r;
 }
 
+// Head and block of workgroup bid in an order by block first, for grids whose
+// low blocks are the heavy ones (causal masks): every head's heavy block
+// starts before any light one, so no long block is left to run alone at the
+// end.  Where the heads divide over the XCDs each XCD keeps its contiguous
+// range of heads (the heads that share K/V stay on one L2).
+__device__ __forceinline__ void heavy_first_order(int bid, int n_heads, int& head, int& block) {
+  if (n_heads % kNumXcd == 0) {
+    const int per = n_heads / kNumXcd;
+    const int r = bid / kNumXcd;
+    block = r / per;
+    head = (bid % kNumXcd) * per + (r - block * per);
+  } else {
+    block = bid / n_heads;
+    head = bid - block * n_heads;
+  }
+}
+
 // max / sum of a value across lanes l and l^32 of a wave64.  v_permlane32_swap
 // with both operands x leaves, in every lane l, x[l % 32] in one result and
 // x[l % 32 + 32] in the other (a VALU op, no LDS round trip).

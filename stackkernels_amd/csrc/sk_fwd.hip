@@ -53,7 +53,9 @@
 //   long rows do not trail at the end of the grid.  Under the causal mask a
 //   workgroup runs query blocks j and n-1-j back to back when the grid
 //   stays at two or more workgroups per CU, which evens out the work per
-//   workgroup and halves the per-item fixed cost.
+//   workgroup and halves the per-item fixed cost; smaller causal grids start
+//   every head's heavy blocks before any light one (bf16, H_q = 32, H_kv = 8,
+//   D = 128, B = 2, S = 1,337, 704 workgroups: 54 us head-major, 43 so).
 #include <algorithm>
 #include <type_traits>
 
@@ -141,8 +143,9 @@ __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
   const int ns = max(1, p.n_splits);
   const int iw = w / ns;
   const int split = w - iw * ns;
-  const int bh = iw / p.n_items;
-  const int item = iw - bh * p.n_items;
+  int bh = iw / p.n_items;
+  int item = iw - bh * p.n_items;
+  if (p.heavy_first) heavy_first_order(blockIdx.x, p.B * p.Hq, bh, item);
   const int b = bh / p.Hq;
   const int hq = bh % p.Hq;
   const int hkv = hq / p.group;
@@ -866,7 +869,12 @@ KernelPlan plan_fwd_mfma(int dtype, const FwdParams& p, bool causal) {
   return KernelPlan{};
 }
 
-hipError_t launch_fwd_mfma(int dtype, const FwdParams& p, bool causal, hipStream_t s) {
+hipError_t launch_fwd_mfma(int dtype, const FwdParams& params, bool causal, hipStream_t s) {
+  FwdParams p = params;
+  // Unpaired causal grids only: paired blocks carry equal work, and head-major
+  // order then keeps each head's K/V in one L2 (B * H = 128, S = 4,096 527 us,
+  // 575 with the blocks outermost).
+  p.heavy_first = causal && !p.pair_items && p.n_splits <= 1;
   const KernelPlan k = plan_fwd_mfma(dtype, p, causal);
   if (!k.fn) return hipErrorInvalidValue;
   return run_plan(k, &p, s);

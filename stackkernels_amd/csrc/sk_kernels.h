@@ -56,6 +56,7 @@ struct FwdParams {
   int n_mblocks;     // ceil(Sq / rows per workgroup)
   int n_items;       // work items per (batch, head): n_mblocks, or ceil(n_mblocks/2) if paired
   int pair_items;    // 1: item j runs query blocks n_mblocks-1-j and j
+  int heavy_first;   // 1: items in heavy_first_order (causal, unpaired, unsplit)
   float scale;       // |sm_scale|
   float scale_log2;  // |sm_scale| * log2(e)
   uint32_t q_sign;   // 0, or the sign-bit mask that negates q when sm_scale < 0
@@ -144,6 +145,8 @@ struct BwdParams {
   float abs_scale_log2;
   uint32_t op_sign;
   int n_mblocks, n_nblocks;
+  int dkv_heavy_first;  // dK/dV: key blocks outermost, pairs fastest
+  int dq_heavy_first;   // dQ: items in heavy_first_order
 };
 
 // dS tile layout of the five-GEMM backward, per query head.  The dK/dV
