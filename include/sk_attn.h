@@ -130,6 +130,16 @@ SK_API int sk_attn_bwd_workspace(int dtype, int B, int Hq, int Hkv, int Sq, int 
                           int is_causal, size_t* bytes);
 
 /*
+ * Most bytes of scratch sk_attn_bwd makes use of with these dims: the above
+ * plus, for 16-bit calls whose dK/dV workgroups leave part of the chip idle,
+ * the fp32 partial sums of a dK/dV split over the query tiles.  A call given
+ * at least this many bytes sums dK and dV in that split's order; one given
+ * less sums them in one pass per key block.
+ */
+SK_API int sk_attn_bwd_workspace_best(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D,
+                               int is_causal, size_t* bytes);
+
+/*
  * Minimum bytes of scratch for sk_attn_bwd: the two row statistics, with
  * which it runs the seven-GEMM backward.  The reference's counterpart is
  * the same delta buffer (src/stackkernels/_opt/memory/workspace.py:16-23).

@@ -47,6 +47,8 @@ SIGNATURES: dict[str, tuple] = {
                                 _i64p, _i64p, _i64p, _i64p, _c_int, *_ROPE, _c_float, _vp]),
     "sk_attn_bwd_workspace": (_c_int, [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                                        _c_int, _sizep]),
+    "sk_attn_bwd_workspace_best": (_c_int, [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
+                                            _c_int, _c_int, _sizep]),
     "sk_attn_bwd_workspace_min": (_c_int, [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                                            _c_int, _c_int, _sizep]),
     "sk_attn_bwd": (_c_int, [_c_int, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,

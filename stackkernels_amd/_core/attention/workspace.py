@@ -46,24 +46,29 @@ def bwd_workspace(dtype: torch.dtype, B: int, Hq: int, Hkv: int, Sq: int, Sk: in
                   is_causal: bool, device) -> torch.Tensor:
     """uint8 scratch for ``sk_attn_bwd`` (D: the kernel head dim; at least 16 bytes).
 
-    The library's preferred size (row statistics plus one chunk of the
-    five-GEMM backward's dS tiles, at most ``SK_BWD_DS_CAP_BYTES`` of them);
-    if torch cannot allocate that, the minimum (row statistics only), with
-    which the call runs the seven-GEMM backward: the same results, slower.
+    The most the call makes use of (``sk_attn_bwd_workspace_best``: row
+    statistics, one chunk of the five-GEMM backward's dS tiles, at most
+    ``SK_BWD_DS_CAP_BYTES`` of them, and the partial sums of a split dK/dV);
+    if torch cannot allocate that, the size without the partial sums, then
+    the minimum (row statistics only), with which the call runs the
+    seven-GEMM backward: slower, and dK/dV summed in another order than a
+    split one sums them.
     """
     lib = _lib.load()
-    code = _lib.dtype_code(dtype)
-    args = (code, B, Hq, Hkv, Sq, Sk, D, int(bool(is_causal)))
+    args = (_lib.dtype_code(dtype), B, Hq, Hkv, Sq, Sk, D, int(bool(is_causal)))
     nb = ctypes.c_size_t(0)
-    _lib.check(lib.sk_attn_bwd_workspace(*args, ctypes.byref(nb)), "flash_attn_bwd")
-    nmin = ctypes.c_size_t(0)
-    _lib.check(lib.sk_attn_bwd_workspace_min(*args, ctypes.byref(nmin)), "flash_attn_bwd")
-    try:
-        return torch.empty(max(nb.value, 16), dtype=torch.uint8, device=device)
-    except torch.OutOfMemoryError:
-        if nb.value <= nmin.value:
-            raise
-    return torch.empty(max(nmin.value, 16), dtype=torch.uint8, device=device)
+    tried = -1
+    for fn in (lib.sk_attn_bwd_workspace_best, lib.sk_attn_bwd_workspace):
+        _lib.check(fn(*args, ctypes.byref(nb)), "flash_attn_bwd")
+        if nb.value == tried:
+            continue
+        tried = nb.value
+        try:
+            return torch.empty(max(nb.value, 16), dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            pass
+    _lib.check(lib.sk_attn_bwd_workspace_min(*args, ctypes.byref(nb)), "flash_attn_bwd")
+    return torch.empty(max(nb.value, 16), dtype=torch.uint8, device=device)
 
 
 def decode_workspace(dtype: torch.dtype, B: int, Hq: int, Hkv: int, Sk: int, D: int, device,

@@ -167,6 +167,25 @@ size_t bwd_ws_bytes(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D, bo
   return bwd_rows_bytes(B, Hq, Sq) + (size_t)chunk * pair;
 }
 
+// Offset of the split dK/dV's partial sums in the workspace, and their bytes
+// (0: the shape runs unsplit, or its pairs in several chunks).
+struct DkvParts {
+  size_t offset = 0, bytes = 0;
+  int iters = 0, chunks = 1;
+};
+DkvParts bwd_parts(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D, bool causal) {
+  DkvParts r;
+  sk::bwd_dkv_split(dtype, B, Hq, Hkv, Sq, Sk, D, causal, &r.iters, &r.chunks);
+  const size_t pair = sk::bwd_ds_pair_bytes(dtype, Hq, Hkv, Sq, Sk, D, causal);
+  const int64_t pairs = (int64_t)B * Hkv;
+  if (r.iters <= 0 ||
+      (pair > 0 && bwd_chunk_pairs(pairs, pair, (size_t)SK_BWD_DS_CAP_BYTES) != pairs))
+    return DkvParts{};
+  r.offset = (bwd_ws_bytes(dtype, B, Hq, Hkv, Sq, Sk, D, causal) + 255) / 256 * 256;
+  r.bytes = (size_t)2 * r.chunks * pairs * Sk * D * sizeof(float);
+  return r;
+}
+
 }  // namespace
 
 extern "C" {
@@ -363,6 +382,15 @@ int sk_attn_bwd_workspace(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int
   return SK_OK;
 }
 
+int sk_attn_bwd_workspace_best(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D,
+                               int is_causal, size_t* bytes) {
+  const int rc = sk_attn_bwd_workspace(dtype, B, Hq, Hkv, Sq, Sk, D, is_causal, bytes);
+  if (rc) return rc;
+  const DkvParts parts = bwd_parts(dtype, B, Hq, Hkv, Sq, Sk, D, is_causal != 0);
+  if (parts.bytes > 0) *bytes = parts.offset + parts.bytes;
+  return SK_OK;
+}
+
 int sk_attn_bwd_workspace_min(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D,
                               int is_causal, size_t* bytes) {
   g_err[0] = 0;
@@ -413,6 +441,14 @@ int sk_attn_bwd(int dtype, const void* dout, const void* q, const void* k, const
   p.ds = chunk > 0 ? (char*)workspace + need : nullptr;
   p.n_pairs = (int)chunk;
   p.bk0 = 0;
+  // Split dK/dV where the workspace holds its partial sums as well.
+  const DkvParts parts = bwd_parts(dtype, B, Hq, Hkv, Sq, Sk, D, is_causal != 0);
+  if (parts.bytes > 0 && workspace_bytes >= parts.offset + parts.bytes) {
+    p.kv_iters = parts.iters;
+    p.kv_chunks = parts.chunks;
+    p.part_dk = (float*)((char*)workspace + parts.offset);
+    p.part_dv = p.part_dk + (size_t)parts.chunks * B * Hkv * Sk * D;
+  }
   p.ds_nqt = (Sq + 31) / 32;
   p.ds_c = sk::ds_causal_c(Sq, Sk);
   p.ds_head_tiles = sk::ds_head_tiles((Sk + 127) / 128, p.ds_nqt, p.ds_c, is_causal != 0);

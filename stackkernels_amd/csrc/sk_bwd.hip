@@ -51,6 +51,7 @@
 // dP^T = V dO^T give one query per lane, and dQ^T += K^T dS^T reads K^T
 // transposed from the ring.
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 
 #include "sk_common.h"
@@ -210,11 +211,16 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv_kernel(BwdParams p) {
 
   // Work item: (batch, KV head) major, then key block (lowest first: under
   // the causal mask it sees the most queries), then head-dim half.
+  // A split launch goes chunk by chunk, pairs fastest: the pairs spread over
+  // the XCDs (a pair's workgroups stay on one where the pairs are a multiple
+  // of 8) and every XCD gets its share of a causal triangle.
   const int per_head = p.n_nblocks * kDSplit;
-  int bkl, rem;
-  if (p.dkv_heavy_first) {
-    rem = blockIdx.x / p.n_pairs;
-    bkl = blockIdx.x - rem * p.n_pairs;
+  int bkl, rem, chunk = 0;
+  if (p.kv_iters > 0 || p.dkv_heavy_first) {
+    const int idx = blockIdx.x / p.n_pairs;
+    bkl = blockIdx.x - idx * p.n_pairs;
+    chunk = idx / per_head;
+    rem = idx - chunk * per_head;
   } else {
     const int w = xcd_work_index(blockIdx.x, gridDim.x);
     bkl = w / per_head;  // pair within this launch
@@ -230,6 +236,21 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv_kernel(BwdParams p) {
   const int key = nw + l32;
   const int diag = p.Sk - p.Sq;
   const int d_out0 = dsp * DO;
+
+  // Query tiles that can see a key of this block (i >= n0 - diag), of every
+  // head of the group, and this workgroup's share of them.
+  const int m_begin = dkv_first_query(nblk, p.Sq, p.Sk, CAUSAL);
+  const int n_mt = dkv_tiles(nblk, p.Sq, p.Sk, CAUSAL);
+  int n_it = p.group * n_mt, it0 = 0, n_chunks = 1;
+  if (p.kv_iters > 0) {
+    n_chunks = dkv_chunks(n_it, p.kv_iters);
+    if (chunk >= n_chunks) return;
+    const int per = (n_it + n_chunks - 1) / n_chunks;
+    it0 = min(chunk * per, n_it);
+    n_it = min(per, n_it - it0);
+  }
+  const int gi0 = n_mt > 0 ? it0 / n_mt : 0;         // first tile: head of the group ...
+  const int m_first = m_begin + (it0 - gi0 * n_mt) * BMQ;  // ... and query
 
   // Resident B operand, rows of this lane's key: K (sign-flipped for a
   // negative scale) for role 0, V for role 1: x[key][16*s + 8*hl .. +7].
@@ -249,12 +270,6 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv_kernel(BwdParams p) {
     }
   }
 
-  // Query tiles that can see a key of this block: i >= n0 - diag.
-  int m_begin = 0;
-  if (CAUSAL) m_begin = max(0, n0 - diag) / BMQ * BMQ;
-  const int n_mt = m_begin < p.Sq ? (p.Sq - m_begin + BMQ - 1) / BMQ : 0;
-  const int n_it = p.group * n_mt;
-
   // DMA: segment j of this wave is segment wave + 8j of the tile pair (Q
   // segments first, then dO); its LDS target and lane source offsets.
   uint32_t goff[LS];
@@ -267,8 +282,8 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv_kernel(BwdParams p) {
   }
   // Issue cursor: query head, first row, and that row's index in [B*Hq*Sq].
   const int64_t bh0 = (int64_t)b * p.Hq + hkv * p.group;
-  int iss_gi = 0, iss_m0 = m_begin;
-  int64_t iss_row = bh0 * p.Sq + m_begin;
+  int iss_gi = gi0, iss_m0 = m_first;
+  int64_t iss_row = (bh0 + gi0) * p.Sq + m_first;
   const float* stat_src = role == 0 ? p.lse_log2 : p.delta;  // role 0: lse*log2e
   const uint32_t lds0 = lds_addr(smem);
   auto issue = [&](int stg) {
@@ -359,7 +374,7 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv_kernel(BwdParams p) {
 
   // Role 0, tile in stage stg (P buffer pb): S, causal mask, P =
   // exp2(S*scale*log2e - lse*log2e), published for role 1, dV^T += dO^T P.
-  int cur_gi = 0, cur_m0 = m_begin;  // role 0's tile
+  int cur_gi = gi0, cur_m0 = m_first;  // role 0's tile
   // Five-GEMM backward: role 1 stores each tile's dS (32 keys x 32 queries,
   // 16-bit) for the dQ kernel.  A lane holds key l32 and, as pieces of 4
   // queries, P_m = queries 8 m + 4 hl + {0..3}: P_0, P_1 = g[0].xy, .zw and
@@ -373,7 +388,7 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv_kernel(BwdParams p) {
   // zero K rows would turn into NaN).  Tile (query head, key tile, query
   // tile) sits where the dS tile layout (DsLayout) puts it, counted from the
   // launch's first pair.
-  int ds_gi = 0, ds_m0 = m_begin;  // role 1's dS tile
+  int ds_gi = gi0, ds_m0 = m_first;  // role 1's dS tile
   const int64_t ds_t0 =
       (int64_t)bkl * p.group * p.ds_head_tiles + 4 * ds_off(nblk, p.ds_nqt, p.ds_c, CAUSAL) +
       (int64_t)kg * ds_cnt(nblk, p.ds_nqt, p.ds_c, CAUSAL) - ds_qb(nblk, p.ds_c, CAUSAL);
@@ -836,6 +851,20 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv_kernel(BwdParams p) {
   const float osc = role == 0 ? 1.f : p.scale;
   if (key >= p.Sk) return;
   const int64_t krow = ((int64_t)bk * p.Sk + key) * p.D;
+  if (n_chunks > 1) {
+    float* po = (role == 0 ? p.part_dv : p.part_dk) +
+                (int64_t)chunk * p.B * p.Hkv * p.Sk * p.D + krow;
+#pragma unroll
+    for (int c = 0; c < DB; ++c)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int d = d_out0 + 32 * c + 8 * i + 4 * hl;
+        if (d < p.D)
+          *reinterpret_cast<f32x4*>(po + d) =
+              f32x4{acc[c][4 * i], acc[c][4 * i + 1], acc[c][4 * i + 2], acc[c][4 * i + 3]};
+      }
+    return;
+  }
   uint16_t* outp = (uint16_t*)(role == 0 ? p.dv : p.dk) + krow;
 #pragma unroll
   for (int c = 0; c < DB; ++c)
@@ -849,6 +878,32 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv_kernel(BwdParams p) {
                   pack2<T>(a[4 * i + 2] * osc, a[4 * i + 3] * osc)};
       }
     }
+}
+
+// Sum of a split dK/dV's partials in chunk order: dK = scale * sum, dV = sum,
+// rounded once to the output type.  One thread per four head-dim values of a
+// key row; blockIdx.y 0: dK, 1: dV.  Key blocks of one chunk are left as the
+// dK/dV kernel wrote them.  Bound by the partials' traffic.
+template <class T>
+__global__ void __launch_bounds__(256) bwd_dkv_reduce_kernel(BwdParams p, bool causal) {
+  const int quads = p.D / 4;
+  const int64_t n = (int64_t)p.B * p.Hkv * p.Sk;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t row = i / quads;
+  if (row >= n) return;
+  const int key = (int)(row % p.Sk);
+  const int chunks =
+      dkv_chunks(p.group * dkv_tiles(key >> 7, p.Sq, p.Sk, causal), p.kv_iters);
+  if (chunks <= 1) return;
+  const bool is_dv = blockIdx.y != 0;
+  const int64_t at = row * p.D + (i - row * quads) * 4;
+  const float* src = (is_dv ? p.part_dv : p.part_dk) + at;
+  f32x4 x = *reinterpret_cast<const f32x4*>(src);
+#pragma unroll 4
+  for (int c = 1; c < chunks; ++c) x += *reinterpret_cast<const f32x4*>(src + c * n * p.D);
+  if (!is_dv) x *= p.scale;
+  *reinterpret_cast<u32x2*>((uint16_t*)(is_dv ? p.dv : p.dk) + at) =
+      u32x2{pack2<T>(x[0], x[1]), pack2<T>(x[2], x[3])};
 }
 
 // ---------------------------------------------------------------------------
@@ -1438,7 +1493,8 @@ static KernelPlan plan_dkv_t(BwdParams& p, bool causal) {
   KernelPlan k;
   k.fn = causal ? (const void*)bwd_dkv_kernel<T, DP, DO, STAGES, true>
                 : (const void*)bwd_dkv_kernel<T, DP, DO, STAGES, false>;
-  k.grid = dim3((unsigned)((int64_t)p.n_nblocks * launch_pairs(p) * (DP / DO)));
+  k.grid = dim3((unsigned)((int64_t)p.n_nblocks * launch_pairs(p) * (DP / DO) *
+                           (p.kv_iters > 0 ? p.kv_chunks : 1)));
   k.block = dim3(512);
   k.kernel = "bwd_dkv_kernel";
   k.elem = T::code;
@@ -1517,6 +1573,77 @@ size_t bwd_ds_pair_bytes(int dtype, int Hq, int Hkv, int Sq, int Sk, int D, bool
   return (size_t)(Hq / Hkv) * (size_t)tiles * 2048;
 }
 
+// Split of the dK/dV kernel where its workgroups (one per CU) leave CUs idle
+// or, under the causal mask, unevenly loaded.
+// The chunk length minimises the kernel's time in steps: one chunk per CU
+// while they fit one round (their length), else the mean load plus half a
+// chunk, each with 4 steps of prologue and epilogue per workgroup, plus the
+// partial sums' write and read at 5 TB/s and 4 us for the merge.  A step takes
+// about 0.45 / 0.85 / 1.5 us at D = 64 / 128 / 256.  Unsplit, heavy blocks
+// first: the heaviest block or the mean load.  Measured (forward excluded,
+// bf16, H_q = 32, H_kv = 8, D = 128, causal): B = 1, S = 2,000 281 -> 171 us
+// (128 workgroups, now 240), B = 2, S = 1,337 204 -> 171; MQA, B = 2, S = 2,048
+// 1,686 -> 339 (32 workgroups).  At B = 4, S = 2,048 (512 workgroups) unsplit
+// and heavy first is the faster one, 462 us against 479.
+void bwd_dkv_split(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D, bool causal,
+                   int* iters, int* chunks) {
+  *iters = 0, *chunks = 1;
+  if (dtype != BF16::code && dtype != F16::code) return;
+  const int64_t pairs = (int64_t)B * Hkv;
+  const int64_t nb = ((int64_t)Sk + 127) / 128;
+  const int group = Hkv > 0 ? Hq / Hkv : 0;
+  if (pairs <= 0 || nb <= 0 || Sq <= 0 || group <= 0) return;
+  const int parts = D > 128 ? 2 : 1;  // workgroups per key block (head-dim halves)
+  if (pairs * nb * parts >= 1024) return;
+  // The last shape's answer: the workspace query and the call ask in turn.
+  struct Memo {
+    int key[7], iters, chunks;
+  };
+  static thread_local Memo memo = {};
+  const int key[7] = {B, Hq, Hkv, Sq, Sk, D, (int)causal};
+  if (std::equal(key, key + 7, memo.key)) {
+    *iters = memo.iters, *chunks = memo.chunks;
+    return;
+  }
+  const double step_us = D <= 64 ? 0.45 : D <= 128 ? 0.85 : 1.5;
+  // Steps of up to 64 evenly spaced key blocks stand for all of them.
+  const int ns = (int)std::min<int64_t>(nb, 64);
+  int steps[64];
+  double total = 0;
+  for (int i = 0; i < ns; ++i) {
+    steps[i] = group * dkv_tiles((int)(i * nb / ns), Sq, Sk, causal);
+    total += steps[i];
+  }
+  const double scale = (double)pairs * parts * nb / ns;  // workgroups a sample stands for
+  total *= scale;
+  const double longest = steps[0];
+  const double wgs = scale * ns;
+  const double whole = causal ? std::max(longest, 1.05 * total / 256)
+                              : std::ceil(wgs / 256) * longest;
+  const double unsplit_us = (whole + 4 * std::ceil(wgs / 256)) * step_us;
+  double best_us = 0.9 * unsplit_us;
+  int best = 0;
+  static const int kCuts[] = {2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 32, 48, 64};
+  for (int cut : kCuts) {
+    const int len = (steps[0] + cut - 1) / cut;
+    if (len < 8) break;
+    double n = 0, split = 0;  // workgroups; those that write partials
+    for (int i = 0; i < ns; ++i) {
+      const int c = dkv_chunks(steps[i], len);
+      n += c;
+      if (c > 1) split += c;
+    }
+    n *= scale, split *= scale / parts;
+    const double load = n <= 256 ? len + 4.0 : std::max<double>(len, total / 256 + 0.5 * len) + 4 * n / 256;
+    const double us = load * step_us + split * 128 * D * 8 * 2 / 5e6 + 4;
+    if (us < best_us) best_us = us, best = len;
+  }
+  memo = Memo{{}, best, 1};
+  std::copy(key, key + 7, memo.key);
+  if (best > 0) memo.chunks = dkv_chunks(steps[0], best);
+  *iters = memo.iters, *chunks = memo.chunks;
+}
+
 template <class T>
 static KernelPlan plan_dq_ds_t(BwdParams& p, bool causal) {
   constexpr int NW = 4, QW = kDqDs.qw;
@@ -1544,6 +1671,18 @@ KernelPlan plan_bwd_dq(int dtype, BwdParams& p, bool causal) {
   if (dtype == F16::code) return plan_dq_dt<F16>(p, causal);
   if (dtype == 0) return plan_bwd_dq_f32(p, causal);
   return KernelPlan{};
+}
+
+// Merge of a split dK/dV (nothing where it is unsplit).
+static hipError_t launch_dkv_reduce(int dtype, const BwdParams& p, bool causal, hipStream_t s) {
+  if (p.kv_iters <= 0) return hipSuccess;
+  const int64_t n = (int64_t)p.B * p.Hkv * p.Sk * (p.D / 4);
+  const dim3 grid((unsigned)((n + 255) / 256), 2);
+  if (dtype == BF16::code)
+    hipLaunchKernelGGL(bwd_dkv_reduce_kernel<BF16>, grid, dim3(256), 0, s, p, causal);
+  else
+    hipLaunchKernelGGL(bwd_dkv_reduce_kernel<F16>, grid, dim3(256), 0, s, p, causal);
+  return hipGetLastError();
 }
 
 // Side streams for the dQ kernel, one per (device, caller stream), each with
@@ -1642,7 +1781,7 @@ hipError_t launch_bwd_mfma(int dtype, const BwdParams& params, bool causal, hipS
       if (e != hipSuccess) return e;
       if ((e = run_plan(dq, &q, s)) != hipSuccess) return e;
     }
-    return hipSuccess;
+    return launch_dkv_reduce(dtype, p, causal, s);
   }
   BwdParams q = p;
   q.bk0 = 0;
@@ -1657,7 +1796,8 @@ hipError_t launch_bwd_mfma(int dtype, const BwdParams& params, bool causal, hipS
   if (!se) {
     hipError_t e = run_plan(kv, &q, s);
     if (e != hipSuccess) return e;
-    return run_plan(dq, &q, s);
+    if ((e = run_plan(dq, &q, s)) != hipSuccess) return e;
+    return launch_dkv_reduce(dtype, q, causal, s);
   }
   hipError_t e = hipEventRecord(se->fork, s);
   if (e == hipSuccess) e = hipStreamWaitEvent(se->side, se->fork, 0);
@@ -1665,7 +1805,8 @@ hipError_t launch_bwd_mfma(int dtype, const BwdParams& params, bool causal, hipS
   // From here on the side stream depends on s (under capture it has joined
   // s's capture), so it is joined back whatever fails.
   const hipError_t e_dq = run_plan(dq, &q, se->side);
-  const hipError_t e_kv = e_dq == hipSuccess ? run_plan(kv, &q, s) : hipSuccess;
+  hipError_t e_kv = e_dq == hipSuccess ? run_plan(kv, &q, s) : hipSuccess;
+  if (e_dq == hipSuccess && e_kv == hipSuccess) e_kv = launch_dkv_reduce(dtype, q, causal, s);
   hipError_t e_join = hipEventRecord(se->join, se->side);
   if (e_join == hipSuccess) e_join = hipStreamWaitEvent(s, se->join, 0);
   if (e_dq != hipSuccess) return e_dq;

@@ -145,9 +145,33 @@ struct BwdParams {
   float abs_scale_log2;
   uint32_t op_sign;
   int n_mblocks, n_nblocks;
-  int dkv_heavy_first;  // dK/dV: key blocks outermost, pairs fastest
+  int dkv_heavy_first;  // dK/dV (unsplit): key blocks outermost, pairs fastest
   int dq_heavy_first;   // dQ: items in heavy_first_order
+  // Split dK/dV (16-bit kernels): the steps (32-query tiles of the group's
+  // heads) of a key block run in dkv_chunks(steps, kv_iters) even chunks, one
+  // workgroup each; the launch has kv_chunks workgroups per key block (and
+  // head-dim part), those past a block's own count exit.  A block of several
+  // chunks writes fp32 partial sums, chunk-major [kv_chunks][B*Hkv][Sk][D], of
+  // dK (unscaled) and dV for bwd_dkv_reduce_kernel; a block of one writes dK
+  // and dV.  kv_iters 0: unsplit.
+  int kv_iters, kv_chunks;
+  float* part_dk;
+  float* part_dv;
 };
+
+// Steps of key block kb (128 keys) per query head: the 32-query tiles from
+// the first that sees its first key.
+__host__ __device__ inline int dkv_first_query(int kb, int Sq, int Sk, bool causal) {
+  const int d = 128 * kb - (Sk - Sq);
+  return causal && d > 0 ? d / 32 * 32 : 0;
+}
+__host__ __device__ inline int dkv_tiles(int kb, int Sq, int Sk, bool causal) {
+  const int m = dkv_first_query(kb, Sq, Sk, causal);
+  return m < Sq ? (Sq - m + 31) / 32 : 0;
+}
+__host__ __device__ inline int dkv_chunks(int steps, int iters) {
+  return steps > iters ? (steps + iters - 1) / iters : 1;
+}
 
 // dS tile layout of the five-GEMM backward, per query head.  The dK/dV
 // workgroup of key block kb (keys 128 kb .. 128 kb + 127) walks the query
@@ -263,6 +287,10 @@ KernelPlan plan_bwd_dq(int dtype, BwdParams& p, bool causal);
 // (its query heads' tiles), or 0 where the seven-GEMM backward runs (head
 // dims other than 65-128, fp32).
 size_t bwd_ds_pair_bytes(int dtype, int Hq, int Hkv, int Sq, int Sk, int D, bool causal);
+// Split of the dK/dV kernel the table takes for the shape: kv_iters and
+// kv_chunks of BwdParams (0 and 1: unsplit).
+void bwd_dkv_split(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D, bool causal,
+                   int* iters, int* chunks);
 KernelPlan plan_bwd_dkv_f32(BwdParams& p, bool causal);
 KernelPlan plan_bwd_dq_f32(BwdParams& p, bool causal);
 
