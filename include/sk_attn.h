@@ -165,9 +165,9 @@ SK_API int sk_attn_bwd_workspace_min(int dtype, int B, int Hq, int Hkv, int Sq, 
  * the workspace and the dQ kernel reads it, both on `stream`.  The results
  * are the same bit for bit for every chunking and equal the seven-GEMM
  * backward's.  Seven-GEMM backward (other head dims, fp32, or a workspace
- * too small for one pair's tiles): when the dK/dV grid runs more than one round of workgroups (more
- * than 256 workgroups), the dQ kernel runs on the library's side stream for
- * `stream`, forked from `stream` after the preprocess pass and joined back
+ * too small for one pair's tiles): where the dK/dV kernel runs more than one round of workgroups
+ * (more than 256) in head-major order (no mask, or S_k >= 2 S_q) for about
+ * 200 us or more, the dQ kernel runs on the library's side stream for `stream`, forked from `stream` after the preprocess pass and joined back
  * into it (also when a launch fails); under graph capture the fork and the
  * join are recorded as graph edges.  A call under capture on a stream that
  * has never run an eager backward keeps the one-stream order.

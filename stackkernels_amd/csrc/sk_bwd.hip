@@ -1573,13 +1573,15 @@ size_t bwd_ds_pair_bytes(int dtype, int Hq, int Hkv, int Sq, int Sk, int D, bool
   return (size_t)(Hq / Hkv) * (size_t)tiles * 2048;
 }
 
+// Microseconds of one dK/dV step (32 queries against 128 keys) of a workgroup.
+static double dkv_step_us(int d) { return d <= 64 ? 0.45 : d <= 128 ? 0.85 : 1.5; }
+
 // Split of the dK/dV kernel where its workgroups (one per CU) leave CUs idle
 // or, under the causal mask, unevenly loaded.
 // The chunk length minimises the kernel's time in steps: one chunk per CU
 // while they fit one round (their length), else the mean load plus half a
 // chunk, each with 4 steps of prologue and epilogue per workgroup, plus the
-// partial sums' write and read at 5 TB/s and 4 us for the merge.  A step takes
-// about 0.45 / 0.85 / 1.5 us at D = 64 / 128 / 256.  Unsplit, heavy blocks
+// partial sums' write and read at 5 TB/s and 4 us for the merge.  Unsplit, heavy blocks
 // first: the heaviest block or the mean load.  Measured (forward excluded,
 // bf16, H_q = 32, H_kv = 8, D = 128, causal): B = 1, S = 2,000 281 -> 171 us
 // (128 workgroups, now 240), B = 2, S = 1,337 204 -> 171; MQA, B = 2, S = 2,048
@@ -1605,7 +1607,7 @@ void bwd_dkv_split(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D, boo
     *iters = memo.iters, *chunks = memo.chunks;
     return;
   }
-  const double step_us = D <= 64 ? 0.45 : D <= 128 ? 0.85 : 1.5;
+  const double step_us = dkv_step_us(D);
   // Steps of up to 64 evenly spaced key blocks stand for all of them.
   const int ns = (int)std::min<int64_t>(nb, 64);
   int steps[64];
@@ -1743,14 +1745,30 @@ static const SideEntry* side_entry(hipStream_t s) {
 }
 
 // dK/dV and dQ only read what the preprocess pass and the caller wrote, and
-// write disjoint outputs.  When the dK/dV grid runs more than one round of
-// workgroups, dQ runs on the caller stream's side stream, forked from the
-// caller's stream after the preprocess pass and joined back with events: the
-// last, partly filled round of each kernel then overlaps the other kernel's
-// work.  Once dQ is queued on the side stream, the caller's stream always
-// waits for it, also when the dK/dV launch fails, so nothing queued after the
-// call can reuse its buffers early and a capture stays joined.
+// write disjoint outputs.  Where that pays, dQ runs on the caller stream's
+// side stream, forked from the caller's stream after the preprocess pass and
+// joined back with events: the last, partly filled round of each kernel then
+// overlaps the other kernel's work.  Once dQ is queued on the side stream, the
+// caller's stream always waits for it, also when the dK/dV launch fails, so
+// nothing queued after the call can reuse its buffers early and a capture
+// stays joined.
 //
+// The fork's stream and event calls take about 40 us of host time (25 us a
+// call without, 65 with), and two kernels that mix on the chip evict each
+// other's tiles, so it is kept for calls of more than one round, in
+// head-major order (heavy-first grids end evenly by themselves) and long
+// enough to hide it: dK/dV of 200 us or more by its step count.  bf16, one
+// stream against the fork: H_q = 32, H_kv = 8, 2,048 x 8,192, D = 64 922 and
+// 879 us, non-causal S = 1,500, D = 256 609 and 535; causal S = 4,096, D = 256
+// 2,620 and 2,996, fp16 S = 1,024, D = 64 (48 heads) 57 and 60 with the host
+// 45 us longer.
+static bool fork_pays(const BwdParams& p, bool causal, int64_t dkv_wgs) {
+  if (dkv_wgs <= 256 || p.dkv_heavy_first) return false;
+  const double seen = causal ? (double)p.Sq * (p.Sk - p.Sq / 2) : (double)p.Sq * p.Sk;
+  const double steps = (double)p.B * p.Hq * (p.D > 128 ? 2 : 1) * seen / (32 * 128);
+  return steps / 256 * dkv_step_us(p.D) >= 200;
+}
+
 // Five-GEMM backward (p.ds set, p.n_pairs the pairs per chunk): for each
 // chunk of (batch, KV head) pairs in turn, the dK/dV kernel writes the
 // chunk's dS tiles and the dQ kernel reads them, both on the caller's stream.
@@ -1792,7 +1810,7 @@ hipError_t launch_bwd_mfma(int dtype, const BwdParams& params, bool causal, hipS
   const int64_t g_kv = (int64_t)q.n_nblocks * p.B * p.Hkv * (kv.head_dim == 256 ? 2 : 1);
   const int64_t g_q = (int64_t)q.n_mblocks * p.B * p.Hq;
   if (g_kv > 0x7fffffffLL || g_q > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-  const SideEntry* se = g_kv > 256 && g_q > 0 ? side_entry(s) : nullptr;
+  const SideEntry* se = fork_pays(q, causal, g_kv) && g_q > 0 ? side_entry(s) : nullptr;
   if (!se) {
     hipError_t e = run_plan(kv, &q, s);
     if (e != hipSuccess) return e;

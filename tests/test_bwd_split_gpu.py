@@ -15,6 +15,7 @@ import pytest
 import torch
 
 from stackkernels_amd._core.attention import _lib
+from stackkernels_amd._core.attention.flash_bwd import flash_attn_bwd
 from stackkernels_amd._core.attention.flash_fwd import flash_attn_fwd
 from stackkernels_amd._reference.torch.attention import attention_reference
 
@@ -56,7 +57,7 @@ def _bwd(do, q, k, v, o, lse, causal, ws_bytes):
     (1, 8, 2, 300, 130, 96, True),     # S_q > S_k
     (2, 8, 1, 257, 129, 80, False),    # ragged, one key in the second block
     (1, 16, 1, 200, 1500, 64, True),
-    (13, 40, 10, 1000, 200, 64, False),  # 260 key blocks: dQ on the side stream
+    (13, 40, 10, 1000, 200, 64, False),  # 260 key blocks, two rounds
     (1, 8, 1, 190, 260, 256, True),    # head-dim halves
 ])
 def test_split_matches_oracle(device, dtype, b, hq, hkv, sq, sk, d, causal):
@@ -104,3 +105,42 @@ def test_many_heads_of_few_queries(device):
     torch.cuda.synchronize()
     for x, y in zip(a, b):
         assert torch.isfinite(x).all() and (x.float() - y.float()).abs().max() <= 2e-2
+
+
+def test_forked_call_replays_match_eager(device):
+    """D = 64, 2,048 x 8,192 (1,024 key blocks, dK/dV of about 400 us): dQ runs on the
+    side stream, eagerly and as a captured graph's fork and join."""
+    b, hq, hkv, sq, sk, d = 2, 32, 8, 2048, 8192, 64
+    gen = torch.Generator(device=device).manual_seed(9)
+
+    def inputs():
+        q, do = (torch.randn(b, hq, sq, d, generator=gen, device=device).to(torch.bfloat16)
+                 for _ in range(2))
+        k, v = (torch.randn(b, hkv, sk, d, generator=gen, device=device).to(torch.bfloat16)
+                for _ in range(2))
+        return q, k, v, do
+
+    q, k, v, do = inputs()
+    o, lse = flash_attn_fwd(q, k, v, is_causal=True)
+    cap = torch.cuda.Stream()
+    cap.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(cap):
+        flash_attn_bwd(do, q, k, v, o, lse, is_causal=True)
+    torch.cuda.current_stream().wait_stream(cap)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=cap):
+        grads = flash_attn_bwd(do, q, k, v, o, lse, is_causal=True)
+    unsplit = _bytes(q, k, True)[1]
+    for step in range(3):
+        new = inputs()
+        o2, lse2 = flash_attn_fwd(*new[:3], is_causal=True)
+        for dst, src in zip((q, k, v, do, o, lse), (*new, o2, lse2)):
+            dst.copy_(src)
+        want = flash_attn_bwd(new[3], *new[:3], o2, lse2, is_causal=True)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for x, y, name in zip(grads, want, ("dQ", "dK", "dV")):
+            assert torch.equal(x, y), f"replay {step}: {name}"
+        for x, y in zip(want, _bwd(new[3], *new[:3], o2, lse2, True, unsplit)):
+            assert torch.equal(x, y)
