@@ -78,20 +78,42 @@ int check_ptr(const char* name, const void* p) {
 //   round; a 64-head group writes 32 KB of partials per split, so fewer,
 //   longer splits also keep that traffic small (C5: 64 splits; 32 and 128
 //   splits measured 15% and 10% slower).
-// Every split keeps at least 256 keys (8 tiles) and the count is capped at
-// 1024 (the combine kernel's LDS weight array).
+// A split keeps at least 256 keys, 128 from 64 (batch, KV head) units on with
+// groups of up to 16 heads.  Small calls (at most 1,024 query heads in all,
+// whose partials cost the combine little) split further, because a split's
+// tiles follow one another: to 64 keys while that gives at most 512
+// workgroups (128 with the 64-key tiles of groups above 32), to one 32-key
+// tile while at most 256.  Microseconds of both kernels (graph replays), H_q =
+// 32, H_kv = 8, D = 128 bf16, 256 keys a split -> now: B = 1, S_k = 1,000 19.2
+// -> 8.4 (32 splits), S_k = 4,096 16.2 -> 10.8 (64); B = 16, S_k = 1,000 22.4
+// -> 19.3 (7); MQA, 64 heads, B = 1, S_k = 8,192 13.8 -> 11.6 (64).  Past
+// those limits more splits lose: B = 1, S_k = 32,768 31 us at 128, 36 at 256;
+// 64 x 64 heads, S_k = 500 16 us whole, 23 at 6.  Caches below 192 keys stay
+// whole.
+// Per-row lengths take their second round only where half of S_k gives each
+// split 512 keys (B = 32, U[1, 4,096]: 54.6 us with 16 splits, 53.1 with 8; B
+// = 64, U[1, 2,048]: 60.1 with 8, 56.5 with 4).  The count is capped at 1024
+// (the combine kernel's LDS weight array).
 int plan_splits(int B, int Hq, int Hkv, int Sk, int D, bool per_row) {
   (void)D;
-  if (Sk <= 0 || B <= 0 || Hkv <= 0) return 1;
+  if (Sk < 192 || B <= 0 || Hkv <= 0) return 1;
   const int group = Hq / Hkv;
   const int waves = group <= 16 ? 1 : group <= 32 ? 2 : 4;
   const int64_t slots = 256LL * 8 / waves;
-  const int rounds = group <= 16 && per_row ? 2 : 1;
   const int64_t units = (int64_t)B * Hkv;
-  int64_t splits = (rounds * slots + units - 1) / units;
-  splits = std::min<int64_t>(splits, std::max(1, Sk / 256));
-  splits = std::max<int64_t>(1, std::min<int64_t>(splits, 1024));
-  return (int)splits;
+  int64_t splits = (slots + units - 1) / units;
+  if (group <= 16 && per_row) {
+    const int64_t two = (2 * slots + units - 1) / units;
+    if (Sk >= two * 1024) splits = two;
+  }
+  int64_t most = Sk / (group <= 16 && units >= 64 ? 128 : 256);
+  if ((int64_t)B * Hq <= 1024) {
+    most = std::max<int64_t>(most, std::min<int64_t>(512 / units, Sk / (group > 32 ? 128 : 64)));
+    if (group <= 32)
+      most = std::max<int64_t>(most, std::min<int64_t>(256 / units, (Sk + 31) / 32));
+  }
+  splits = std::min(splits, most);
+  return (int)std::max<int64_t>(1, std::min<int64_t>(splits, 1024));
 }
 
 int keys_per_split_for(int Sk, int splits) {

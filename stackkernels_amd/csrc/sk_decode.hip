@@ -192,9 +192,6 @@ __global__ void __launch_bounds__(NWH * 64) decode_split_kernel(DecParams p) {
   const uint16_t* kbase = (const uint16_t*)p.k + b * p.k_sb + hkv * p.k_sh;
   const uint16_t* vbase = (const uint16_t*)p.v + b * p.v_sb + hkv * p.v_sh;
 
-  u32x4 qreg[KD];
-  load_q<T>(p, b, hq, head_ok, g, qreg);
-
   // Paged: the page of tile t + 2 is read (vector load) while tile t runs,
   // and used when tile t + 2's loads are issued, one iteration later.
   PageTable ptab{};
@@ -253,6 +250,10 @@ __global__ void __launch_bounds__(NWH * 64) decode_split_kernel(DecParams p) {
     if (n_tiles > 1) pg_nxt = page_of(1);
     load_tile(0, pg_cur);
   }
+  // q (and its rotation's table rows) behind the first tile's loads: the two
+  // latencies overlap.
+  u32x4 qreg[KD];
+  load_q<T>(p, b, hq, head_ok, g, qreg);
   for (int t = 0; t < n_tiles; ++t) {
     store_tile();
     __syncthreads();
