@@ -2,6 +2,7 @@
 
 from __future__ import annotations
 
+import ctypes
 import math
 
 import torch
@@ -64,6 +65,20 @@ def kernel_operand(t: torch.Tensor) -> torch.Tensor:
     if c.data_ptr() % 16 != 0:
         c = c.clone()
     return c
+
+
+def operand(t: torch.Tensor, dk: int) -> tuple[torch.Tensor, int, ctypes.Array]:
+    """``t`` zero-padded to head dim ``dk`` where needed, as the library reads it
+    (``kernel_operand``): the tensor, its address and its (b, h, s) strides."""
+    if t.shape[-1] != dk:
+        t = pad_head(t, dk)
+    st = t.stride()
+    unit = 3 if t.dtype == torch.float32 else 7
+    ptr = t.data_ptr()
+    if ptr & 15 or (st[0] | st[1] | st[2]) & unit or (st[3] != 1 and t.shape[-1] != 1):
+        t = kernel_operand(t)
+        return t, t.data_ptr(), _lib.strides3(t)
+    return t, ptr, _lib._I64x3(st[0], st[1], st[2])
 
 
 def stream_of(device: torch.device) -> int:

@@ -9,6 +9,7 @@ is no silent fallback to another implementation.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 import threading
@@ -147,10 +148,13 @@ def check(rc: int, what: str) -> None:
     raise RuntimeError(f"{what} failed (code {rc}): {msg}")
 
 
+_I64x3 = ctypes.c_int64 * 3
+
+
 def strides3(t) -> ctypes.Array:
     """(b, h, s) element strides of a BHSD tensor as an int64[3]."""
     st = t.stride()
-    return (ctypes.c_int64 * 3)(st[0], st[1], st[2])
+    return _I64x3(st[0], st[1], st[2])
 
 
 def dtype_code(dtype) -> int:
@@ -166,9 +170,23 @@ def dtype_code(dtype) -> int:
 
 
 def stream_ptr(device) -> int:
+    """Torch's current stream on `device` as a hipStream_t (the raw handle: building
+    a torch Stream object for it costs 2 us a call)."""
     import torch
 
-    return torch.cuda.current_stream(device).cuda_stream
+    if device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+_HERE = contextlib.nullcontext()
+
+
+def device_guard(device):
+    """torch.cuda.device(device), or nothing where it is current already."""
+    import torch
+
+    return _HERE if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
 
 
 def loaded_hip_runtimes() -> list[str]:

@@ -88,7 +88,7 @@ def rope_rotate(x: torch.Tensor, rope: RopeArgs, inverse: bool = False,
     if out is None:
         out = torch.empty_like(x, memory_format=torch.contiguous_format)
     lib = _lib.load()
-    with torch.cuda.device(x.device):
+    with _lib.device_guard(x.device):
         rc = lib.sk_rope_rotate(_lib.dtype_code(x.dtype), x.data_ptr(), out.data_ptr(), b, h, s,
                                 d, _lib.strides3(x), _lib.strides3(out), *rope.args,
                                 int(bool(inverse)), _lib.stream_ptr(x.device))

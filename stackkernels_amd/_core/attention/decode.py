@@ -24,8 +24,7 @@ from stackkernels_amd._core.attention._common import (
     check_device,
     default_scale,
     kernel_head_dim,
-    kernel_operand,
-    pad_head,
+    operand,
     stream_of,
 )
 from stackkernels_amd._core.attention.layout import validate_attention_layout
@@ -72,34 +71,23 @@ def flash_decode(q, k, v, sm_scale: float | None = None, num_splits: int | None 
     rope = rope_args(rope_cos, rope_sin, start_pos, b, d, dev)
     scale = default_scale(d, sm_scale)
     dk = kernel_head_dim(d)
-    qk, kk, vk = (kernel_operand(pad_head(t, dk)) for t in (q, k, v))
+    qk, qp, qs = operand(q, dk)
+    kk, kp, ks = operand(k, dk)
+    vk, vp, vs = operand(v, dk)
     lib = _lib.load()
-    code = _lib.dtype_code(q.dtype)
     ws, ns = decode_workspace(q.dtype, b, hq, hkv, sk, dk, dev, num_splits,
                               per_row=lens is not None)
-    out = torch.empty((b, hq, 1, dk), dtype=q.dtype, device=dev)
-    with torch.cuda.device(dev):
+    out = q.new_empty((b, hq, 1, dk))
+    args = (_lib.dtype_code(q.dtype), qp, kp, vp, out.data_ptr(), ws.data_ptr(), ws.numel(), ns, b,
+            hq, hkv, sk, dk, qs, ks, vs, _lib.strides3(out))
+    with _lib.device_guard(dev):
         if rope is not None:
-            rc = lib.sk_decode_rope(
-                code, qk.data_ptr(), kk.data_ptr(), vk.data_ptr(), out.data_ptr(), ws.data_ptr(),
-                ws.numel(), ns, b, hq, hkv, sk, dk,
-                _lib.strides3(qk), _lib.strides3(kk), _lib.strides3(vk), _lib.strides3(out),
-                None if lens is None else lens.data_ptr(), *rope.args, scale, stream_of(dev),
-            )
+            rc = lib.sk_decode_rope(*args, None if lens is None else lens.data_ptr(), *rope.args,
+                                    scale, stream_of(dev))
         elif lens is None:
-            rc = lib.sk_decode(
-                code, qk.data_ptr(), kk.data_ptr(), vk.data_ptr(), out.data_ptr(), ws.data_ptr(),
-                ws.numel(), ns, b, hq, hkv, sk, dk,
-                _lib.strides3(qk), _lib.strides3(kk), _lib.strides3(vk), _lib.strides3(out),
-                scale, stream_of(dev),
-            )
+            rc = lib.sk_decode(*args, scale, stream_of(dev))
         else:
-            rc = lib.sk_decode_varlen(
-                code, qk.data_ptr(), kk.data_ptr(), vk.data_ptr(), out.data_ptr(), ws.data_ptr(),
-                ws.numel(), ns, b, hq, hkv, sk, dk,
-                _lib.strides3(qk), _lib.strides3(kk), _lib.strides3(vk), _lib.strides3(out),
-                lens.data_ptr(), scale, stream_of(dev),
-            )
+            rc = lib.sk_decode_varlen(*args, lens.data_ptr(), scale, stream_of(dev))
     _lib.check(rc, "flash_decode")
     if dk != d:
         out = out[..., :d].contiguous()
@@ -151,17 +139,17 @@ def flash_decode_paged(q, k_pool, v_pool, block_table, cache_seqlens,
     max_pages = table.shape[1]
     scale = default_scale(d, sm_scale)
     dk = kernel_head_dim(d)
-    qk, kk, vk = (kernel_operand(pad_head(t, dk)) for t in (q, k_pool, v_pool))
+    qk, qp, qs = operand(q, dk)
+    kk, kp, ks = operand(k_pool, dk)
+    vk, vp, vs = operand(v_pool, dk)
     lib = _lib.load()
-    code = _lib.dtype_code(q.dtype)
     sk = max_pages * page_size
     ws, ns = decode_workspace(q.dtype, b, hq, hkv, sk, dk, dev, num_splits, per_row=True)
-    out = torch.empty((b, hq, 1, dk), dtype=q.dtype, device=dev)
-    paged_args = (code, qk.data_ptr(), kk.data_ptr(), vk.data_ptr(), out.data_ptr(),
-                  ws.data_ptr(), ws.numel(), ns, b, hq, hkv, num_pages, page_size, max_pages, dk,
-                  _lib.strides3(qk), _lib.strides3(kk), _lib.strides3(vk), _lib.strides3(out),
-                  table.data_ptr(), lens.data_ptr())
-    with torch.cuda.device(dev):
+    out = q.new_empty((b, hq, 1, dk))
+    paged_args = (_lib.dtype_code(q.dtype), qp, kp, vp, out.data_ptr(), ws.data_ptr(), ws.numel(),
+                  ns, b, hq, hkv, num_pages, page_size, max_pages, dk, qs, ks, vs,
+                  _lib.strides3(out), table.data_ptr(), lens.data_ptr())
+    with _lib.device_guard(dev):
         if rope is None:
             rc = lib.sk_decode_paged(*paged_args, scale, stream_of(dev))
         else:

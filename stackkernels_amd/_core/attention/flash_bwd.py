@@ -34,13 +34,13 @@ def flash_attn_bwd(do, q, k, v, out, lse, is_causal: bool = False, sm_scale: flo
     dk_ = kernel_head_dim(d)
     do_, q_, k_, v_, o_ = (_contig(pad_head(t, dk_)) for t in (do, q, k, v, out))
     lse_ = _contig(lse.float())
-    dq = torch.empty((b, hq, sq, dk_), dtype=q.dtype, device=dev)
-    dkk = torch.empty((b, hkv, sk, dk_), dtype=q.dtype, device=dev)
-    dvv = torch.empty((b, hkv, sk, dk_), dtype=q.dtype, device=dev)
+    dq = q.new_empty((b, hq, sq, dk_))
+    dkk = q.new_empty((b, hkv, sk, dk_))
+    dvv = q.new_empty((b, hkv, sk, dk_))
     lib = _lib.load()
     code = _lib.dtype_code(q.dtype)
     ws = bwd_workspace(q.dtype, b, hq, hkv, sq, sk, dk_, is_causal, dev)
-    with torch.cuda.device(dev):
+    with _lib.device_guard(dev):
         rc = lib.sk_attn_bwd(
             code, do_.data_ptr(), q_.data_ptr(), k_.data_ptr(), v_.data_ptr(), o_.data_ptr(),
             lse_.data_ptr(), dq.data_ptr(), dkk.data_ptr(), dvv.data_ptr(), ws.data_ptr(),

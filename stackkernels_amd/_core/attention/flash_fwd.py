@@ -21,8 +21,7 @@ from stackkernels_amd._core.attention._common import (
     check_device,
     default_scale,
     kernel_head_dim,
-    kernel_operand,
-    pad_head,
+    operand,
     stream_of,
 )
 from stackkernels_amd._core.attention.layout import validate_attention_layout
@@ -40,16 +39,17 @@ def flash_attn_fwd(q, k, v, is_causal: bool = False, sm_scale: float | None = No
     rope = rope_args(rope_cos, rope_sin, start_pos, b, d, dev)
     scale = default_scale(d, sm_scale)
     dk = kernel_head_dim(d)
-    qk, kk, vk = (kernel_operand(pad_head(t, dk)) for t in (q, k, v))
-    out = torch.empty((b, hq, sq, dk), dtype=q.dtype, device=dev)
+    qk, qp, qs = operand(q, dk)
+    kk, kp, ks = operand(k, dk)
+    vk, vp, vs = operand(v, dk)
+    out = q.new_empty((b, hq, sq, dk))
     lse = torch.empty((b, hq, sq), dtype=torch.float32, device=dev)
     lib = _lib.load()
     code = _lib.dtype_code(q.dtype)
     ws = fwd_workspace(code, b, hq, hkv, sq, sk, dk, is_causal, dev)
-    ptrs = (code, qk.data_ptr(), kk.data_ptr(), vk.data_ptr(), out.data_ptr(), lse.data_ptr())
-    shape = (b, hq, hkv, sq, sk, dk, _lib.strides3(qk), _lib.strides3(kk), _lib.strides3(vk),
-             _lib.strides3(out), int(bool(is_causal)))
-    with torch.cuda.device(dev):
+    ptrs = (code, qp, kp, vp, out.data_ptr(), lse.data_ptr())
+    shape = (b, hq, hkv, sq, sk, dk, qs, ks, vs, _lib.strides3(out), int(bool(is_causal)))
+    with _lib.device_guard(dev):
         if ws is not None:
             rc = lib.sk_attn_fwd_ws(*ptrs, ws.data_ptr(), ws.numel(), 0, *shape,
                                     *(_NO_ROPE if rope is None else rope.args), scale,

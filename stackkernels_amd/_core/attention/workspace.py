@@ -42,6 +42,22 @@ def fwd_workspace(code: int, B: int, Hq: int, Hkv: int, Sq: int, Sk: int, D: int
         return None
 
 
+@functools.lru_cache(maxsize=512)
+def _bwd_workspace_bytes(code: int, B: int, Hq: int, Hkv: int, Sq: int, Sk: int, D: int,
+                         is_causal: bool) -> tuple[int, ...]:
+    """The sizes bwd_workspace tries, largest first (each at least 16 bytes)."""
+    lib = _lib.load()
+    nb = ctypes.c_size_t(0)
+    sizes = []
+    for fn in (lib.sk_attn_bwd_workspace_best, lib.sk_attn_bwd_workspace,
+               lib.sk_attn_bwd_workspace_min):
+        _lib.check(fn(code, B, Hq, Hkv, Sq, Sk, D, int(is_causal), ctypes.byref(nb)),
+                   "flash_attn_bwd")
+        if max(nb.value, 16) not in sizes:
+            sizes.append(max(nb.value, 16))
+    return tuple(sizes)
+
+
 def bwd_workspace(dtype: torch.dtype, B: int, Hq: int, Hkv: int, Sq: int, Sk: int, D: int,
                   is_causal: bool, device) -> torch.Tensor:
     """uint8 scratch for ``sk_attn_bwd`` (D: the kernel head dim; at least 16 bytes).
@@ -54,21 +70,26 @@ def bwd_workspace(dtype: torch.dtype, B: int, Hq: int, Hkv: int, Sq: int, Sk: in
     seven-GEMM backward: slower, and dK/dV summed in another order than a
     split one sums them.
     """
-    lib = _lib.load()
-    args = (_lib.dtype_code(dtype), B, Hq, Hkv, Sq, Sk, D, int(bool(is_causal)))
-    nb = ctypes.c_size_t(0)
-    tried = -1
-    for fn in (lib.sk_attn_bwd_workspace_best, lib.sk_attn_bwd_workspace):
-        _lib.check(fn(*args, ctypes.byref(nb)), "flash_attn_bwd")
-        if nb.value == tried:
-            continue
-        tried = nb.value
+    code = _lib.dtype_code(dtype)
+    sizes = _bwd_workspace_bytes(code, B, Hq, Hkv, Sq, Sk, D, bool(is_causal))
+    for nb in sizes[:-1]:
         try:
-            return torch.empty(max(nb.value, 16), dtype=torch.uint8, device=device)
+            return torch.empty(nb, dtype=torch.uint8, device=device)
         except torch.OutOfMemoryError:
             pass
-    _lib.check(lib.sk_attn_bwd_workspace_min(*args, ctypes.byref(nb)), "flash_attn_bwd")
-    return torch.empty(max(nb.value, 16), dtype=torch.uint8, device=device)
+    return torch.empty(sizes[-1], dtype=torch.uint8, device=device)
+
+
+@functools.lru_cache(maxsize=512)
+def _decode_plan(code: int, B: int, Hq: int, Hkv: int, Sk: int, D: int,
+                 per_row: bool) -> tuple[int, int]:
+    """(split count, workspace bytes) of the library's table."""
+    lib = _lib.load()
+    ns, nb = ctypes.c_int(0), ctypes.c_size_t(0)
+    fn = lib.sk_decode_plan_varlen if per_row else lib.sk_decode_plan
+    _lib.check(fn(code, B, Hq, Hkv, Sk, D, ctypes.byref(ns), ctypes.byref(nb)),
+               "flash_decode plan")
+    return ns.value, nb.value
 
 
 def decode_workspace(dtype: torch.dtype, B: int, Hq: int, Hkv: int, Sk: int, D: int, device,
@@ -77,19 +98,16 @@ def decode_workspace(dtype: torch.dtype, B: int, Hq: int, Hkv: int, Sk: int, D: 
     """(uint8 scratch, split count) for ``sk_decode*`` (D: the kernel head dim):
     the gfx950 table's split count when ``num_splits`` is None (``per_row``:
     the plan for per-row cache lengths and paged pools), else the given one."""
-    lib = _lib.load()
     code = _lib.dtype_code(dtype)
-    nb = ctypes.c_size_t(0)
     if num_splits is None:
-        ns = ctypes.c_int(0)
-        fn = lib.sk_decode_plan_varlen if per_row else lib.sk_decode_plan
-        _lib.check(fn(code, B, Hq, Hkv, Sk, D, ctypes.byref(ns), ctypes.byref(nb)),
-                   "flash_decode plan")
-        num_splits = ns.value
+        num_splits, nb = _decode_plan(code, B, Hq, Hkv, Sk, D, bool(per_row))
     else:
-        _lib.check(lib.sk_decode_workspace(code, B, Hq, Hkv, Sk, D, int(num_splits),
-                                           ctypes.byref(nb)), "flash_decode")
-    return torch.empty(max(nb.value, 16), dtype=torch.uint8, device=device), int(num_splits)
+        size = ctypes.c_size_t(0)
+        num_splits = int(num_splits)
+        _lib.check(_lib.load().sk_decode_workspace(code, B, Hq, Hkv, Sk, D, num_splits,
+                                                   ctypes.byref(size)), "flash_decode")
+        nb = size.value
+    return torch.empty(max(nb, 16), dtype=torch.uint8, device=device), num_splits
 
 
 __all__ = ["fwd_workspace", "bwd_workspace", "decode_workspace"]

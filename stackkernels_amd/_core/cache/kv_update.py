@@ -64,7 +64,7 @@ def kv_cache_update(k, v, k_cache, v_cache, slot_indices, paged: bool = False,
     rope = rope_args(rope_cos, rope_sin, start_pos, b, d, dev)
     lib = _lib.load()
     sts = (_lib.strides3(k), _lib.strides3(v), _lib.strides3(k_cache), _lib.strides3(v_cache))
-    with torch.cuda.device(dev):
+    with _lib.device_guard(dev):
         if rope is not None and paged:
             rc = lib.sk_kv_cache_update_paged_rope(
                 _lib.dtype_code(k.dtype), k.data_ptr(), v.data_ptr(), k_cache.data_ptr(),

@@ -31,6 +31,24 @@ from stackkernels_amd.torch._dispatch import should_use_hip
 from stackkernels_amd.torch._utils import ensure_contiguous
 
 
+# Row strides up to which the forward reads q, k, v in place (elements): a
+# 64-row tile then spans at most 1 GiB of fp32, inside the kernels' 31-bit
+# tile offsets.
+_MAX_ROW_STRIDE = 1 << 22
+
+
+def _saved_or_read(ctx, use_hip, *tensors):
+    """q, k, v for the forward: contiguous where a backward will read them again,
+    or on the reference path; else as they are.  The HIP forward reads any
+    strides of 16-byte-aligned rows in place, so a projection's transposed view
+    or a slice of a KV cache is not copied (B = 2, H_q = 32, H_kv = 8, S =
+    1,337, D = 128 bf16: 29 us of copies before a 43 us kernel)."""
+    if use_hip and not any(ctx.needs_input_grad[:3]) and all(
+            t.dim() == 4 and t.stride(2) <= _MAX_ROW_STRIDE for t in tensors):
+        return tensors
+    return tuple(ensure_contiguous(t) for t in tensors)
+
+
 class FlashAttentionFunction(torch.autograd.Function):
     """FlashAttention-2 forward/backward with MHA, GQA and MQA support.
 
@@ -53,7 +71,7 @@ class FlashAttentionFunction(torch.autograd.Function):
         ctx.use_hip = use_hip
         ctx.is_causal = is_causal
         ctx.sm_scale = scale
-        qc, kc, vc = ensure_contiguous(q), ensure_contiguous(k), ensure_contiguous(v)
+        qc, kc, vc = _saved_or_read(ctx, use_hip, q, k, v)
         if use_hip:
             out, lse = flash_attn_fwd(qc, kc, vc, is_causal=is_causal, sm_scale=scale)
         else:
@@ -140,7 +158,7 @@ class _FlashAttentionRoPEFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx: Any, q, k, v, is_causal, sm_scale, rope_cos, rope_sin, start_pos):
         scale = 1.0 / math.sqrt(q.shape[-1]) if sm_scale is None else sm_scale
-        qc, kc, vc = ensure_contiguous(q), ensure_contiguous(k), ensure_contiguous(v)
+        qc, kc, vc = _saved_or_read(ctx, True, q, k, v)
         out, lse = flash_attn_fwd(qc, kc, vc, is_causal=is_causal, sm_scale=scale,
                                   rope_cos=rope_cos, rope_sin=rope_sin, start_pos=start_pos)
         ctx.is_causal = is_causal
