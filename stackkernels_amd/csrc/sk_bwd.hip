@@ -169,14 +169,18 @@ __device__ __forceinline__ u32x4 lds_tr_pair(const uint8_t* lo, const uint8_t* h
 // ahead so that every step interleaves MFMAs with the VALU work of the
 // previous tile in the same wave (a wave overlaps MFMA and VALU issue only
 // with its own instructions).
-template <class T, int DP, int DO, int STAGES, bool CAUSAL>
+//
+// DP: the head dim the LDS tiles are laid out for; DC <= DP: the one the
+// MFMAs cover (a multiple of 32, at least D); DO: output columns of a
+// workgroup.
+template <class T, int DP, int DC, int DO, int STAGES, bool CAUSAL>
 __global__ void __launch_bounds__(512, 1) bwd_dkv_kernel(BwdParams p) {
   constexpr int NW = 8;   // waves: two roles per key group
   constexpr int NKG = 4;  // key groups of 32 keys
   constexpr int BMQ = 32;  // queries per tile (one 32x32 score block per wave)
   using L = BwdTile<DP, BMQ>;  // Q and dO tiles
   constexpr int BNK = 128;
-  constexpr int KD = DP / 16;  // k-steps over the head dim (S, dP)
+  constexpr int KD = DC / 16;  // k-steps over the head dim (S, dP)
   constexpr int DB = DO / 32;  // 32-wide output head-dim blocks
   constexpr int LS = 2 * L::kSegs / NW;  // Q + dO segments per wave per tile
   constexpr int QT = L::kTileBytes;
@@ -191,7 +195,8 @@ __global__ void __launch_bounds__(512, 1) bwd_dkv_kernel(BwdParams p) {
   constexpr int kLds = kPReg + 2 * 4 * kPBlock;
   constexpr int kLoads = LS + 1;  // DMAs per wave per tile
   constexpr int PD = 2;  // tiles issued ahead
-  constexpr int kDSplit = DP / DO;
+  constexpr int kDSplit = DC / DO;
+  static_assert(DC % DO == 0, "whole output parts");
   // 4 stages: S and P of a tile in one step (any D).  6 stages (D <= 128):
   // the pipelined schedule below, S one step ahead of P.
   constexpr bool kV2 = STAGES == 6;
@@ -909,14 +914,14 @@ __global__ void __launch_bounds__(256) bwd_dkv_reduce_kernel(BwdParams p, bool c
 // ---------------------------------------------------------------------------
 // dQ
 // ---------------------------------------------------------------------------
-template <class T, int DP, int BN, int NW, int STAGES, int OCC, int MODE, bool CAUSAL>
+template <class T, int DP, int DC, int BN, int NW, int STAGES, int OCC, int MODE, bool CAUSAL>
 __global__ void __launch_bounds__(NW * 64, OCC) bwd_dq_kernel(BwdParams p) {
   static_assert(MODE == 0 || MODE == 2, "dQ schedule: 0 (tiles in order) or 2");
   using L = BwdTile<DP, BN>;  // K and V tiles
   constexpr int BM = 32 * NW;
-  constexpr int KD = DP / 16;  // k-steps over the head dim (S^T, dP^T)
+  constexpr int KD = DC / 16;  // k-steps over the head dim (S^T, dP^T)
   constexpr int KB = BN / 32;  // 32-key blocks per tile
-  constexpr int DB = DP / 32;  // 32-wide head-dim blocks of dQ^T
+  constexpr int DB = DC / 32;  // 32-wide head-dim blocks of dQ^T
   constexpr int KN = BN / 16;  // k-steps over keys (dQ^T)
   constexpr int LK = L::kSegs / NW;
   constexpr int kStageBytes = 2 * L::kTileBytes;  // K tile, then V tile
@@ -1267,7 +1272,7 @@ struct DqDsTile {
 };
 constexpr DqDsTile kDqDs{SK_BWD_DQDS_TILE};
 
-template <class T, int DP, int QW, int STAGES, int OCC, bool CAUSAL>
+template <class T, int DP, int DC, int QW, int STAGES, int OCC, bool CAUSAL>
 __global__ void __launch_bounds__(256, OCC) bwd_dq_ds_kernel(BwdParams p) {
   constexpr int NW = 4;
   constexpr int BN = 32;
@@ -1275,7 +1280,7 @@ __global__ void __launch_bounds__(256, OCC) bwd_dq_ds_kernel(BwdParams p) {
   static_assert(STAGES >= 3, "a ring of at least three stages");
   using L = BwdTile<DP, BN>;  // K tiles
   constexpr int BM = 32 * QW * NW;
-  constexpr int DB = DP / 32;  // 32-wide head-dim blocks of dQ^T
+  constexpr int DB = DC / 32;  // 32-wide head-dim blocks of dQ^T
   constexpr int KN = BN / 16;  // k-steps over keys
   constexpr int LK = L::kSegs / NW;
   constexpr int kDs = 2048;  // one 32-query dS tile
@@ -1482,7 +1487,7 @@ static int64_t launch_pairs(const BwdParams& p) {
   return p.n_pairs > 0 ? p.n_pairs : (int64_t)p.B * p.Hkv;
 }
 
-template <class T, int DP, int DO>
+template <class T, int DP, int DO, int DC = DP>
 static KernelPlan plan_dkv_t(BwdParams& p, bool causal) {
   // D = 128 and D = 64: the 6-deep pipelined schedule (S one step ahead of
   // P; 3%-7% faster at D = 128, up to 10% at D = 64); SK_BWD_DKV_STAGES=4
@@ -1491,9 +1496,9 @@ static KernelPlan plan_dkv_t(BwdParams& p, bool causal) {
   constexpr int STAGES = DP == 128 ? SK_BWD_DKV_STAGES : DP == 64 ? SK_BWD_DKV_STAGES_D64 : 4;
   p.n_nblocks = (p.Sk + 127) / 128;
   KernelPlan k;
-  k.fn = causal ? (const void*)bwd_dkv_kernel<T, DP, DO, STAGES, true>
-                : (const void*)bwd_dkv_kernel<T, DP, DO, STAGES, false>;
-  k.grid = dim3((unsigned)((int64_t)p.n_nblocks * launch_pairs(p) * (DP / DO) *
+  k.fn = causal ? (const void*)bwd_dkv_kernel<T, DP, DC, DO, STAGES, true>
+                : (const void*)bwd_dkv_kernel<T, DP, DC, DO, STAGES, false>;
+  k.grid = dim3((unsigned)((int64_t)p.n_nblocks * launch_pairs(p) * (DC / DO) *
                            (p.kv_iters > 0 ? p.kv_chunks : 1)));
   k.block = dim3(512);
   k.kernel = "bwd_dkv_kernel";
@@ -1506,15 +1511,15 @@ static KernelPlan plan_dkv_t(BwdParams& p, bool causal) {
   return k;
 }
 
-template <class T, int DP>
+template <class T, int DP, int DC = DP>
 static KernelPlan plan_dq_t(BwdParams& p, bool causal) {
   constexpr int NW = 4;  // dQ waves per workgroup
   constexpr int STAGES = 4;
   using QC = DqConfig<DP>;
   p.n_mblocks = (p.Sq + 32 * NW - 1) / (32 * NW);
   KernelPlan k;
-  k.fn = causal ? (const void*)bwd_dq_kernel<T, DP, QC::kBn, NW, STAGES, QC::kOcc, QC::kMode, true>
-                : (const void*)bwd_dq_kernel<T, DP, QC::kBn, NW, STAGES, QC::kOcc, QC::kMode, false>;
+  k.fn = causal ? (const void*)bwd_dq_kernel<T, DP, DC, QC::kBn, NW, STAGES, QC::kOcc, QC::kMode, true>
+                : (const void*)bwd_dq_kernel<T, DP, DC, QC::kBn, NW, STAGES, QC::kOcc, QC::kMode, false>;
   k.grid = dim3((unsigned)((int64_t)p.n_mblocks * p.B * p.Hq));
   k.block = dim3(NW * 64);
   k.kernel = "bwd_dq_kernel";
@@ -1530,6 +1535,9 @@ static KernelPlan plan_dq_t(BwdParams& p, bool causal) {
 template <class T>
 static KernelPlan plan_dkv_dt(BwdParams& p, bool causal) {
   if (p.D <= 64) return plan_dkv_t<T, 64, 64>(p, causal);
+  // Up to 96: the D = 128 tiles with three quarters of the MFMAs (here and in
+  // both dQ kernels).
+  if (p.D <= 96) return plan_dkv_t<T, 128, 96, 96>(p, causal);
   if (p.D <= 128) return plan_dkv_t<T, 128, 128>(p, causal);
   if (p.D <= 256) return plan_dkv_t<T, 256, SK_BWD_DKV_DO_D256>(p, causal);
   return KernelPlan{};
@@ -1538,6 +1546,7 @@ static KernelPlan plan_dkv_dt(BwdParams& p, bool causal) {
 template <class T>
 static KernelPlan plan_dq_dt(BwdParams& p, bool causal) {
   if (p.D <= 64) return plan_dq_t<T, 64>(p, causal);
+  if (p.D <= 96) return plan_dq_t<T, 128, 96>(p, causal);
   if (p.D <= 128) return plan_dq_t<T, 128>(p, causal);
   if (p.D <= 256) return plan_dq_t<T, 256>(p, causal);
   return KernelPlan{};
@@ -1646,13 +1655,13 @@ void bwd_dkv_split(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D, boo
   *iters = memo.iters, *chunks = memo.chunks;
 }
 
-template <class T>
+template <class T, int DC>
 static KernelPlan plan_dq_ds_t(BwdParams& p, bool causal) {
   constexpr int NW = 4, QW = kDqDs.qw;
   p.n_mblocks = (p.Sq + 32 * QW * NW - 1) / (32 * QW * NW);
   KernelPlan k;
-  k.fn = causal ? (const void*)bwd_dq_ds_kernel<T, 128, QW, kDqDs.stages, kDqDs.occ, true>
-                : (const void*)bwd_dq_ds_kernel<T, 128, QW, kDqDs.stages, kDqDs.occ, false>;
+  k.fn = causal ? (const void*)bwd_dq_ds_kernel<T, 128, DC, QW, kDqDs.stages, kDqDs.occ, true>
+                : (const void*)bwd_dq_ds_kernel<T, 128, DC, QW, kDqDs.stages, kDqDs.occ, false>;
   k.grid = dim3((unsigned)((int64_t)p.n_mblocks * launch_pairs(p) * p.group));
   k.block = dim3(NW * 64);
   k.kernel = "bwd_dq_ds_kernel";
@@ -1668,7 +1677,9 @@ static KernelPlan plan_dq_ds_t(BwdParams& p, bool causal) {
 KernelPlan plan_bwd_dq(int dtype, BwdParams& p, bool causal) {
   if (p.ds != nullptr &&
       bwd_ds_pair_bytes(dtype, p.Hq, p.Hkv, p.Sq, p.Sk, p.D, causal) > 0)
-    return dtype == BF16::code ? plan_dq_ds_t<BF16>(p, causal) : plan_dq_ds_t<F16>(p, causal);
+    return dtype == BF16::code
+               ? (p.D <= 96 ? plan_dq_ds_t<BF16, 96>(p, causal) : plan_dq_ds_t<BF16, 128>(p, causal))
+               : (p.D <= 96 ? plan_dq_ds_t<F16, 96>(p, causal) : plan_dq_ds_t<F16, 128>(p, causal));
   if (dtype == BF16::code) return plan_dq_dt<BF16>(p, causal);
   if (dtype == F16::code) return plan_dq_dt<F16>(p, causal);
   if (dtype == 0) return plan_bwd_dq_f32(p, causal);

@@ -105,13 +105,15 @@ constexpr bool softmax_pairs_fit(int ns, int db, int fl, int ng) {
   return true;
 }
 
-template <class T, int DP, int BN, int NW, int STAGES, int OCC, bool CAUSAL, bool ROPE>
+// DP: the head dim the LDS tiles are laid out for; DC <= DP: the one the
+// MFMAs cover (a multiple of 32, at least D).
+template <class T, int DP, int DC, int BN, int NW, int STAGES, int OCC, bool CAUSAL, bool ROPE>
 __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
   using L = FwdLds<DP, BN>;
   constexpr int BM = 32 * NW;
-  constexpr int KD = DP / 16;  // k-steps over the head dim for S^T
+  constexpr int KD = DC / 16;  // k-steps over the head dim for S^T
   constexpr int KB = BN / 32;  // 32-key blocks per tile
-  constexpr int DB = DP / 32;  // 32-wide head-dim blocks of O^T
+  constexpr int DB = DC / 32;  // 32-wide head-dim blocks of O^T
   constexpr int KN = BN / 16;  // k-steps over keys for O^T
   constexpr int LK = L::kSegs / NW;  // K (and V) segments each wave loads per tile
   constexpr int KT = L::kTileBytes;
@@ -816,18 +818,18 @@ int fwd_key_splits(int dtype, int d, int64_t bh, int sq, int sk, bool causal) {
   return (sk + keys - 1) / keys;
 }
 
-template <class T, int DP, int BN, int NW, int OCC, int STAGES = 4>
+template <class T, int DP, int BN, int NW, int OCC, int STAGES = 4, int DC = DP>
 static KernelPlan plan_fwd_t(const FwdParams& p, bool causal) {
   KernelPlan k;
   const bool rope = p.rope.cos != nullptr;
   if (causal && !rope)
-    k.fn = (const void*)fwd_mfma_kernel<T, DP, BN, NW, STAGES, OCC, true, false>;
+    k.fn = (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, true, false>;
   else if (!rope)
-    k.fn = (const void*)fwd_mfma_kernel<T, DP, BN, NW, STAGES, OCC, false, false>;
+    k.fn = (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, false, false>;
   else if (causal)
-    k.fn = (const void*)fwd_mfma_kernel<T, DP, BN, NW, STAGES, OCC, true, true>;
+    k.fn = (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, true, true>;
   else
-    k.fn = (const void*)fwd_mfma_kernel<T, DP, BN, NW, STAGES, OCC, false, true>;
+    k.fn = (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, false, true>;
   k.grid = dim3((unsigned)(p.n_items * p.B * p.Hq * std::max(1, p.n_splits)));
   k.block = dim3(NW * 64);
   k.kernel = "fwd_mfma_kernel";
@@ -852,6 +854,13 @@ static KernelPlan plan_fwd_dt(const FwdParams& p, bool causal) {
       return plan_fwd_t<T, 64, kFwdD64Long.bn, kFwdD64Long.nw, kFwdD64Long.occ,
                         kFwdD64Long.stages>(p, causal);
     case 128:
+      // Up to 96: the same tiles with three quarters of the MFMAs.
+      if (p.D <= 96 && sh)
+        return plan_fwd_t<T, 128, kFwdD128Short.bn, kFwdD128Short.nw, kFwdD128Short.occ,
+                          kFwdD128Short.stages, 96>(p, causal);
+      if (p.D <= 96)
+        return plan_fwd_t<T, 128, kFwdD128Long.bn, kFwdD128Long.nw, kFwdD128Long.occ,
+                          kFwdD128Long.stages, 96>(p, causal);
       if (sh)
         return plan_fwd_t<T, 128, kFwdD128Short.bn, kFwdD128Short.nw, kFwdD128Short.occ,
                           kFwdD128Short.stages>(p, causal);
