@@ -314,7 +314,7 @@ static int fwd_impl(int dtype, const void* q, const void* k, const void* v, void
     // One query block per workgroup and split (pairing evens out the causal
     // triangle on full grids only).
     p.pair_items = 0;
-    p.n_items = p.n_mblocks;
+    p.n_items = p.n_mblocks = sk::fwd_split_blocks(Sq);
     p.n_splits = splits;
     p.split_keys = sk::fwd_split_keys(Sk, splits);
     p.part_o = (float*)workspace;

@@ -106,8 +106,11 @@ constexpr bool softmax_pairs_fit(int ns, int db, int fl, int ng) {
 }
 
 // DP: the head dim the LDS tiles are laid out for; DC <= DP: the one the
-// MFMAs cover (a multiple of 32, at least D).
-template <class T, int DP, int DC, int BN, int NW, int STAGES, int OCC, bool CAUSAL, bool ROPE>
+// MFMAs cover (a multiple of 32, at least D).  SPLIT: key splits that write
+// partials (a kernel of its own: their epilogue in every kernel cost the
+// unsplit forward 0.7% at S = 4,096).
+template <class T, int DP, int DC, int BN, int NW, int STAGES, int OCC, bool CAUSAL, bool ROPE,
+          bool SPLIT>
 __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
   using L = FwdLds<DP, BN>;
   constexpr int BM = 32 * NW;
@@ -142,19 +145,18 @@ __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
   // With key splits the item's splits are neighbours, so the query blocks of a
   // head that read one key range run side by side.
   const int w = xcd_work_index(blockIdx.x, gridDim.x);
-  const int ns = max(1, p.n_splits);
-  const int iw = w / ns;
-  const int split = w - iw * ns;
+  const int iw = SPLIT ? w / p.n_splits : w;
+  const int split = SPLIT ? w - iw * p.n_splits : 0;
   int bh = iw / p.n_items;
   int item = iw - bh * p.n_items;
-  if (p.heavy_first) heavy_first_order(blockIdx.x, p.B * p.Hq, bh, item);
+  if (CAUSAL && !SPLIT && p.heavy_first) heavy_first_order(blockIdx.x, p.B * p.Hq, bh, item);
   const int b = bh / p.Hq;
   const int hq = bh % p.Hq;
   const int hkv = hq / p.group;
   // The split's keys: sk of them from n_lo, numbered from 0 below (so query i
   // sees key j of them iff j <= i + diag).
-  const int n_lo = split * p.split_keys;
-  const int sk = ns > 1 ? min(p.split_keys, p.Sk - n_lo) : p.Sk;
+  const int n_lo = SPLIT ? split * p.split_keys : 0;
+  const int sk = SPLIT ? min(p.split_keys, p.Sk - n_lo) : p.Sk;
   const int diag = p.Sk - p.Sq - n_lo;
 
   const uint16_t* kbase =
@@ -571,7 +573,7 @@ __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
   }
 
   const float l_tot = xhalf_sum(l_run);
-  if (ns > 1) {
+  if constexpr (SPLIT) {
     // A split's partial: a row that saw no key leaves its output unwritten
     // (the combine skips it); a NaN row keeps its NaN.
     if (row < p.Sq) {
@@ -620,7 +622,7 @@ __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
   const int first = p.n_mblocks - 1 - item;  // heaviest block first
   run_item(first);
   const int second = item;
-  if (p.pair_items && second != first) {
+  if (!SPLIT && p.pair_items && second != first) {
     __syncthreads();  // every wave is done with the LDS ring before it is refilled
     run_item(second);
   }
@@ -789,6 +791,8 @@ int fwd_pair_min(int dtype, int d, int64_t bh, int sq, int sk, bool causal) {
 // A predicted gain under 15% is left alone (causal squares, whose blocks
 // differ: 1,000 x 1,000 at 8 heads 20 us either way), and from 384 query
 // blocks on (1.5 per CU) nothing is split.
+int fwd_split_blocks(int sq) { return (sq + 127) / 128; }
+
 int fwd_split_keys(int sk, int splits) {
   const int per = (sk + splits - 1) / splits;
   return (per + 63) / 64 * 64;
@@ -797,18 +801,18 @@ int fwd_split_keys(int sk, int splits) {
 int fwd_key_splits(int dtype, int d, int64_t bh, int sq, int sk, bool causal) {
   if (dtype != BF16::code && dtype != F16::code) return 1;
   if (sq <= 0 || sk <= 0 || bh <= 0) return 1;
-  const FwdConfig c = fwd_config(d, bh, sq, sk, causal);
-  const int64_t items = (sq + 32 * c.nw - 1) / (32 * c.nw) * bh;
+  if (d <= 128 && (d <= 64 ? kFwdD64Short : kFwdD128Short).nw != 4) return 1;  // tile study
+  const int64_t items = (int64_t)fwd_split_blocks(sq) * bh;
   if (items >= 384) return 1;
   const double tile_us = d <= 64 ? 0.5 : d <= 128 ? 1.0 : 1.15;
-  const double tiles = (double)sk / c.bn;
+  const double tiles = (double)sk / (d <= 128 ? 64 : 32);
   const double merge_us = (double)bh * sq * d * 8 / 1.2e7;  // per split
   int best = 1;
   double best_us = 0, one_us = 0;
   for (int ns = 1; ns <= 32; ++ns) {
     if (ns > 1 && sk < ns * 256) break;
     const int64_t load = (items * ns + 255) / 256;
-    const double eff = load > 1 && c.occ > 1 ? 0.95 : 1.0;
+    const double eff = load > 1 && d <= 128 ? 0.95 : 1.0;
     const double us = load * eff * (tiles / ns + 2) * tile_us + (ns > 1 ? 8 + ns * merge_us : 0);
     if (ns == 1) one_us = us;
     if (ns == 1 || us < best_us) best = ns, best_us = us;
@@ -822,14 +826,20 @@ template <class T, int DP, int BN, int NW, int OCC, int STAGES = 4, int DC = DP>
 static KernelPlan plan_fwd_t(const FwdParams& p, bool causal) {
   KernelPlan k;
   const bool rope = p.rope.cos != nullptr;
-  if (causal && !rope)
-    k.fn = (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, true, false>;
-  else if (!rope)
-    k.fn = (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, false, false>;
+  // (Key splits run the 4-wave entries only.)
+  constexpr bool kSplits = NW == 4;
+  if (p.n_splits > 1 && !kSplits) return k;
+  if (kSplits && p.n_splits > 1)
+    k.fn = causal ? (rope ? (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, true, true, kSplits>
+                          : (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, true, false, kSplits>)
+                  : (rope ? (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, false, true, kSplits>
+                          : (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, false, false, kSplits>);
   else if (causal)
-    k.fn = (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, true, true>;
+    k.fn = rope ? (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, true, true, false>
+                : (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, true, false, false>;
   else
-    k.fn = (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, false, true>;
+    k.fn = rope ? (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, false, true, false>
+                : (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, false, false, false>;
   k.grid = dim3((unsigned)(p.n_items * p.B * p.Hq * std::max(1, p.n_splits)));
   k.block = dim3(NW * 64);
   k.kernel = "fwd_mfma_kernel";
@@ -845,7 +855,7 @@ static KernelPlan plan_fwd_t(const FwdParams& p, bool causal) {
 
 template <class T>
 static KernelPlan plan_fwd_dt(const FwdParams& p, bool causal) {
-  const bool sh = fwd_short(p.D, (int64_t)p.B * p.Hq, p.Sq, p.Sk, causal);
+  const bool sh = p.n_splits > 1 || fwd_short(p.D, (int64_t)p.B * p.Hq, p.Sq, p.Sk, causal);
   switch (fwd_config(p.D, (int64_t)p.B * p.Hq, p.Sq, p.Sk, causal).dp) {
     case 64:
       if (sh)

@@ -316,6 +316,9 @@ int fwd_pair_min(int dtype, int d, int64_t bh, int sq, int sk, bool causal);
 // keys each covers.
 int fwd_key_splits(int dtype, int d, int64_t bh, int sq, int sk, bool causal);
 int fwd_split_keys(int sk, int splits);
+// Query blocks per (batch, head) of a split forward (its kernels are the
+// 4-wave entries, 128 rows a workgroup, at every head dim).
+int fwd_split_blocks(int sq);
 // Padded head dim the kernels are compiled for (64, 96, 128 or 256), or 0.
 int padded_head_dim(int d);
 
