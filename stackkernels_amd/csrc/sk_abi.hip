@@ -189,22 +189,27 @@ size_t bwd_ws_bytes(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D, bo
   return bwd_rows_bytes(B, Hq, Sq) + (size_t)chunk * pair;
 }
 
-// Offset of the split dK/dV's partial sums in the workspace, and their bytes
-// (0: the shape runs unsplit, or its pairs in several chunks).
-struct DkvParts {
+// Splits of the backward's kernels (kv_iters .. dq_chunks of p), and the
+// offset and bytes of their partial sums in the workspace (0: the shape runs
+// unsplit, or its pairs in several chunks).
+struct BwdParts {
   size_t offset = 0, bytes = 0;
-  int iters = 0, chunks = 1;
+  sk::BwdParams p{};
 };
-DkvParts bwd_parts(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D, bool causal) {
-  DkvParts r;
-  sk::bwd_dkv_split(dtype, B, Hq, Hkv, Sq, Sk, D, causal, &r.iters, &r.chunks);
+BwdParts bwd_parts(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D, bool causal) {
+  BwdParts r;
+  if (dtype == SK_F32)
+    sk::bwd_f32_split(B, Hq, Hkv, Sq, Sk, D, causal, &r.p);
+  else
+    sk::bwd_dkv_split(dtype, B, Hq, Hkv, Sq, Sk, D, causal, &r.p.kv_iters, &r.p.kv_chunks);
   const size_t pair = sk::bwd_ds_pair_bytes(dtype, Hq, Hkv, Sq, Sk, D, causal);
   const int64_t pairs = (int64_t)B * Hkv;
-  if (r.iters <= 0 ||
+  if ((r.p.kv_iters <= 0 && r.p.dq_iters <= 0) ||
       (pair > 0 && bwd_chunk_pairs(pairs, pair, (size_t)SK_BWD_DS_CAP_BYTES) != pairs))
-    return DkvParts{};
+    return BwdParts{};
   r.offset = (bwd_ws_bytes(dtype, B, Hq, Hkv, Sq, Sk, D, causal) + 255) / 256 * 256;
-  r.bytes = (size_t)2 * r.chunks * pairs * Sk * D * sizeof(float);
+  if (r.p.kv_iters > 0) r.bytes += (size_t)2 * r.p.kv_chunks * pairs * Sk * D * sizeof(float);
+  if (r.p.dq_iters > 0) r.bytes += (size_t)r.p.dq_chunks * B * Hq * Sq * D * sizeof(float);
   return r;
 }
 
@@ -303,8 +308,8 @@ static int fwd_impl(int dtype, const void* q, const void* k, const void* v, void
   if (splits == 0) {
     splits = fwd_splits(dtype, B, Hq, Sq, Sk, D, is_causal != 0, workspace_bytes);
   } else if (splits > 1) {
-    if (dtype == SK_F32) splits = 1;
-    const int keys = sk::fwd_split_keys(Sk, splits);
+    if (dtype == SK_F32 && sk::fwd_f32_rows_per_block(D, Sq) < 256) splits = 1;  // vector kernel
+    const int keys = splits > 1 ? sk::fwd_split_keys(Sk, splits) : 0;
     splits = keys > 0 ? (Sk + keys - 1) / keys : 1;
     const size_t need = fwd_ws_bytes(B, Hq, Sq, D, splits);
     if (need > workspace_bytes)
@@ -314,7 +319,8 @@ static int fwd_impl(int dtype, const void* q, const void* k, const void* v, void
     // One query block per workgroup and split (pairing evens out the causal
     // triangle on full grids only).
     p.pair_items = 0;
-    p.n_items = p.n_mblocks = sk::fwd_split_blocks(Sq);
+    if (dtype != SK_F32) p.n_mblocks = sk::fwd_split_blocks(Sq);
+    p.n_items = p.n_mblocks;
     p.n_splits = splits;
     p.split_keys = sk::fwd_split_keys(Sk, splits);
     p.part_o = (float*)workspace;
@@ -408,7 +414,7 @@ int sk_attn_bwd_workspace_best(int dtype, int B, int Hq, int Hkv, int Sq, int Sk
                                int is_causal, size_t* bytes) {
   const int rc = sk_attn_bwd_workspace(dtype, B, Hq, Hkv, Sq, Sk, D, is_causal, bytes);
   if (rc) return rc;
-  const DkvParts parts = bwd_parts(dtype, B, Hq, Hkv, Sq, Sk, D, is_causal != 0);
+  const BwdParts parts = bwd_parts(dtype, B, Hq, Hkv, Sq, Sk, D, is_causal != 0);
   if (parts.bytes > 0) *bytes = parts.offset + parts.bytes;
   return SK_OK;
 }
@@ -463,13 +469,18 @@ int sk_attn_bwd(int dtype, const void* dout, const void* q, const void* k, const
   p.ds = chunk > 0 ? (char*)workspace + need : nullptr;
   p.n_pairs = (int)chunk;
   p.bk0 = 0;
-  // Split dK/dV where the workspace holds its partial sums as well.
-  const DkvParts parts = bwd_parts(dtype, B, Hq, Hkv, Sq, Sk, D, is_causal != 0);
+  // Split kernels where the workspace holds their partial sums as well.
+  const BwdParts parts = bwd_parts(dtype, B, Hq, Hkv, Sq, Sk, D, is_causal != 0);
   if (parts.bytes > 0 && workspace_bytes >= parts.offset + parts.bytes) {
-    p.kv_iters = parts.iters;
-    p.kv_chunks = parts.chunks;
-    p.part_dk = (float*)((char*)workspace + parts.offset);
-    p.part_dv = p.part_dk + (size_t)parts.chunks * B * Hkv * Sk * D;
+    p.kv_iters = parts.p.kv_iters, p.kv_chunks = parts.p.kv_chunks;
+    p.dq_iters = parts.p.dq_iters, p.dq_chunks = parts.p.dq_chunks;
+    float* part = (float*)((char*)workspace + parts.offset);
+    if (p.kv_iters > 0) {
+      const size_t n = (size_t)p.kv_chunks * B * Hkv * Sk * D;
+      p.part_dk = part, p.part_dv = part + n;
+      part += 2 * n;
+    }
+    p.part_dq = part;
   }
   p.ds_nqt = (Sq + 31) / 32;
   p.ds_c = sk::ds_causal_c(Sq, Sk);

@@ -1585,17 +1585,51 @@ size_t bwd_ds_pair_bytes(int dtype, int Hq, int Hkv, int Sq, int Sk, int D, bool
 // Microseconds of one dK/dV step (32 queries against 128 keys) of a workgroup.
 static double dkv_step_us(int d) { return d <= 64 ? 0.45 : d <= 128 ? 0.85 : 1.5; }
 
+// Chunk length (steps) for a grid of blocks of steps[0..n) steps, each sample
+// standing for `stands_for` workgroups, one resident per CU; 0: unsplit.  It
+// minimises the grid's time: the chunk while they fit one round, else, where
+// the blocks differ (causal), the mean load plus half a chunk, or whole
+// rounds; each with `fixed` steps of prologue and epilogue per workgroup, plus
+// chunk_us of partial sums written and read per chunk and 4 us for the merge.
+// Unsplit, heavy blocks first: the heaviest block or the mean load.
+int best_chunk(const int* steps, int n, double stands_for, bool causal, double step_us,
+               double fixed, double chunk_us) {
+  double total = 0;
+  int longest = 0;
+  for (int i = 0; i < n; ++i) total += steps[i], longest = std::max(longest, steps[i]);
+  total *= stands_for;
+  const double wgs = stands_for * n;
+  const double whole = causal ? std::max<double>(longest, 1.05 * total / 256)
+                              : std::ceil(wgs / 256) * longest;
+  double best_us = 0.9 * (whole + fixed * std::ceil(wgs / 256)) * step_us;
+  int best = 0;
+  static const int kCuts[] = {2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 32, 48, 64};
+  for (int cut : kCuts) {
+    const int len = (longest + cut - 1) / cut;
+    if (len * step_us < 3) break;  // a chunk's fixed cost would be most of it
+    double m = 0, split = 0;  // workgroups; those that write partials
+    for (int i = 0; i < n; ++i) {
+      const int c = dkv_chunks(steps[i], len);
+      m += c;
+      if (c > 1) split += c;
+    }
+    m *= stands_for, split *= stands_for;
+    const double load = m <= 256 ? len + fixed
+                        : causal ? std::max<double>(len, total / 256 + 0.5 * len) + fixed * m / 256
+                                 : std::ceil(m / 256) * (len + fixed);
+    const double us = load * step_us + split * chunk_us + 4;
+    if (us < best_us) best_us = us, best = len;
+  }
+  return best;
+}
+
 // Split of the dK/dV kernel where its workgroups (one per CU) leave CUs idle
 // or, under the causal mask, unevenly loaded.
-// The chunk length minimises the kernel's time in steps: one chunk per CU
-// while they fit one round (their length), else the mean load plus half a
-// chunk, each with 4 steps of prologue and epilogue per workgroup, plus the
-// partial sums' write and read at 5 TB/s and 4 us for the merge.  Unsplit, heavy blocks
-// first: the heaviest block or the mean load.  Measured (forward excluded,
-// bf16, H_q = 32, H_kv = 8, D = 128, causal): B = 1, S = 2,000 281 -> 171 us
-// (128 workgroups, now 240), B = 2, S = 1,337 204 -> 171; MQA, B = 2, S = 2,048
-// 1,686 -> 339 (32 workgroups).  At B = 4, S = 2,048 (512 workgroups) unsplit
-// and heavy first is the faster one, 462 us against 479.
+// Measured (forward excluded, bf16, H_q = 32, H_kv = 8, D = 128, causal): B =
+// 1, S = 2,000 281 -> 171 us (128 workgroups, now 240), B = 2, S = 1,337 204
+// -> 171; MQA, B = 2, S = 2,048 1,686 -> 339 us (32 workgroups).  At B = 4, S =
+// 2,048 (512 workgroups) unsplit and heavy first is the faster one, 462 us
+// against 479.
 void bwd_dkv_split(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D, bool causal,
                    int* iters, int* chunks) {
   *iters = 0, *chunks = 1;
@@ -1612,46 +1646,18 @@ void bwd_dkv_split(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D, boo
   };
   static thread_local Memo memo = {};
   const int key[7] = {B, Hq, Hkv, Sq, Sk, D, (int)causal};
-  if (std::equal(key, key + 7, memo.key)) {
-    *iters = memo.iters, *chunks = memo.chunks;
-    return;
+  if (!std::equal(key, key + 7, memo.key)) {
+    // Steps of up to 64 evenly spaced key blocks stand for all of them.
+    const int n = (int)std::min<int64_t>(nb, 64);
+    int steps[64];
+    for (int i = 0; i < n; ++i) steps[i] = group * dkv_tiles((int)(i * nb / n), Sq, Sk, causal);
+    const double stands_for = (double)pairs * parts * nb / n;
+    const int best = best_chunk(steps, n, stands_for, causal, dkv_step_us(D), 4,
+                                128.0 * D * 8 * 2 / 5e6 / parts);
+    memo.iters = best;
+    memo.chunks = best > 0 ? dkv_chunks(steps[0], best) : 1;
+    std::copy(key, key + 7, memo.key);
   }
-  const double step_us = dkv_step_us(D);
-  // Steps of up to 64 evenly spaced key blocks stand for all of them.
-  const int ns = (int)std::min<int64_t>(nb, 64);
-  int steps[64];
-  double total = 0;
-  for (int i = 0; i < ns; ++i) {
-    steps[i] = group * dkv_tiles((int)(i * nb / ns), Sq, Sk, causal);
-    total += steps[i];
-  }
-  const double scale = (double)pairs * parts * nb / ns;  // workgroups a sample stands for
-  total *= scale;
-  const double longest = steps[0];
-  const double wgs = scale * ns;
-  const double whole = causal ? std::max(longest, 1.05 * total / 256)
-                              : std::ceil(wgs / 256) * longest;
-  const double unsplit_us = (whole + 4 * std::ceil(wgs / 256)) * step_us;
-  double best_us = 0.9 * unsplit_us;
-  int best = 0;
-  static const int kCuts[] = {2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 32, 48, 64};
-  for (int cut : kCuts) {
-    const int len = (steps[0] + cut - 1) / cut;
-    if (len < 8) break;
-    double n = 0, split = 0;  // workgroups; those that write partials
-    for (int i = 0; i < ns; ++i) {
-      const int c = dkv_chunks(steps[i], len);
-      n += c;
-      if (c > 1) split += c;
-    }
-    n *= scale, split *= scale / parts;
-    const double load = n <= 256 ? len + 4.0 : std::max<double>(len, total / 256 + 0.5 * len) + 4 * n / 256;
-    const double us = load * step_us + split * 128 * D * 8 * 2 / 5e6 + 4;
-    if (us < best_us) best_us = us, best = len;
-  }
-  memo = Memo{{}, best, 1};
-  std::copy(key, key + 7, memo.key);
-  if (best > 0) memo.chunks = dkv_chunks(steps[0], best);
   *iters = memo.iters, *chunks = memo.chunks;
 }
 

@@ -9,6 +9,8 @@
 // share one row, each holding a quarter of the head dimension, and q.k
 // partial sums are combined with two cross-lane adds; K/V (or Q/dO) tiles of
 // 16 rows are staged in LDS and the online softmax is updated once per tile.
+#include <algorithm>
+
 #include "sk_common.h"
 #include "sk_kernels.h"
 #include "sk_rope.h"
@@ -160,7 +162,9 @@ __global__ void __launch_bounds__(256) fwd_f32_kernel(FwdParams p) {
 //   path as in fwd_f32_kernel.
 constexpr int kF32MmaRows = 256;
 
-template <int DP, bool CAUSAL>
+// SPLIT: key splits that write fp32 partials for fwd_combine_kernel
+// (FwdParams::n_splits).
+template <int DP, bool CAUSAL, bool SPLIT>
 __global__ void __launch_bounds__(512, 1) fwd_f32_mfma_kernel(FwdParams p) {
   constexpr int NW = 8;
   constexpr int BN = 64;
@@ -185,14 +189,19 @@ __global__ void __launch_bounds__(512, 1) fwd_f32_mfma_kernel(FwdParams p) {
 
   // Heaviest query block first under the causal mask; XCD-aware order.
   const int w = xcd_work_index(blockIdx.x, gridDim.x);
-  const int bh = w / p.n_mblocks;
-  const int mblk = p.n_mblocks - 1 - (w - bh * p.n_mblocks);
+  const int iw = SPLIT ? w / p.n_splits : w;
+  const int split = SPLIT ? w - iw * p.n_splits : 0;
+  const int bh = iw / p.n_mblocks;
+  const int mblk = p.n_mblocks - 1 - (iw - bh * p.n_mblocks);
   const int b = bh / p.Hq, hq = bh % p.Hq, hkv = hq / p.group;
   const int m0 = mblk * kF32MmaRows;
   const int mw = m0 + 32 * wave;
   const int row = mw + l32;
   const bool row_ok = row < p.Sq;
-  const int diag = p.Sk - p.Sq;
+  // The split's keys, numbered from 0: sk of them from n_lo.
+  const int n_lo = SPLIT ? split * p.split_keys : 0;
+  const int sk = SPLIT ? min(p.split_keys, p.Sk - n_lo) : p.Sk;
+  const int diag = p.Sk - p.Sq - n_lo;
 
   // Q^T operand: lane holds q[row][hl * KS + s] at k-step s (rotated when
   // the call carries RoPE tables; zero past S_q and D; negated for a
@@ -226,8 +235,8 @@ __global__ void __launch_bounds__(512, 1) fwd_f32_mfma_kernel(FwdParams p) {
 
   // DMA: segment j of this wave is segment wave + 8 j of the tile; the
   // lane's global byte offset of the chunk that lands at its LDS slot.
-  const float* kbase = (const float*)p.k + b * p.k_sb + hkv * p.k_sh;
-  const float* vbase = (const float*)p.v + b * p.v_sb + hkv * p.v_sh;
+  const float* kbase = (const float*)p.k + b * p.k_sb + hkv * p.k_sh + (int64_t)n_lo * p.k_ss;
+  const float* vbase = (const float*)p.v + b * p.v_sb + hkv * p.v_sh + (int64_t)n_lo * p.v_ss;
   uint32_t koff[LK], voff[LK];
 #pragma unroll
   for (int j = 0; j < LK; ++j) {
@@ -243,7 +252,7 @@ __global__ void __launch_bounds__(512, 1) fwd_f32_mfma_kernel(FwdParams p) {
   };
   auto issue = [&](int t) {
     const int n0 = t * BN;
-    const int rows = min(BN, p.Sk - n0);
+    const int rows = min(BN, sk - n0);
     const int st = t & 1;
     const i32x4 kr = make_rsrc_words(kbase + (int64_t)n0 * p.k_ss, range(rows, p.k_ss));
     const i32x4 vr = make_rsrc_words(vbase + (int64_t)n0 * p.v_ss, range(rows, p.v_ss));
@@ -255,8 +264,8 @@ __global__ void __launch_bounds__(512, 1) fwd_f32_mfma_kernel(FwdParams p) {
       buffer_load_lds_b128(vr, lds0 + (2 + st) * KT + (wave + j * NW) * 1024, voff[j]);
   };
 
-  int n_end = p.Sk;
-  if (CAUSAL) n_end = min(p.Sk, m0 + kF32MmaRows + diag);
+  int n_end = sk;
+  if (CAUSAL) n_end = min(sk, m0 + kF32MmaRows + diag);
   const int n_tiles = n_end > 0 ? (n_end + BN - 1) / BN : 0;
   // Tiles [0, vis) hold keys this wave's rows can see.
   int vis = mw < p.Sq ? n_tiles : 0;
@@ -299,8 +308,8 @@ __global__ void __launch_bounds__(512, 1) fwd_f32_mfma_kernel(FwdParams p) {
     }
     // Register r of block kb: key n0 + 32 kb + 8 (r/4) + 4 hl + r%4.
     const int n0 = t * BN;
-    if (n0 + BN > p.Sk || (CAUSAL && n0 + BN - 1 > mw + diag)) {
-      int lim = p.Sk - 1;
+    if (n0 + BN > sk || (CAUSAL && n0 + BN - 1 > mw + diag)) {
+      int lim = sk - 1;
       if (CAUSAL) lim = min(lim, row + diag);
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
@@ -344,6 +353,27 @@ __global__ void __launch_bounds__(512, 1) fwd_f32_mfma_kernel(FwdParams p) {
   const float l_tot = xhalf_sum(l_run);
   if (!row_ok) return;
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+  if constexpr (SPLIT) {
+    // (A row that saw no key leaves its output unwritten; a NaN stays NaN.)
+    const int64_t r = ((int64_t)split * p.B * p.Hq + bh) * p.Sq + row;
+    if (l_tot != 0.f) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int d = DB * (8 * (i >> 2) + 4 * hl + (i & 3));
+        if (d < p.D) {
+          vrow_t x;
+#pragma unroll
+          for (int c = 0; c < DB; ++c) x[c] = oacc[c][i] * inv;
+          *reinterpret_cast<vrow_t*>(p.part_o + r * p.D + d) = x;
+        }
+      }
+    }
+    if (hl == 0)
+      p.part_lse[r] = l_tot > 0.f    ? m_run * p.scale + logf(l_tot)
+                      : l_tot == 0.f ? kNegInf
+                                     : l_tot;
+    return;
+  }
   float* op = (float*)p.o + b * p.o_sb + hq * p.o_sh + (int64_t)row * p.o_ss;
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
@@ -590,13 +620,43 @@ static bool fwd_f32_on_mfma(int d, int sq) {
   return SK_F32_MFMA && dp > 0 && dp <= 128 && sq >= 32;
 }
 
+// Key splits of the matrix-core forward, one 256-row workgroup per CU: the
+// model of fwd_key_splits with its tile times (64 keys: 8.4 us at D <= 64,
+// 16.5 at 128; half a tile of prologue).  B * H = 16, S = 1,024, D = 64: 64
+// workgroups 135 us, 4 splits 58 with the merge (MQA, 8 heads, 300 x 3,000, D =
+// 96: 703 and 72).
+int fwd_f32_key_splits(int d, int64_t bh, int sq, int sk) {
+  if (!fwd_f32_on_mfma(d, sq) || sk <= 0 || bh <= 0) return 1;
+  const int64_t items = (int64_t)((sq + kF32MmaRows - 1) / kF32MmaRows) * bh;
+  if (items >= 384) return 1;
+  const double tile_us = d <= 64 ? 8.4 : 16.5;
+  const double tiles = sk / 64.0;
+  const double merge_us = (double)bh * sq * d * 8 / 1.2e7;
+  int best = 1;
+  double best_us = 0, one_us = 0;
+  for (int ns = 1; ns <= 32; ++ns) {
+    if (ns > 1 && sk < ns * 64) break;
+    const int64_t load = (items * ns + 255) / 256;
+    const double us = load * (tiles / ns + 0.5) * tile_us + (ns > 1 ? 8 + ns * merge_us : 0);
+    if (ns == 1) one_us = us;
+    if (ns == 1 || us < best_us) best = ns, best_us = us;
+  }
+  if (best_us > 0.85 * one_us) return 1;
+  const int keys = fwd_split_keys(sk, best);
+  return (sk + keys - 1) / keys;
+}
+
 int fwd_f32_rows_per_block(int d, int sq) { return fwd_f32_on_mfma(d, sq) ? kF32MmaRows : kF32Rows; }
 
 template <int DP>
 static KernelPlan plan_fwd_f32_mfma(const FwdParams& p, bool causal) {
   KernelPlan k;
-  k.fn = causal ? (const void*)fwd_f32_mfma_kernel<DP, true> : (const void*)fwd_f32_mfma_kernel<DP, false>;
-  k.grid = dim3((unsigned)(p.n_mblocks * p.B * p.Hq));
+  const bool split = p.n_splits > 1;
+  k.fn = causal ? (split ? (const void*)fwd_f32_mfma_kernel<DP, true, true>
+                         : (const void*)fwd_f32_mfma_kernel<DP, true, false>)
+                : (split ? (const void*)fwd_f32_mfma_kernel<DP, false, true>
+                         : (const void*)fwd_f32_mfma_kernel<DP, false, false>);
+  k.grid = dim3((unsigned)(p.n_mblocks * p.B * p.Hq * (split ? p.n_splits : 1)));
   k.block = dim3(512);
   k.kernel = "fwd_f32_mfma_kernel";
   k.elem = 0;
@@ -672,7 +732,7 @@ __device__ __forceinline__ int f32_piece(int r, int m) {
 // 32-key K and V tiles stream.  S^T = K Q^T and dP^T = V dO^T (two chains),
 // then dQ^T += K^T dS^T.
 template <int DP, bool CAUSAL>
-__global__ void __launch_bounds__(256, 1) bwd_dq_f32_mfma_kernel(BwdParams p) {
+__global__ void __launch_bounds__(256, DP == 64 ? 2 : 1) bwd_dq_f32_mfma_kernel(BwdParams p) {
   constexpr int NW = 4, BN = kF32MmaTile, BM = 32 * NW;
   constexpr int KS = DP / 2, DB = DP / 32, RB = DP * 4, KT = BN * RB;
   constexpr int CPR = RB / 16, SEGR = 1024 / RB, LK = KT / 1024 / NW;
@@ -686,15 +746,37 @@ __global__ void __launch_bounds__(256, 1) bwd_dq_f32_mfma_kernel(BwdParams p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31;
   const int hl = lane >> 5;
-  const int w = xcd_work_index(blockIdx.x, gridDim.x);
-  const int bh = w / p.n_mblocks;
-  const int mblk = p.n_mblocks - 1 - (w - bh * p.n_mblocks);
+  // A split launch (BwdParams::dq_iters) goes chunk by chunk, heads fastest.
+  int bh, mblk, chunk = 0;
+  if (p.dq_iters > 0) {
+    const int heads = p.B * p.Hq;
+    const int idx = blockIdx.x / heads;
+    bh = blockIdx.x - idx * heads;
+    chunk = idx / p.n_mblocks;
+    mblk = idx - chunk * p.n_mblocks;
+  } else {
+    const int w = xcd_work_index(blockIdx.x, gridDim.x);
+    bh = w / p.n_mblocks;
+    mblk = w - bh * p.n_mblocks;
+  }
+  mblk = p.n_mblocks - 1 - mblk;
   const int b = bh / p.Hq, hq = bh % p.Hq, hkv = hq / p.group;
   const int m0 = mblk * BM;
   const int mw = m0 + 32 * wave;
   const int row = mw + l32;
   const bool row_ok = row < p.Sq;
   const int diag = p.Sk - p.Sq;
+
+  // Key tiles [t0, n_tiles) of the block's, or this chunk's share of them.
+  int n_tiles = dq_tiles(mblk, p.Sq, p.Sk, CAUSAL);
+  int t0 = 0, n_chunks = 1;
+  if (p.dq_iters > 0) {
+    n_chunks = dkv_chunks(n_tiles, p.dq_iters);
+    if (chunk >= n_chunks) return;
+    const int per = (n_tiles + n_chunks - 1) / n_chunks;
+    t0 = min(chunk * per, n_tiles);
+    n_tiles = min(t0 + per, n_tiles);
+  }
 
   const int64_t qrow = ((int64_t)bh * p.Sq + row) * p.D;
   float qv[KS], gv[KS];
@@ -735,9 +817,6 @@ __global__ void __launch_bounds__(256, 1) bwd_dq_f32_mfma_kernel(BwdParams p) {
       buffer_load_lds_b128(vr, lds0 + (2 + st) * KT + (wave + j * NW) * 1024, goff[j]);
   };
 
-  int n_end = p.Sk;
-  if (CAUSAL) n_end = min(p.Sk, m0 + BM + diag);
-  const int n_tiles = n_end > 0 ? (n_end + BN - 1) / BN : 0;
   int vis = mw < p.Sq ? n_tiles : 0;
   if (CAUSAL) {
     const int last_key = mw + 31 + diag;
@@ -754,8 +833,8 @@ __global__ void __launch_bounds__(256, 1) bwd_dq_f32_mfma_kernel(BwdParams p) {
   f32x16 acc[DB];
 #pragma unroll
   for (int c = 0; c < DB; ++c) acc[c] = f32x16{};
-  if (n_tiles > 0) issue(0);
-  for (int t = 0; t < n_tiles; ++t) {
+  if (t0 < n_tiles) issue(t0);
+  for (int t = t0; t < n_tiles; ++t) {
     wait_vmcnt<0>();  // tile t landed for this wave ...
     __syncthreads();  // ... and for all; every read of tile t-1 retired
     if (t + 1 < n_tiles) issue(t + 1);
@@ -791,14 +870,17 @@ __global__ void __launch_bounds__(256, 1) bwd_dq_f32_mfma_kernel(BwdParams p) {
     }
   }
   if (!row_ok) return;
+  float* out = n_chunks > 1 ? p.part_dq + (int64_t)chunk * p.B * p.Hq * p.Sq * p.D + qrow
+                            : (float*)p.dq + qrow;
+  const float qs = n_chunks > 1 ? 1.f : p.scale;
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int d = DB * (8 * (r >> 2) + 4 * hl + (r & 3));
     if (d < p.D) {
       vrow_t x;
 #pragma unroll
-      for (int c = 0; c < DB; ++c) x[c] = acc[c][r] * p.scale;
-      *reinterpret_cast<vrow_t*>((float*)p.dq + qrow + d) = x;
+      for (int c = 0; c < DB; ++c) x[c] = acc[c][r] * qs;
+      *reinterpret_cast<vrow_t*>(out + d) = x;
     }
   }
 }
@@ -808,7 +890,7 @@ __global__ void __launch_bounds__(256, 1) bwd_dq_f32_mfma_kernel(BwdParams p) {
 // statistics), so the GQA sum happens in registers.  S = Q K^T and dP = dO
 // V^T (two chains), then dV^T += dO^T P and dK^T += Q^T dS.
 template <int DP, bool CAUSAL>
-__global__ void __launch_bounds__(256, 1) bwd_dkv_f32_mfma_kernel(BwdParams p) {
+__global__ void __launch_bounds__(256, DP == 64 ? 2 : 1) bwd_dkv_f32_mfma_kernel(BwdParams p) {
   constexpr int NW = 4, BMQ = kF32MmaTile, BNK = 32 * NW;
   constexpr int KS = DP / 2, DB = DP / 32, RB = DP * 4, QT = BMQ * RB;
   constexpr int CPR = RB / 16, SEGR = 1024 / RB, LQ = QT / 1024 / NW;
@@ -824,15 +906,37 @@ __global__ void __launch_bounds__(256, 1) bwd_dkv_f32_mfma_kernel(BwdParams p) {
   const int l32 = lane & 31;
   const int hl = lane >> 5;
   // Lowest key block first: under the causal mask it sees the most queries.
-  const int w = xcd_work_index(blockIdx.x, gridDim.x);
-  const int bk = w / p.n_nblocks;
-  const int nblk = w - bk * p.n_nblocks;
+  // A split launch (BwdParams::kv_iters) goes chunk by chunk, pairs fastest.
+  int bk, nblk, chunk = 0;
+  if (p.kv_iters > 0) {
+    const int pairs = p.B * p.Hkv;
+    const int idx = blockIdx.x / pairs;
+    bk = blockIdx.x - idx * pairs;
+    chunk = idx / p.n_nblocks;
+    nblk = idx - chunk * p.n_nblocks;
+  } else {
+    const int w = xcd_work_index(blockIdx.x, gridDim.x);
+    bk = w / p.n_nblocks;
+    nblk = w - bk * p.n_nblocks;
+  }
   const int b = bk / p.Hkv, hkv = bk % p.Hkv;
   const int n0 = nblk * BNK;
   const int nw = n0 + 32 * wave;
   const int key = nw + l32;
   const bool key_ok = key < p.Sk;
   const int diag = p.Sk - p.Sq;
+
+  // Query tiles that can see a key of this block, and this chunk's share.
+  const int m_begin = dkv_first_query(nblk, p.Sq, p.Sk, CAUSAL);
+  const int n_mt = dkv_tiles(nblk, p.Sq, p.Sk, CAUSAL);
+  int n_it = n0 < p.Sk ? p.group * n_mt : 0, it0 = 0, n_chunks = 1;
+  if (p.kv_iters > 0) {
+    n_chunks = dkv_chunks(n_it, p.kv_iters);
+    if (chunk >= n_chunks) return;
+    const int per = (n_it + n_chunks - 1) / n_chunks;
+    it0 = min(chunk * per, n_it);
+    n_it = min(per, n_it - it0);
+  }
 
   const int64_t krow = ((int64_t)bk * p.Sk + key) * p.D;
   float kv[KS], vv[KS];
@@ -848,12 +952,6 @@ __global__ void __launch_bounds__(256, 1) bwd_dkv_f32_mfma_kernel(BwdParams p) {
     for (int e = 0; e < 4; ++e) kv[4 * j + e] = x[e], vv[4 * j + e] = y[e];
   }
 
-  // Query tiles that can see a key of this block: rows i >= n0 - diag.
-  int m_begin = 0;
-  if (CAUSAL) m_begin = max(0, n0 - diag) / BMQ * BMQ;
-  const int n_mt = m_begin < p.Sq ? (p.Sq - m_begin + BMQ - 1) / BMQ : 0;
-  const int n_it = n0 < p.Sk ? p.group * n_mt : 0;
-
   uint32_t goff[LQ];
 #pragma unroll
   for (int j = 0; j < LQ; ++j) {
@@ -864,8 +962,8 @@ __global__ void __launch_bounds__(256, 1) bwd_dkv_f32_mfma_kernel(BwdParams p) {
   const uint32_t lds0 = lds_addr(smem);
   const int64_t bh0 = (int64_t)b * p.Hq + hkv * p.group;
   auto issue = [&](int it) {
-    const int gi = it / n_mt;
-    const int m = m_begin + (it - gi * n_mt) * BMQ;
+    const int gi = (it0 + it) / n_mt;
+    const int m = m_begin + (it0 + it - gi * n_mt) * BMQ;
     const int rows = min(BMQ, p.Sq - m);
     const int64_t r0 = (bh0 + gi) * p.Sq + m;
     const i32x4 qr = make_rsrc_words((const float*)p.q + r0 * p.D, rows * p.D * 4);
@@ -898,7 +996,7 @@ __global__ void __launch_bounds__(256, 1) bwd_dkv_f32_mfma_kernel(BwdParams p) {
     wait_vmcnt<0>();  // step it's tiles landed for this wave ...
     __syncthreads();  // ... and for all; every read of step it-1 retired
     if (it + 1 < n_it) issue(it + 1);
-    const int m = m_begin + (it % n_mt) * BMQ;
+    const int m = m_begin + ((it0 + it) % n_mt) * BMQ;
     // Skip a tile none of this wave's keys can see (or keys past S_k).
     if (nw >= p.Sk || (CAUSAL && m + BMQ - 1 + diag < nw)) continue;
     const uint8_t* qt = smem + (it & 1) * QT;
@@ -942,15 +1040,20 @@ __global__ void __launch_bounds__(256, 1) bwd_dkv_f32_mfma_kernel(BwdParams p) {
     }
   }
   if (!key_ok) return;
+  // A chunk's partial sums (dK unscaled), or the gradients.
+  const int64_t at = n_chunks > 1 ? (int64_t)chunk * p.B * p.Hkv * p.Sk * p.D + krow : krow;
+  float* dko = (n_chunks > 1 ? p.part_dk : (float*)p.dk) + at;
+  float* dvo = (n_chunks > 1 ? p.part_dv : (float*)p.dv) + at;
+  const float ks = n_chunks > 1 ? 1.f : p.scale;
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int d = DB * (8 * (r >> 2) + 4 * hl + (r & 3));
     if (d < p.D) {
       vrow_t x, y;
 #pragma unroll
-      for (int c = 0; c < DB; ++c) x[c] = dk[c][r] * p.scale, y[c] = dv[c][r];
-      *reinterpret_cast<vrow_t*>((float*)p.dk + krow + d) = x;
-      *reinterpret_cast<vrow_t*>((float*)p.dv + krow + d) = y;
+      for (int c = 0; c < DB; ++c) x[c] = dk[c][r] * ks, y[c] = dv[c][r];
+      *reinterpret_cast<vrow_t*>(dko + d) = x;
+      *reinterpret_cast<vrow_t*>(dvo + d) = y;
     }
   }
 }
@@ -962,7 +1065,7 @@ static KernelPlan plan_bwd_f32_mfma(BwdParams& p, bool causal, bool dq) {
     p.n_mblocks = (p.Sq + 127) / 128;
     k.fn = causal ? (const void*)bwd_dq_f32_mfma_kernel<DP, true>
                   : (const void*)bwd_dq_f32_mfma_kernel<DP, false>;
-    k.grid = dim3((unsigned)((int64_t)p.n_mblocks * p.B * p.Hq));
+    k.grid = dim3((unsigned)((int64_t)p.n_mblocks * p.B * p.Hq * (p.dq_iters > 0 ? p.dq_chunks : 1)));
     k.kernel = "bwd_dq_f32_mfma_kernel";
     k.block_m = 128;
     k.block_n = kF32MmaTile;
@@ -970,7 +1073,7 @@ static KernelPlan plan_bwd_f32_mfma(BwdParams& p, bool causal, bool dq) {
     p.n_nblocks = (p.Sk + 127) / 128;
     k.fn = causal ? (const void*)bwd_dkv_f32_mfma_kernel<DP, true>
                   : (const void*)bwd_dkv_f32_mfma_kernel<DP, false>;
-    k.grid = dim3((unsigned)((int64_t)p.n_nblocks * p.B * p.Hkv));
+    k.grid = dim3((unsigned)((int64_t)p.n_nblocks * p.B * p.Hkv * (p.kv_iters > 0 ? p.kv_chunks : 1)));
     k.kernel = "bwd_dkv_f32_mfma_kernel";
     k.block_m = kF32MmaTile;
     k.block_n = 128;
@@ -981,6 +1084,80 @@ static KernelPlan plan_bwd_f32_mfma(BwdParams& p, bool causal, bool dq) {
   k.stages = 2;
   k.causal = causal;
   return k;
+}
+
+// Sums of the fp32 backward's partials in chunk order: blockIdx.y 0 dQ (scaled),
+// 1 dK (scaled), 2 dV.  One thread per four head-dim values of a row; rows of
+// blocks of one chunk are left as the gradient kernels wrote them.
+__global__ void __launch_bounds__(256) bwd_f32_reduce_kernel(BwdParams p, bool causal) {
+  const int which = blockIdx.y;
+  const int quads = p.D / 4;
+  const int len = which == 0 ? p.Sq : p.Sk;
+  const int64_t rows = (int64_t)p.B * (which == 0 ? p.Hq : p.Hkv) * len;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t row = i / quads;
+  if (row >= rows) return;
+  const int blk = (int)(row % len) >> 7;
+  const int iters = which == 0 ? p.dq_iters : p.kv_iters;
+  if (iters <= 0) return;
+  const int chunks = which == 0
+                         ? dkv_chunks(dq_tiles(blk, p.Sq, p.Sk, causal), iters)
+                         : dkv_chunks(p.group * dkv_tiles(blk, p.Sq, p.Sk, causal), iters);
+  if (chunks <= 1) return;
+  const int64_t at = row * p.D + (i - row * quads) * 4;
+  const float* src = (which == 0 ? p.part_dq : which == 1 ? p.part_dk : p.part_dv) + at;
+  f32x4 x = *reinterpret_cast<const f32x4*>(src);
+#pragma unroll 4
+  for (int c = 1; c < chunks; ++c) x += *reinterpret_cast<const f32x4*>(src + c * rows * p.D);
+  if (which != 2) x *= p.scale;
+  *reinterpret_cast<f32x4*>((float*)(which == 0 ? p.dq : which == 1 ? p.dk : p.dv) + at) = x;
+}
+
+// Chunk lengths of the matrix-core backward's two kernels (steps of 32 queries
+// against 128 keys, and of 32 keys against 128 queries) where their 4-wave
+// workgroups leave CUs idle, by the 16-bit kernel's model with these kernels'
+// step times.
+// Backward, before and now: 2 x 8 heads, S = 1,024, D = 64 294 and 176 us; 32
+// query heads on one KV head, S = 700, D = 64 3,659 and 204; 4 x 8 heads, S =
+// 1,024, D = 128 causal 525 and 440.
+void bwd_f32_split(int B, int Hq, int Hkv, int Sq, int Sk, int D, bool causal, BwdParams* p) {
+  p->kv_iters = p->dq_iters = 0;
+  p->kv_chunks = p->dq_chunks = 1;
+  const int dp = padded_head_dim(D);
+  if (!SK_F32_MFMA || dp <= 0 || dp > 128 || B <= 0 || Hkv <= 0 || Hq <= 0 || Sq <= 0 || Sk <= 0)
+    return;
+  const double step_us = dp <= 64 ? 4.0 : 8.0;
+  const double chunk_us = 128.0 * D * 4 * 2 / 5e6;  // per gradient
+  struct Memo {  // the last shape's answer
+    int key[7], it[4];
+  };
+  static thread_local Memo memo = {};
+  const int key[7] = {B, Hq, Hkv, Sq, Sk, D, (int)causal};
+  if (!std::equal(key, key + 7, memo.key)) {
+    int steps[64];
+    const int group = Hq / Hkv;
+    const int64_t nb = ((int64_t)Sk + 127) / 128, nm = ((int64_t)Sq + 127) / 128;
+    for (int k = 0; k < 4; ++k) memo.it[k] = k & 1;
+    if (nb * B * Hkv < 1024) {
+      const int n = (int)std::min<int64_t>(nb, 64);
+      for (int i = 0; i < n; ++i) steps[i] = group * dkv_tiles((int)(i * nb / n), Sq, Sk, causal);
+      memo.it[0] = best_chunk(steps, n, (double)B * Hkv * nb / n, causal, step_us * 1.3,
+                              0.5, 2 * chunk_us);
+      if (memo.it[0] > 0) memo.it[1] = dkv_chunks(steps[0], memo.it[0]);
+    }
+    if (nm * B * Hq < 1024) {
+      const int n = (int)std::min<int64_t>(nm, 64);
+      for (int i = 0; i < n; ++i) {
+        const int64_t mb = i == n - 1 ? nm - 1 : i * nm / n;  // (the last is the longest)
+        steps[i] = dq_tiles((int)mb, Sq, Sk, causal);
+      }
+      memo.it[2] = best_chunk(steps, n, (double)B * Hq * nm / n, causal, step_us, 0.5, chunk_us);
+      if (memo.it[2] > 0) memo.it[3] = dkv_chunks(steps[n - 1], memo.it[2]);
+    }
+    std::copy(key, key + 7, memo.key);
+  }
+  p->kv_iters = memo.it[0], p->kv_chunks = memo.it[1];
+  p->dq_iters = memo.it[2], p->dq_chunks = memo.it[3];
 }
 
 template <int DP>
@@ -1031,7 +1208,12 @@ hipError_t launch_bwd_f32(const BwdParams& p, bool causal, hipStream_t s) {
   if (!dq.fn || !kv.fn) return hipErrorInvalidValue;
   hipError_t e = run_plan(dq, &q, s);
   if (e != hipSuccess) return e;
-  return run_plan(kv, &q, s);
+  if ((e = run_plan(kv, &q, s)) != hipSuccess) return e;
+  if (q.dq_iters <= 0 && q.kv_iters <= 0) return hipSuccess;
+  const int64_t rows = std::max((int64_t)q.B * q.Hq * q.Sq, (int64_t)q.B * q.Hkv * q.Sk);
+  const dim3 grid((unsigned)((rows * (q.D / 4) + 255) / 256), 3);
+  hipLaunchKernelGGL(bwd_f32_reduce_kernel, grid, dim3(256), 0, s, q, causal);
+  return hipGetLastError();
 }
 
 }  // namespace sk

@@ -799,6 +799,7 @@ int fwd_split_keys(int sk, int splits) {
 }
 
 int fwd_key_splits(int dtype, int d, int64_t bh, int sq, int sk, bool causal) {
+  if (dtype == 0) return fwd_f32_key_splits(d, bh, sq, sk);
   if (dtype != BF16::code && dtype != F16::code) return 1;
   if (sq <= 0 || sk <= 0 || bh <= 0) return 1;
   if (d <= 128 && (d <= 64 ? kFwdD64Short : kFwdD128Short).nw != 4) return 1;  // tile study

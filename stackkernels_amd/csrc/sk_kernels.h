@@ -157,6 +157,10 @@ struct BwdParams {
   int kv_iters, kv_chunks;
   float* part_dk;
   float* part_dv;
+  // fp32 matrix-core backward: dQ split the same way over its key tiles
+  // (steps of 32 keys against 128 queries), partials [dq_chunks][B*Hq*Sq][D].
+  int dq_iters, dq_chunks;
+  float* part_dq;
 };
 
 // Steps of key block kb (128 keys) per query head: the 32-query tiles from
@@ -168,6 +172,12 @@ __host__ __device__ inline int dkv_first_query(int kb, int Sq, int Sk, bool caus
 __host__ __device__ inline int dkv_tiles(int kb, int Sq, int Sk, bool causal) {
   const int m = dkv_first_query(kb, Sq, Sk, causal);
   return m < Sq ? (Sq - m + 31) / 32 : 0;
+}
+// 32-key tiles that the fp32 dQ kernel's query block mb (128 rows) walks.
+__host__ __device__ inline int dq_tiles(int mb, int Sq, int Sk, bool causal) {
+  int end = Sk;
+  if (causal && 128 * mb + 128 + Sk - Sq < end) end = 128 * mb + 128 + Sk - Sq;
+  return end > 0 ? (end + 31) / 32 : 0;
 }
 __host__ __device__ inline int dkv_chunks(int steps, int iters) {
   return steps > iters ? (steps + iters - 1) / iters : 1;
@@ -287,10 +297,15 @@ KernelPlan plan_bwd_dq(int dtype, BwdParams& p, bool causal);
 // (its query heads' tiles), or 0 where the seven-GEMM backward runs (head
 // dims other than 65-128, fp32).
 size_t bwd_ds_pair_bytes(int dtype, int Hq, int Hkv, int Sq, int Sk, int D, bool causal);
+// Chunk length for a grid of blocks of uneven steps (sk_bwd.hip), or 0.
+int best_chunk(const int* steps, int n, double stands_for, bool causal, double step_us,
+               double fixed, double chunk_us);
 // Split of the dK/dV kernel the table takes for the shape: kv_iters and
 // kv_chunks of BwdParams (0 and 1: unsplit).
 void bwd_dkv_split(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D, bool causal,
                    int* iters, int* chunks);
+// The same for the fp32 backward: kv_iters / kv_chunks / dq_iters / dq_chunks of p.
+void bwd_f32_split(int B, int Hq, int Hkv, int Sq, int Sk, int D, bool causal, BwdParams* p);
 KernelPlan plan_bwd_dkv_f32(BwdParams& p, bool causal);
 KernelPlan plan_bwd_dq_f32(BwdParams& p, bool causal);
 
@@ -315,9 +330,10 @@ int fwd_pair_min(int dtype, int d, int64_t bh, int sq, int sk, bool causal);
 // Key splits the forward's table takes for that shape (1: unsplit), and the
 // keys each covers.
 int fwd_key_splits(int dtype, int d, int64_t bh, int sq, int sk, bool causal);
+int fwd_f32_key_splits(int d, int64_t bh, int sq, int sk);
 int fwd_split_keys(int sk, int splits);
-// Query blocks per (batch, head) of a split forward (its kernels are the
-// 4-wave entries, 128 rows a workgroup, at every head dim).
+// Query blocks per (batch, head) of a split 16-bit forward (its kernels are
+// the 4-wave entries, 128 rows a workgroup, at every head dim).
 int fwd_split_blocks(int sq);
 // Padded head dim the kernels are compiled for (64, 96, 128 or 256), or 0.
 int padded_head_dim(int d);

@@ -57,7 +57,7 @@ def _bwd(do, q, k, v, o, lse, causal, ws_bytes):
     (1, 8, 2, 300, 130, 96, True),     # S_q > S_k
     (2, 8, 1, 257, 129, 80, False),    # ragged, one key in the second block
     (1, 16, 1, 200, 1500, 64, True),
-    (13, 40, 10, 1000, 200, 64, False),  # 260 key blocks, two rounds
+    (13, 40, 10, 2000, 200, 64, False),  # 260 key blocks, two rounds
     (1, 8, 1, 190, 260, 256, True),    # head-dim halves
 ])
 def test_split_matches_oracle(device, dtype, b, hq, hkv, sq, sk, d, causal):
