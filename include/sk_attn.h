@@ -209,8 +209,9 @@ SK_API int sk_decode_plan_varlen(int dtype, int B, int Hq, int Hkv, int Sk, int 
  *   q (B,Hq,1,D), k/v (B,Hkv,Sk,D) with any b/h/s strides  ->  o (B,Hq,1,D).
  *
  * num_splits: as returned by sk_decode_plan, or any value in [1, Sk] (0 lets
- * the library plan).  workspace: >= the plan's bytes for that split count
- * (sk_decode_workspace), any contents.
+ * the library plan; fp32: one split).  workspace: >= the plan's bytes for that
+ * split count (sk_decode_workspace), any contents.  fp32 runs unsplit where the
+ * workspace holds one split's bytes only, and for groups above 64 heads.
  */
 SK_API int sk_decode(int dtype, const void* q, const void* k, const void* v, void* o,
               void* workspace, size_t workspace_bytes, int num_splits,
@@ -228,7 +229,7 @@ SK_API int sk_decode(int dtype, const void* q, const void* k, const void* v, voi
  * allocates nothing.  num_splits 0 takes the gfx950 table's split count,
  * lowered until the partials fit; an explicit split count whose partials do
  * not fit (B * Hq * num_splits * (padded D + 1) * 4 bytes) is rejected with
- * SK_EWORKSPACE.  fp32 runs unsplit with its B * Hq LSE values in the scratch.
+ * SK_EWORKSPACE (fp32 then runs unsplit; it also does with num_splits 0).
  * Every call on one GPU shares that GPU's scratch, which keeps the last call's
  * contents: calls that overlap on one GPU (concurrent streams, threads) race
  * and must be ordered by the caller.  Results equal sk_decode's for the same

@@ -122,10 +122,17 @@ int keys_per_split_for(int Sk, int splits) {
   return std::max(kps, 32);
 }
 
+// Head-dim columns of a split's partials: the kernel's padded head dim (the
+// fp32 kernel is compiled for 64, 128 and 256).
+size_t decode_dpad(int dtype, int D) {
+  const int dp = sk::padded_head_dim(D);
+  return (size_t)(dtype == SK_F32 && dp == 96 ? 128 : dp);
+}
+
 size_t decode_ws_bytes(int dtype, int B, int Hq, int D, int splits) {
-  if (dtype == SK_F32) return (size_t)B * Hq * sizeof(float);  // LSE of the fp32 forward
-  if (splits <= 1) return 0;
-  const size_t dpad = (size_t)sk::padded_head_dim(D);
+  // (One fp32 split: the LSE of the fp32 forward that serves groups above 64.)
+  if (splits <= 1) return dtype == SK_F32 ? (size_t)B * Hq * sizeof(float) : 0;
+  const size_t dpad = decode_dpad(dtype, D);
   return (size_t)B * Hq * splits * (dpad + 1) * sizeof(float);
 }
 
@@ -258,10 +265,10 @@ static int fwd_splits(int dtype, int B, int Hq, int Sq, int Sk, int D, bool caus
 }
 
 // Split count and keys per split of a decode call (num_splits 0: the gfx950
-// table's pick).  fp32 decode runs unsplit.
+// table's pick; for fp32 one split, and always one for fp32 groups above 64).
 static int decode_splits(int dtype, int B, int Hq, int Hkv, int Sk, int D, bool per_row, int num_splits,
                          int* splits, int* kps) {
-  if (dtype == SK_F32) num_splits = 1;
+  if (dtype == SK_F32 && (num_splits == 0 || Hq / Hkv > 64)) num_splits = 1;
   if (num_splits == 0) num_splits = plan_splits(B, Hq, Hkv, Sk, D, per_row);
   if (num_splits < 1 || num_splits > 1024)
     return fail(SK_EINVAL, "num_splits=%d outside [1, 1024]", num_splits);
@@ -509,7 +516,7 @@ static int decode_plan_impl(int dtype, int B, int Hq, int Hkv, int Sk, int D, bo
   int rc = check_dims(dtype, B, Hq, Hkv, 1, Sk, D);
   if (rc) return rc;
   if (!num_splits || !workspace_bytes) return fail(SK_EINVAL, "output pointer is NULL");
-  int splits = dtype == SK_F32 ? 1 : plan_splits(B, Hq, Hkv, Sk, D, per_row);
+  int splits = dtype == SK_F32 && Hq / Hkv > 64 ? 1 : plan_splits(B, Hq, Hkv, Sk, D, per_row);
   if (splits > 1) splits = (Sk + keys_per_split_for(Sk, splits) - 1) / keys_per_split_for(Sk, splits);
   *num_splits = splits;
   *workspace_bytes = decode_ws_bytes(dtype, B, Hq, D, splits);
@@ -589,14 +596,20 @@ static int decode_impl(int dtype, const void* q, const void* k, const void* v, v
   if ((rc = decode_splits(dtype, B, Hq, Hkv, Sk, D, seqlens != nullptr, num_splits, &num_splits,
                           &kps)))
     return rc;
-  const size_t need = decode_ws_bytes(dtype, B, Hq, D, num_splits);
+  size_t need = decode_ws_bytes(dtype, B, Hq, D, num_splits);
+  if (dtype == SK_F32 && num_splits > 1 && workspace_bytes < need) {
+    // (fp32 ran unsplit whatever the count: a caller's scratch of that size still serves.)
+    num_splits = 1;
+    kps = keys_per_split_for(Sk, 1);
+    need = decode_ws_bytes(dtype, B, Hq, D, 1);
+  }
   if (need > 0 && (!workspace || workspace_bytes < need))
     return fail(SK_EWORKSPACE, "workspace of %zu bytes given, %zu needed", workspace_bytes, need);
   if (need > 0 && (rc = check_ptr("workspace", workspace))) return rc;
   hipStream_t s = (hipStream_t)stream;
 
-  if (dtype == SK_F32) {
-    // fp32 decode is the fp32 forward with one query row (reference:
+  if (dtype == SK_F32 && Hq / Hkv > 64) {
+    // The fp32 forward with one query row (reference:
     // src/stackkernels/torch/attention.py:154 computes it the same way).
     sk::FwdParams p{};
     p.q = q, p.k = k, p.v = v, p.o = o, p.lse = (float*)workspace;
@@ -627,7 +640,7 @@ static int decode_impl(int dtype, const void* q, const void* k, const void* v, v
   p.B = B, p.Hq = Hq, p.Hkv = Hkv, p.Sk = Sk, p.D = D, p.group = Hq / Hkv;
   p.num_splits = num_splits;
   p.keys_per_split = kps;
-  p.dpad = sk::padded_head_dim(D);
+  p.dpad = (int)decode_dpad(dtype, D);
   p.scale = std::fabs(sm_scale);
   p.scale_log2 = p.scale * 1.4426950408889634f;
   p.q_sign = sm_scale < 0.f ? 0x80008000u : 0u;
@@ -725,7 +738,8 @@ int sk_decode_noalloc(int dtype, const void* q, const void* k, const void* v, vo
   }
   int splits = 0, kps = 0;
   if ((rc = decode_splits(dtype, B, Hq, Hkv, Sk, D, false, num_splits, &splits, &kps))) return rc;
-  const size_t need = decode_ws_bytes(dtype, B, Hq, D, splits);
+  size_t need = decode_ws_bytes(dtype, B, Hq, D, splits);
+  if (dtype == SK_F32 && need > kBytes) splits = 1, need = decode_ws_bytes(dtype, B, Hq, D, 1);
   if (need > kBytes)
     return fail(SK_EWORKSPACE,
                 "sk_decode_noalloc: %d split(s) need %zu bytes of scratch, more than the "
@@ -1013,8 +1027,8 @@ int sk_kernel_config(int op, int dtype, int B, int Hq, int Hkv, int Sq, int Sk, 
   sk::KernelPlan k;
   int64_t splits = 1, kps = 0, paired = 0, chunks = 1;
   size_t ws = 0;
-  if (op == SK_OP_FWD || (decode && dtype == SK_F32)) {
-    if (op == SK_OP_DECODE_COMBINE) {  // fp32 decode has no combine pass
+  if (op == SK_OP_FWD || (decode && dtype == SK_F32 && Hq / Hkv > 64)) {
+    if (op == SK_OP_DECODE_COMBINE) {  // (unsplit: no combine pass)
       cfg[SK_CFG_SPLITS] = 1;
       return SK_OK;
     }
@@ -1055,7 +1069,7 @@ int sk_kernel_config(int op, int dtype, int B, int Hq, int Hkv, int Sq, int Sk, 
     if ((rc = decode_splits(dtype, B, Hq, Hkv, Sk, D, per_row, num_splits, &ns, &per))) return rc;
     sk::DecParams p{};
     p.B = B, p.Hq = Hq, p.Hkv = Hkv, p.Sk = Sk, p.D = D, p.group = Hq / Hkv;
-    p.num_splits = ns, p.keys_per_split = per, p.dpad = sk::padded_head_dim(D);
+    p.num_splits = ns, p.keys_per_split = per, p.dpad = (int)decode_dpad(dtype, D);
     if (rope) p.rope.cos = &kStandIn;
     if (paged) p.block_table = &kStandIn;
     splits = ns, kps = per;

@@ -19,6 +19,8 @@
 //   combine kernel merges them with weights exp(LSE_s - max LSE), which is
 //   the reference's (acc, l, m) merge (decode.py:166-186) rewritten on
 //   normalised partials.  With one split the kernel writes O directly.
+#include <type_traits>
+
 #include "sk_common.h"
 #include "sk_kernels.h"
 #include "sk_rope.h"
@@ -351,12 +353,226 @@ __global__ void __launch_bounds__(NWH * 64) decode_split_kernel(DecParams p) {
   }
 }
 
+// fp32 split decode on the matrix cores (v_mfma_f32_16x16x4_f32: fp32 products,
+// fp32 accumulation), organised as decode_split_kernel: one workgroup per
+// (batch, KV head, key split) serves the group's query heads, 16 per wave, so
+// the cache is read once; tiles of 32 keys (16 at D = 256) staged in registers
+// one tile ahead, through one padded LDS buffer.
+// * S^T = K Q^T: k-step s contracts head-dim column DP/4 g + s in lane group g
+//   = lane / 16, on both operands, so one 16-byte LDS read gives a lane four
+//   k-steps of its key's row; the row padding of 4 floats puts the 16 rows of
+//   a lane group in distinct bank quads.
+// * O^T += V^T P^T: register r of a lane group is key 4 g + r, which is the B
+//   operand of k-step r as it stands; output block c holds columns DB m + c (m
+//   its row, DB = DP / 16), so a lane reads DB consecutive floats of a V row
+//   for all blocks and writes its outputs in whole pieces.
+// Bound by the cache's HBM traffic for large batches: the MFMAs of a tile take
+// about a third of its share of the bandwidth.  It replaced, for groups of up
+// to 64 heads, the fp32 forward at one query row, which used one of its 64
+// rows, read the cache once per query head and had no splits.  H_q = 32, H_kv =
+// 8, D = 128, both kernels: 32 rows of U[1, 4,096] keys, paged 3,613 -> 105 us;
+// 8 rows, H_q = 16, H_kv = 4, S_k = 5,000, D = 256 7,358 -> 93 us.
+template <int DP>
+constexpr int dec_f32_bn() {
+  return DP <= 128 ? 32 : 16;
+}
+
+template <int DP, int NWH, bool PAGED>
+__global__ void __launch_bounds__(NWH * 64) decode_split_f32_kernel(DecParams p) {
+  constexpr int BN = dec_f32_bn<DP>();
+  constexpr int NKB = BN / 16;
+  constexpr int NT = NWH * 64;
+  constexpr int STR = DP + 4;       // floats per LDS row
+  constexpr int CPR = DP / 4;       // 16-byte chunks per row
+  constexpr int LOADS = BN * CPR / NT;
+  constexpr int KS = DP / 4;        // k-steps of S^T
+  constexpr int DB = DP / 16;       // output blocks
+  static_assert(BN * CPR % NT == 0, "whole rounds of loads");
+
+  __shared__ __attribute__((aligned(16))) float ks[BN * STR];
+  __shared__ __attribute__((aligned(16))) float vs[BN * STR];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  const int c16 = lane & 15;
+  const int g = lane >> 4;
+
+  const int split = blockIdx.x;
+  const int bk = blockIdx.y;
+  const int b = p.longest_first ? row_of_rank(p, bk / p.Hkv) : bk / p.Hkv;
+  const int hkv = bk % p.Hkv;
+  const int sk_b =
+      p.seqlens ? min(max(__builtin_amdgcn_readfirstlane(p.seqlens[b]), 0), p.Sk) : p.Sk;
+  const int kps = p.seqlens ? max(32, ((sk_b + p.num_splits - 1) / p.num_splits + 31) / 32 * 32)
+                            : p.keys_per_split;
+  const int k_lo = split * kps;
+  const int k_hi = min(sk_b, k_lo + kps);
+  const int n_tiles = k_hi > k_lo ? (k_hi - k_lo + BN - 1) / BN : 0;
+
+  const int hd = 16 * wave + c16;
+  const bool head_ok = hd < p.group;
+  const int hq = hkv * p.group + (head_ok ? hd : 0);
+
+  const float* kbase = (const float*)p.k + b * p.k_sb + hkv * p.k_sh;
+  const float* vbase = (const float*)p.v + b * p.v_sb + hkv * p.v_sh;
+
+  f32x4 kreg[LOADS], vreg[LOADS];
+  bool ok_cur = true, ok_nxt = true;  // the tile's page lies in the pool (paged)
+  auto load_tile = [&](int t) {
+    const int n0 = k_lo + t * BN;
+    const float* kr = kbase + (int64_t)n0 * p.k_ss;
+    const float* vr = vbase + (int64_t)n0 * p.v_ss;
+    bool ok = true;
+    if constexpr (PAGED) {
+      const int page = p.block_table[(int64_t)b * p.max_pages + n0 / p.page_size];
+      ok = page >= 0 && page < p.num_pages;
+      const int64_t pg = ok ? page : 0, off = n0 % p.page_size;
+      kr = (const float*)p.k + pg * p.k_sb + (int64_t)hkv * p.k_sh + off * p.k_ss;
+      vr = (const float*)p.v + pg * p.v_sb + (int64_t)hkv * p.v_sh + off * p.v_ss;
+    }
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int c = tid + i * NT;
+      const int r = c / CPR;
+      const int d = (c % CPR) * 4;
+      f32x4 kx = {0.f, 0.f, 0.f, 0.f}, vx = {0.f, 0.f, 0.f, 0.f};
+      if (ok && n0 + r < k_hi && d < p.D) {
+        kx = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(kr + (int64_t)r * p.k_ss + d));
+        vx = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(vr + (int64_t)r * p.v_ss + d));
+      }
+      kreg[i] = kx;
+      vreg[i] = vx;
+    }
+    return ok;
+  };
+  auto store_tile = [&]() {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int c = tid + i * NT;
+      const int at = c / CPR * STR + (c % CPR) * 4;
+      *reinterpret_cast<f32x4*>(ks + at) = kreg[i];
+      *reinterpret_cast<f32x4*>(vs + at) = vreg[i];
+    }
+  };
+
+  if (n_tiles > 0) ok_cur = load_tile(0);
+  // Q^T operand: lane holds q[hq][KS g + s], rotated when the call carries
+  // RoPE tables, negated for a negative scale (zero past D and past the group).
+  float qv[KS];
+  {
+    const float* qp = (const float*)p.q + b * p.q_sb + hq * p.q_sh;
+    const int row = rope_row(p.rope, b, 0);
+    const int half = p.D >> 1;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int d = KS * g + s;
+      float x = 0.f;
+      if (head_ok && d < p.D) x = row >= 0 ? rope1(qp, d, half, p.rope, row) : qp[d];
+      qv[s] = p.q_sign ? -x : x;
+    }
+  }
+
+  f32x4 oacc[DB];
+#pragma unroll
+  for (int c = 0; c < DB; ++c) oacc[c] = f32x4{};
+  float m_run = kNegInf, l_run = 0.f;
+  const float* kq = ks + c16 * STR + KS * g;
+  const float* vq = vs + 4 * g * STR + DB * c16;
+
+  for (int t = 0; t < n_tiles; ++t) {
+    store_tile();
+    __syncthreads();
+    if (t + 1 < n_tiles) ok_nxt = load_tile(t + 1);
+    const int n0 = k_lo + t * BN;
+    f32x4 sc[NKB];
+#pragma unroll
+    for (int kb = 0; kb < NKB; ++kb) sc[kb] = f32x4{};
+#pragma unroll
+    for (int j = 0; j < KS / 4; ++j)
+#pragma unroll
+      for (int kb = 0; kb < NKB; ++kb) {
+        const f32x4 a = *reinterpret_cast<const f32x4*>(kq + 16 * kb * STR + 4 * j);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          sc[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], qv[4 * j + e], sc[kb], 0, 0, 0);
+      }
+    if (!ok_cur || n0 + BN > k_hi) {
+#pragma unroll
+      for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (!ok_cur || n0 + 16 * kb + 4 * g + r >= k_hi) sc[kb][r] = kNegInf;
+    }
+    ok_cur = ok_nxt;
+    float mt = kNegInf;
+#pragma unroll
+    for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mt = fmaxf(mt, sc[kb][r]);
+    mt = fmaxf(mt, __shfl_xor(mt, 16));
+    mt = xhalf_max(mt);
+    const float m_new = fmaxf(m_run, mt);
+    const float m_sub = m_new == kNegInf ? 0.f : m_new;
+    const float alpha = fast_exp2((m_run - m_sub) * p.scale_log2);
+    const float neg_m = -m_sub * p.scale_log2;
+    m_run = m_new;
+    float ps = 0.f;
+#pragma unroll
+    for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        sc[kb][r] = fast_exp2(fmaf(sc[kb][r], p.scale_log2, neg_m));
+        ps += sc[kb][r];
+      }
+    l_run = l_run * alpha + ps;
+#pragma unroll
+    for (int c = 0; c < DB; ++c) oacc[c] *= alpha;
+#pragma unroll
+    for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float* vr = vq + (16 * kb + r) * STR;
+#pragma unroll
+        for (int j = 0; j < DB / 4; ++j) {
+          const f32x4 x = *reinterpret_cast<const f32x4*>(vr + 4 * j);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            oacc[4 * j + e] =
+                __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], sc[kb][r], oacc[4 * j + e], 0, 0, 0);
+        }
+      }
+    __syncthreads();
+  }
+
+  float l_tot = l_run + __shfl_xor(l_run, 16);
+  l_tot = xhalf_sum(l_tot);
+  if (!head_ok) return;
+  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+  const int64_t row = ((int64_t)b * p.Hq + hq) * p.num_splits + split;
+  float* op = p.num_splits == 1 ? (float*)p.o + b * p.o_sb + hq * p.o_sh : p.part_o + row * p.dpad;
+  const int dlim = p.num_splits == 1 ? p.D : DP;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < DB / 4; ++j) {
+      const int d = DB * (4 * g + i) + 4 * j;
+      if (d < dlim)
+        *reinterpret_cast<f32x4*>(op + d) = f32x4{oacc[4 * j][i] * inv, oacc[4 * j + 1][i] * inv,
+                                                  oacc[4 * j + 2][i] * inv, oacc[4 * j + 3][i] * inv};
+    }
+  if (p.num_splits > 1 && g == 0)
+    p.part_lse[row] = l_tot > 0.f ? m_run * p.scale + logf(l_tot) : kNegInf;
+}
+
 // Merge split partials: one 256-thread workgroup per (batch, query head).
 // Split weights exp(LSE_s - max) go to LDS; then 8 groups of 32 lanes each
 // sum a strided subset of the splits with 16-byte loads (4 head-dim values
 // per lane) and the 8 partial sums are added through LDS.
 template <class T>
 __global__ void __launch_bounds__(256) decode_combine_kernel(DecParams p) {
+  constexpr bool kF32 = __is_same(T, float);
+  using E = typename std::conditional<kF32, float, uint16_t>::type;
   __shared__ float w[1024];
   __shared__ float red[8][2];
   __shared__ __attribute__((aligned(16))) float part[8][256];
@@ -393,7 +609,7 @@ __global__ void __launch_bounds__(256) decode_combine_kernel(DecParams p) {
   mx = fmaxf(fmaxf(red[0][0], red[1][0]), fmaxf(red[2][0], red[3][0]));
   float den = 0.f;
   for (int s = tid; s < ns; s += 256) {
-    const float x = mx == kNegInf ? 0.f : __expf(lse[s] - mx);
+    const float x = mx == kNegInf ? 0.f : kF32 ? expf(lse[s] - mx) : __expf(lse[s] - mx);
     w[s] = x;
     den += x;
   }
@@ -404,7 +620,7 @@ __global__ void __launch_bounds__(256) decode_combine_kernel(DecParams p) {
   den = (red[0][1] + red[1][1]) + (red[2][1] + red[3][1]);
   const float inv = den > 0.f ? 1.f / den : 0.f;
 
-  uint16_t* op = (uint16_t*)p.o + b * p.o_sb + hq * p.o_sh;
+  E* op = (E*)p.o + b * p.o_sb + hq * p.o_sh;
   for (int d0 = 0; d0 < p.D; d0 += 128) {
     const int d = d0 + d4;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -429,7 +645,10 @@ __global__ void __launch_bounds__(256) decode_combine_kernel(DecParams p) {
           a0 += part[k][dd];
           a1 += part[k][dd + 1];
         }
-        *reinterpret_cast<uint32_t*>(op + d0 + dd) = pack2<T>(a0 * inv, a1 * inv);
+        if constexpr (kF32)
+          *reinterpret_cast<f32x2*>(op + d0 + dd) = f32x2{a0 * inv, a1 * inv};
+        else
+          *reinterpret_cast<uint32_t*>(op + d0 + dd) = pack2<T>(a0 * inv, a1 * inv);
       }
     }
     __syncthreads();
@@ -493,7 +712,41 @@ static KernelPlan plan_decode_t(const DecParams& p) {
   return p.block_table ? plan_decode_tp<T, true>(p) : plan_decode_tp<T, false>(p);
 }
 
+// fp32, groups of up to 64 heads (none beyond: the fp32 forward at one query
+// row serves those).
+template <int DP, bool PAGED>
+static KernelPlan plan_decode_f32_dp(const DecParams& p) {
+  KernelPlan k;
+  const int nwh = p.group <= 16 ? 1 : p.group <= 32 ? 2 : 4;
+  k.fn = nwh == 1   ? (const void*)decode_split_f32_kernel<DP, 1, PAGED>
+         : nwh == 2 ? (const void*)decode_split_f32_kernel<DP, 2, PAGED>
+                    : (const void*)decode_split_f32_kernel<DP, 4, PAGED>;
+  k.grid = dim3((unsigned)p.num_splits, (unsigned)(p.B * p.Hkv));
+  k.block = dim3(64 * nwh);
+  k.kernel = "decode_split_f32_kernel";
+  k.elem = 0;
+  k.head_dim = DP;
+  k.block_m = 16 * nwh;
+  k.block_n = dec_f32_bn<DP>();
+  k.paged = PAGED;
+  k.rope = p.rope.cos != nullptr;
+  return k;
+}
+
+static KernelPlan plan_decode_f32(const DecParams& p) {
+  const bool pg = p.block_table != nullptr;
+  if (p.group > 64) return KernelPlan{};
+  switch (padded_head_dim(p.D)) {
+    case 64: return pg ? plan_decode_f32_dp<64, true>(p) : plan_decode_f32_dp<64, false>(p);
+    case 96:
+    case 128: return pg ? plan_decode_f32_dp<128, true>(p) : plan_decode_f32_dp<128, false>(p);
+    case 256: return pg ? plan_decode_f32_dp<256, true>(p) : plan_decode_f32_dp<256, false>(p);
+    default: return KernelPlan{};
+  }
+}
+
 KernelPlan plan_decode_mfma(int dtype, const DecParams& p) {
+  if (dtype == 0) return plan_decode_f32(p);
   if (dtype == BF16::code) return plan_decode_t<BF16>(p);
   if (dtype == F16::code) return plan_decode_t<F16>(p);
   return KernelPlan{};
@@ -511,6 +764,8 @@ KernelPlan plan_decode_combine(int dtype, const DecParams& p) {
     k.fn = (const void*)decode_combine_kernel<BF16>;
   else if (dtype == F16::code)
     k.fn = (const void*)decode_combine_kernel<F16>;
+  else if (dtype == 0)
+    k.fn = (const void*)decode_combine_kernel<float>;
   else
     return k;
   k.grid = dim3((unsigned)(p.B * p.Hq));
