@@ -91,8 +91,9 @@ int check_ptr(const char* name, const void* p) {
 // 64 x 64 heads, S_k = 500 16 us whole, 23 at 6.  Caches below 192 keys stay
 // whole.
 // Per-row lengths take their second round only where half of S_k gives each
-// split 512 keys (B = 32, U[1, 4,096]: 54.6 us with 16 splits, 53.1 with 8; B
-// = 64, U[1, 2,048]: 60.1 with 8, 56.5 with 4).  The count is capped at 1024
+// split 256 keys (B = 32, U[1, 4,096]: 54.6 us with 16 splits, 53.1 with 8; B
+// = 64, U[1, 2,048]: 60.1 with 8, 56.5 with 4; 9 rows of 32 KV heads, U[1,
+// 8,664]: 118 with 15, 123 with 8).  The count is capped at 1024
 // (the combine kernel's LDS weight array).
 int plan_splits(int B, int Hq, int Hkv, int Sk, int D, bool per_row) {
   (void)D;
@@ -104,7 +105,7 @@ int plan_splits(int B, int Hq, int Hkv, int Sk, int D, bool per_row) {
   int64_t splits = (slots + units - 1) / units;
   if (group <= 16 && per_row) {
     const int64_t two = (2 * slots + units - 1) / units;
-    if (Sk >= two * 1024) splits = two;
+    if (Sk >= two * 512) splits = two;
   }
   int64_t most = Sk / (group <= 16 && units >= 64 ? 128 : 256);
   if ((int64_t)B * Hq <= 1024) {
