@@ -251,18 +251,9 @@ static int fwd_shape(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D, i
 }
 
 // Bytes of the split forward's partials (per split and query row, D fp32
-// values and an LSE), 0 for one split.
-static size_t fwd_ws_bytes(int B, int Hq, int Sq, int D, int splits) {
-  if (splits <= 1) return 0;
-  return (size_t)splits * B * Hq * Sq * (D + 1) * sizeof(float);
-}
-
-// Splits a forward call runs with: the table's where the workspace holds
-// their partials, else one.
-static int fwd_splits(int dtype, int B, int Hq, int Sq, int Sk, int D, bool causal,
-                      size_t workspace_bytes) {
-  const int ns = sk::fwd_key_splits(dtype, D, (int64_t)B * Hq, Sq, Sk, causal);
-  return fwd_ws_bytes(B, Hq, Sq, D, ns) <= workspace_bytes ? ns : 1;
+// values and an LSE), 0 where it runs without.
+static size_t fwd_ws_bytes(int B, int Hq, int Sq, int D, const sk::FwdSplit& f) {
+  return f.on() ? (size_t)f.splits * B * Hq * Sq * (D + 1) * sizeof(float) : 0;
 }
 
 // Split count and keys per split of a decode call (num_splits 0: the gfx950
@@ -312,28 +303,33 @@ static int fwd_impl(int dtype, const void* q, const void* k, const void* v, void
   const bool neg = sm_scale < 0.f;
   if ((rc = fwd_shape(dtype, B, Hq, Hkv, Sq, Sk, D, is_causal, &p))) return rc;
   p.rope = rope;
-  int splits = num_splits;
-  if (splits == 0) {
-    splits = fwd_splits(dtype, B, Hq, Sq, Sk, D, is_causal != 0, workspace_bytes);
-  } else if (splits > 1) {
-    if (dtype == SK_F32 && sk::fwd_f32_rows_per_block(D, Sq) < 256) splits = 1;  // vector kernel
-    const int keys = splits > 1 ? sk::fwd_split_keys(Sk, splits) : 0;
-    splits = keys > 0 ? (Sk + keys - 1) / keys : 1;
-    const size_t need = fwd_ws_bytes(B, Hq, Sq, D, splits);
+  sk::FwdSplit f;
+  if (num_splits == 0) {
+    f = sk::fwd_key_splits(dtype, D, B, Hq, Hkv, Sq, Sk, is_causal != 0);
+    // (Packed heads' rows are addressed from the first one's in 31 bits.)
+    if (((int64_t)(f.pack - 1) * q_strides[1] + (int64_t)Sq * q_strides[2] + D) * 2 >= 0x7fffffffLL)
+      f.pack = 1;
+    if (fwd_ws_bytes(B, Hq, Sq, D, f) > workspace_bytes) f = sk::FwdSplit{};
+  } else if (num_splits > 1 && (dtype != SK_F32 || sk::fwd_f32_rows_per_block(D, Sq) == 256)) {
+    const int keys = sk::fwd_split_keys(Sk, num_splits);  // (else the fp32 vector kernel: unsplit)
+    f.splits = keys > 0 ? (Sk + keys - 1) / keys : 1;
+    const size_t need = fwd_ws_bytes(B, Hq, Sq, D, f);
     if (need > workspace_bytes)
       return fail(SK_EWORKSPACE, "workspace of %zu bytes given, %zu needed", workspace_bytes, need);
   }
-  if (splits > 1) {
+  p.pack_heads = 1;
+  if (f.on()) {
     // One query block per workgroup and split (pairing evens out the causal
     // triangle on full grids only).
     p.pair_items = 0;
-    if (dtype != SK_F32) p.n_mblocks = sk::fwd_split_blocks(Sq);
+    p.pack_heads = f.pack;
+    if (dtype != SK_F32) p.n_mblocks = sk::fwd_split_blocks((int64_t)f.pack * Sq);
     p.n_items = p.n_mblocks;
-    p.n_splits = splits;
-    p.split_keys = sk::fwd_split_keys(Sk, splits);
+    p.n_splits = f.splits;
+    p.split_keys = sk::fwd_split_keys(Sk, f.splits);
     p.part_o = (float*)workspace;
-    p.part_lse = p.part_o + (size_t)splits * B * Hq * Sq * D;
-    if ((int64_t)p.n_items * B * Hq * splits > 0x7fffffffLL)
+    p.part_lse = p.part_o + (size_t)f.splits * B * Hq * Sq * D;
+    if ((int64_t)p.n_items * B * Hq * f.splits > 0x7fffffffLL)
       return fail(SK_EINVAL, "grid too large");
   }
   hipStream_t s = (hipStream_t)stream;
@@ -345,7 +341,7 @@ static int fwd_impl(int dtype, const void* q, const void* k, const void* v, void
     p.q_sign = neg ? 0x80008000u : 0u;
     e = sk::launch_fwd_mfma(dtype, p, is_causal != 0, s);
   }
-  if (e == hipSuccess && p.n_splits > 1) e = sk::launch_fwd_combine(dtype, p, s);
+  if (e == hipSuccess && p.part_o) e = sk::launch_fwd_combine(dtype, p, s);
   if (e != hipSuccess) return hip_fail(e, "sk_attn_fwd launch");
   return SK_OK;
 }
@@ -368,7 +364,7 @@ int sk_attn_fwd_workspace(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int
   if (rc) return rc;
   if (!bytes) return fail(SK_EINVAL, "bytes pointer is NULL");
   *bytes = fwd_ws_bytes(B, Hq, Sq, D,
-                        sk::fwd_key_splits(dtype, D, (int64_t)B * Hq, Sq, Sk, is_causal != 0));
+                        sk::fwd_key_splits(dtype, D, B, Hq, Hkv, Sq, Sk, is_causal != 0));
   return SK_OK;
 }
 
@@ -1044,9 +1040,10 @@ int sk_kernel_config(int op, int dtype, int B, int Hq, int Hkv, int Sq, int Sk, 
     if (decode) {
       ws = decode_ws_bytes(dtype, B, Hq, D, 1);
     } else {
-      splits = sk::fwd_key_splits(dtype, D, (int64_t)B * Hq, Sq, Sk, is_causal != 0);
-      if (splits > 1) kps = sk::fwd_split_keys(Sk, (int)splits);
-      ws = fwd_ws_bytes(B, Hq, Sq, D, (int)splits);
+      const sk::FwdSplit f = sk::fwd_key_splits(dtype, D, B, Hq, Hkv, Sq, Sk, is_causal != 0);
+      splits = f.splits;
+      if (f.on()) kps = sk::fwd_split_keys(Sk, f.splits);
+      ws = fwd_ws_bytes(B, Hq, Sq, D, f);
     }
   } else if (op == SK_OP_BWD_DKV || op == SK_OP_BWD_DQ) {
     sk::BwdParams p{};

@@ -651,7 +651,7 @@ int fwd_f32_rows_per_block(int d, int sq) { return fwd_f32_on_mfma(d, sq) ? kF32
 template <int DP>
 static KernelPlan plan_fwd_f32_mfma(const FwdParams& p, bool causal) {
   KernelPlan k;
-  const bool split = p.n_splits > 1;
+  const bool split = p.part_o != nullptr;
   k.fn = causal ? (split ? (const void*)fwd_f32_mfma_kernel<DP, true, true>
                          : (const void*)fwd_f32_mfma_kernel<DP, true, false>)
                 : (split ? (const void*)fwd_f32_mfma_kernel<DP, false, true>

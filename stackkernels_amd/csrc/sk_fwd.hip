@@ -150,8 +150,13 @@ __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
   int bh = iw / p.n_items;
   int item = iw - bh * p.n_items;
   if (CAUSAL && !SPLIT && p.heavy_first) heavy_first_order(blockIdx.x, p.B * p.Hq, bh, item);
-  const int b = bh / p.Hq;
-  const int hq = bh % p.Hq;
+  // Packed rows (split kernels): the unit is a (batch, KV head) and its rows
+  // are the group's heads one after the other, row r query r % Sq of head
+  // r / Sq; hq is the first head.  Else the rows are one head's queries.
+  const int pack = SPLIT ? p.pack_heads : 1;
+  const int n_rows = SPLIT ? pack * p.Sq : p.Sq;
+  const int b = SPLIT ? bh / (p.Hq / pack) : bh / p.Hq;
+  const int hq = SPLIT ? bh % (p.Hq / pack) * pack : bh % p.Hq;
   const int hkv = hq / p.group;
   // The split's keys: sk of them from n_lo, numbered from 0 below (so query i
   // sees key j of them iff j <= i + diag).
@@ -200,33 +205,54 @@ __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
   const int m0 = mblk * BM;
   const int mw = m0 + wave * 32;
   const int row = mw + l32;
+  // Packed: this lane's query, and the wave's first and last (0 and Sq - 1
+  // where it spans heads).
+  const bool packed = SPLIT && pack > 1;
+  const bool one_head = !packed || mw / p.Sq == (mw + 31) / p.Sq;
+  const int qi = packed ? row % p.Sq : row;
+  const int q_first = !packed ? mw : one_head ? mw % p.Sq : 0;
+  const int q_last = !packed ? mw + 31 : one_head ? (mw + 31) % p.Sq : p.Sq - 1;
   int n_end = sk;
   if (CAUSAL) n_end = min(sk, m0 + BM + diag);
+  if (CAUSAL && packed)
+    n_end = min(sk, (m0 / p.Sq == (m0 + BM - 1) / p.Sq ? (m0 + BM - 1) % p.Sq : p.Sq - 1) + 1 + diag);
   const int n_tiles = n_end > 0 ? (n_end + BN - 1) / BN : 0;
 
   // Q^T operand: lane holds q[row][16*s + 8*hl .. +7] (zero past S_q and D).
   u32x4 qreg[KD];
   {
     const int qrows = max(0, min(32, p.Sq - mw));
-    const buf_rsrc qr = make_rsrc((const uint16_t*)p.q + b * p.q_sb + hq * p.q_sh +
-                                      (int64_t)min(mw, p.Sq) * p.q_ss,
-                                  tile_bytes(qrows, p.q_ss, p.D));
+    const buf_rsrc qr = packed
+        // A resource over the unit's heads from the first one's row 0 (its
+        // bytes fit 31 bits, which the host checks).
+        ? make_rsrc((const uint16_t*)p.q + b * p.q_sb + hq * p.q_sh,
+                    (int)(((int64_t)(pack - 1) * p.q_sh + (int64_t)(p.Sq - 1) * p.q_ss + p.D) * 2))
+        : make_rsrc((const uint16_t*)p.q + b * p.q_sb + hq * p.q_sh +
+                        (int64_t)min(mw, p.Sq) * p.q_ss,
+                    tile_bytes(qrows, p.q_ss, p.D));
+    int q_row = 0;  // packed: element offset of the lane's row, or -1
+    if constexpr (SPLIT) {
+      q_row = l32 * (int)p.q_ss;
+      if (packed) q_row = row < n_rows ? (int)((row / p.Sq) * p.q_sh + qi * p.q_ss) : -1;
+    }
 #pragma unroll
     for (int s = 0; s < KD; ++s) {
       const int d0 = 16 * s + 8 * hl;
-      const uint32_t off = d0 < p.D ? (uint32_t)((l32 * p.q_ss + d0) * 2) : kBufferOob;
+      const bool ok = d0 < p.D && (!SPLIT || q_row >= 0);
+      const uint32_t off = ok ? (uint32_t)(((SPLIT ? q_row : l32 * p.q_ss) + d0) * 2) : kBufferOob;
       qreg[s] = buffer_load_b128(qr, off);
     }
     if constexpr (ROPE) {
       // RoPE on load: query row i is token i of its batch row.  Rows past
       // S_q read zeros and stay zero.
-      const int rrow = rope_row(p.rope, b, row);
+      const int rrow = rope_row(p.rope, b, SPLIT ? qi : row);
       const int half = p.D >> 1;
 #pragma unroll
       for (int s = 0; s < KD; ++s) {
         const int d0 = 16 * s + 8 * hl;
         const int dq = d0 < half ? d0 + half : d0 - half;
-        const uint32_t off = d0 < p.D ? (uint32_t)((l32 * p.q_ss + dq) * 2) : kBufferOob;
+        const bool ok = d0 < p.D && (!SPLIT || q_row >= 0);
+        const uint32_t off = ok ? (uint32_t)(((SPLIT ? q_row : l32 * p.q_ss) + dq) * 2) : kBufferOob;
         const u32x4 y = buffer_load_b128(qr, off);
         if (rrow >= 0 && d0 < p.D) qreg[s] = rope8_at<T>(qreg[s], y, d0, half, p.rope, rrow);
       }
@@ -267,11 +293,11 @@ __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
   float m_run = kNegInf;
   float l_run = 0.f;
 
-  const bool wave_has_rows = mw < p.Sq;
+  const bool wave_has_rows = mw < (SPLIT ? n_rows : p.Sq);
   // Tiles [0, vis_tiles) hold keys this wave can see.
   int vis_tiles = wave_has_rows ? n_tiles : 0;
   if (CAUSAL) {
-    const int last_key = mw + 31 + diag;  // last key the wave's last row sees
+    const int last_key = (SPLIT ? q_last : mw + 31) + diag;  // last key the wave's last row sees
     vis_tiles = last_key < 0 ? 0 : min(vis_tiles, last_key / BN + 1);
   }
   auto active = [&](int t) { return t < vis_tiles; };
@@ -306,10 +332,10 @@ __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
   auto mask_max = [&](int t, f32x16 (&sc)[KB]) {
     const int n0 = t * BN;
     const bool tail = n0 + BN > sk;
-    const bool straddle = CAUSAL && (n0 + BN - 1 > mw + diag);
+    const bool straddle = CAUSAL && (n0 + BN - 1 > (SPLIT ? q_first : mw) + diag);
     if (tail || straddle) {
       int lim = sk - 1;
-      if (CAUSAL) lim = min(lim, row + diag);
+      if (CAUSAL) lim = min(lim, (SPLIT ? qi : row) + diag);
       // Element offset o (32*kb + 8*(r/4) + r%4) is masked iff o > lim - n0 - 4*hl.
       // keep = all-ones iff visible; one bitfield insert per element selects
       // the score or -inf (no per-element condition registers).
@@ -471,7 +497,7 @@ __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
   f32x16 s0[KB], s1[KB];
   auto masked = [&](int t) {
     const int n0 = t * BN;
-    return n0 + BN > sk || (CAUSAL && (n0 + BN - 1 > mw + diag));
+    return n0 + BN > sk || (CAUSAL && (n0 + BN - 1 > (SPLIT ? q_first : mw) + diag));
   };
   auto barrier_issue = [&](int k, int u_k) {  // before body k; u_k = k % 4
     if constexpr (kSync == 2) {
@@ -576,10 +602,11 @@ __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
   if constexpr (SPLIT) {
     // A split's partial: a row that saw no key leaves its output unwritten
     // (the combine skips it); a NaN row keeps its NaN.
-    if (row < p.Sq) {
+    if (row < n_rows) {
       const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
       const int64_t rows = (int64_t)p.B * p.Hq * p.Sq;
-      const int64_t r = split * rows + (int64_t)bh * p.Sq + row;
+      // (Packed heads are neighbours, so their rows follow one another here too.)
+      const int64_t r = split * rows + ((int64_t)b * p.Hq + hq) * p.Sq + row;
       if (l_tot != 0.f) {
         float* po = p.part_o + r * p.D;
 #pragma unroll
@@ -791,36 +818,56 @@ int fwd_pair_min(int dtype, int d, int64_t bh, int sq, int sk, bool causal) {
 // A predicted gain under 15% is left alone (causal squares, whose blocks
 // differ: 1,000 x 1,000 at 8 heads 20 us either way), and from 384 query
 // blocks on (1.5 per CU) nothing is split.
-int fwd_split_blocks(int sq) { return (sq + 127) / 128; }
+// Where the group's heads share blocks of 128 rows to a gain (few queries per
+// head), a (batch, KV head)'s rows are packed, which also reads the keys once
+// per group: 8 rows of 35 queries, H_q = 64, H_kv = 8, 19,392 keys 532 us
+// unpacked, 249 packed; 40 x 12,000, H_q = 32, H_kv = 4, B = 4, D = 256 217 and
+// 106.
+int fwd_split_blocks(int64_t rows) { return (int)((rows + 127) / 128); }
 
 int fwd_split_keys(int sk, int splits) {
   const int per = (sk + splits - 1) / splits;
   return (per + 63) / 64 * 64;
 }
 
-int fwd_key_splits(int dtype, int d, int64_t bh, int sq, int sk, bool causal) {
-  if (dtype == 0) return fwd_f32_key_splits(d, bh, sq, sk);
-  if (dtype != BF16::code && dtype != F16::code) return 1;
-  if (sq <= 0 || sk <= 0 || bh <= 0) return 1;
-  if (d <= 128 && (d <= 64 ? kFwdD64Short : kFwdD128Short).nw != 4) return 1;  // tile study
-  const int64_t items = (int64_t)fwd_split_blocks(sq) * bh;
-  if (items >= 384) return 1;
+FwdSplit fwd_key_splits(int dtype, int d, int B, int Hq, int Hkv, int sq, int sk, bool causal) {
+  const int64_t bh = (int64_t)B * Hq;
+  FwdSplit out;
+  if (sq <= 0 || sk <= 0 || bh <= 0 || Hkv <= 0) return out;
+  if (dtype == 0) {
+    out.splits = fwd_f32_key_splits(d, bh, sq, sk);
+    return out;
+  }
+  if (dtype != BF16::code && dtype != F16::code) return out;
+  if (d <= 128 && (d <= 64 ? kFwdD64Short : kFwdD128Short).nw != 4) return out;  // tile study
+  const int group = Hq / Hkv;
+  const int64_t whole = (int64_t)fwd_split_blocks(sq) * bh;
+  const int64_t packed = (int64_t)fwd_split_blocks((int64_t)group * sq) * B * Hkv;
   const double tile_us = d <= 64 ? 0.5 : d <= 128 ? 1.0 : 1.15;
   const double tiles = (double)sk / (d <= 128 ? 64 : 32);
-  const double merge_us = (double)bh * sq * d * 8 / 1.2e7;  // per split
-  int best = 1;
-  double best_us = 0, one_us = 0;
-  for (int ns = 1; ns <= 32; ++ns) {
-    if (ns > 1 && sk < ns * 256) break;
-    const int64_t load = (items * ns + 255) / 256;
+  const double merge_us = (double)bh * sq * d * 8 / 1.2e7 + 0.5;  // per split
+  auto us = [&](int64_t blocks, int ns, bool merge) {
+    const int64_t load = (blocks * ns + 255) / 256;
     const double eff = load > 1 && d <= 128 ? 0.95 : 1.0;
-    const double us = load * eff * (tiles / ns + 2) * tile_us + (ns > 1 ? 8 + ns * merge_us : 0);
-    if (ns == 1) one_us = us;
-    if (ns == 1 || us < best_us) best = ns, best_us = us;
+    return load * eff * (tiles / ns + 2) * tile_us + (merge ? 8 + ns * merge_us : 0);
+  };
+  const double one_us = us(whole, 1, false);
+  int best = 1;
+  bool pack = false;
+  double best_us = one_us;
+  for (int form = 0; form < 2; ++form) {
+    const int64_t items = form ? packed : whole;
+    if (items >= 384 || (form && packed >= whole)) continue;
+    for (int ns = form ? 1 : 2; ns <= 32 && (ns == 1 || sk >= ns * 256); ++ns) {
+      const double x = us(items, ns, true);
+      if (x < best_us) best = ns, best_us = x, pack = form != 0;
+    }
   }
-  if (best_us > 0.85 * one_us) return 1;
+  if (best_us > 0.85 * one_us) return out;
   const int keys = fwd_split_keys(sk, best);
-  return (sk + keys - 1) / keys;
+  out.splits = (sk + keys - 1) / keys;
+  if (pack) out.pack = group;
+  return out;
 }
 
 template <class T, int DP, int BN, int NW, int OCC, int STAGES = 4, int DC = DP>
@@ -829,8 +876,8 @@ static KernelPlan plan_fwd_t(const FwdParams& p, bool causal) {
   const bool rope = p.rope.cos != nullptr;
   // (Key splits run the 4-wave entries only.)
   constexpr bool kSplits = NW == 4;
-  if (p.n_splits > 1 && !kSplits) return k;
-  if (kSplits && p.n_splits > 1)
+  if (p.part_o && !kSplits) return k;
+  if (kSplits && p.part_o)
     k.fn = causal ? (rope ? (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, true, true, kSplits>
                           : (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, true, false, kSplits>)
                   : (rope ? (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, false, true, kSplits>
@@ -841,7 +888,7 @@ static KernelPlan plan_fwd_t(const FwdParams& p, bool causal) {
   else
     k.fn = rope ? (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, false, true, false>
                 : (const void*)fwd_mfma_kernel<T, DP, DC, BN, NW, STAGES, OCC, false, false, false>;
-  k.grid = dim3((unsigned)(p.n_items * p.B * p.Hq * std::max(1, p.n_splits)));
+  k.grid = dim3((unsigned)(p.n_items * p.B * (p.Hq / std::max(1, p.pack_heads)) * std::max(1, p.n_splits)));
   k.block = dim3(NW * 64);
   k.kernel = "fwd_mfma_kernel";
   k.elem = T::code;
@@ -856,7 +903,7 @@ static KernelPlan plan_fwd_t(const FwdParams& p, bool causal) {
 
 template <class T>
 static KernelPlan plan_fwd_dt(const FwdParams& p, bool causal) {
-  const bool sh = p.n_splits > 1 || fwd_short(p.D, (int64_t)p.B * p.Hq, p.Sq, p.Sk, causal);
+  const bool sh = p.part_o || fwd_short(p.D, (int64_t)p.B * p.Hq, p.Sq, p.Sk, causal);
   switch (fwd_config(p.D, (int64_t)p.B * p.Hq, p.Sq, p.Sk, causal).dp) {
     case 64:
       if (sh)
@@ -894,7 +941,7 @@ hipError_t launch_fwd_mfma(int dtype, const FwdParams& params, bool causal, hipS
   // Unpaired causal grids only: paired blocks carry equal work, and head-major
   // order then keeps each head's K/V in one L2 (B * H = 128, S = 4,096 527 us,
   // 575 with the blocks outermost).
-  p.heavy_first = causal && !p.pair_items && p.n_splits <= 1;
+  p.heavy_first = causal && !p.pair_items && !p.part_o;
   const KernelPlan k = plan_fwd_mfma(dtype, p, causal);
   if (!k.fn) return hipErrorInvalidValue;
   return run_plan(k, &p, s);

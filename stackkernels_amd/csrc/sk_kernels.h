@@ -60,12 +60,11 @@ struct FwdParams {
   float scale;       // |sm_scale|
   float scale_log2;  // |sm_scale| * log2(e)
   uint32_t q_sign;   // 0, or the sign-bit mask that negates q when sm_scale < 0
-  // Key splits (MFMA kernels): split s of a work item covers keys
-  // [s * split_keys, (s + 1) * split_keys), split_keys a multiple of 64.  With
-  // one split (0 and 1 both mean that) the kernel writes O and LSE; with more
-  // it writes each split's normalised output and its LSE in fp32 for
-  // fwd_combine_kernel: part_o [n_splits][B*Hq*Sq][D] (rows of a split that
-  // sees no key are not written), part_lse [n_splits][B*Hq*Sq] (-inf there).
+  // Key splits (MFMA kernels; part_o set): split s of a work item covers keys
+  // [s * split_keys, (s + 1) * split_keys), split_keys a multiple of 64, and
+  // writes its normalised output and LSE in fp32 for fwd_combine_kernel:
+  // part_o [n_splits][B*Hq*Sq][D] (rows of a split that sees no key are not
+  // written), part_lse [n_splits][B*Hq*Sq] (-inf there).
   int n_splits, split_keys;
   float* part_o;
   float* part_lse;
@@ -77,6 +76,8 @@ struct FwdParams {
   int page_size, max_pages, num_pages;
   // Rotation of q on load; query row i of batch row b is token i.
   RopeParams rope;
+  // 16-bit split kernels: heads of a group whose rows share blocks, 1 or the group.
+  int pack_heads;
 };
 
 // Split-KV decode (Sq == 1).
@@ -327,14 +328,17 @@ int fwd_rows_per_block(int dtype, int d, int64_t bh, int sq, int sk, bool causal
 // Fewest paired workgroups for which a causal forward of that shape pairs
 // its query blocks.
 int fwd_pair_min(int dtype, int d, int64_t bh, int sq, int sk, bool causal);
-// Key splits the forward's table takes for that shape (1: unsplit), and the
-// keys each covers.
-int fwd_key_splits(int dtype, int d, int64_t bh, int sq, int sk, bool causal);
+// Key splits the forward's table takes for a shape (1 and pack 1: one
+// workgroup per query block, no scratch) and the heads that share blocks of
+// rows; the keys a split covers; 128-row blocks of a 16-bit split kernel.
+struct FwdSplit {
+  int splits = 1, pack = 1;
+  bool on() const { return splits > 1 || pack > 1; }
+};
+FwdSplit fwd_key_splits(int dtype, int d, int B, int Hq, int Hkv, int sq, int sk, bool causal);
 int fwd_f32_key_splits(int d, int64_t bh, int sq, int sk);
 int fwd_split_keys(int sk, int splits);
-// Query blocks per (batch, head) of a split 16-bit forward (its kernels are
-// the 4-wave entries, 128 rows a workgroup, at every head dim).
-int fwd_split_blocks(int sq);
+int fwd_split_blocks(int64_t rows);
 // Padded head dim the kernels are compiled for (64, 96, 128 or 256), or 0.
 int padded_head_dim(int d);
 

@@ -104,3 +104,43 @@ def test_scratch_limits(device):
     assert lib.sk_attn_fwd(2, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
                            lse.data_ptr(), 1, 4, 1, 40, 5000, 128, *st, 1, 0.1, stream) == 0
     assert torch.equal(o, o1) and torch.equal(lse, l1)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("b,hq,hkv,sq,sk,d", [
+    (1, 8, 2, 17, 3000, 128),   # four heads in one block
+    (2, 8, 1, 33, 2500, 64),    # MQA, heads across waves and blocks
+    (1, 16, 4, 100, 2000, 80),  # blocks that end inside a head
+    (1, 8, 2, 1, 4000, 96),     # one query per head
+    (1, 6, 2, 50, 2100, 256),
+    (1, 8, 2, 60, 59, 128),     # S_q > S_k: the table leaves it alone
+])
+def test_packed_heads_match_oracle(device, dtype, causal, b, hq, hkv, sq, sk, d):
+    """Few queries per head: the table packs a group's heads into shared 128-row
+    blocks (q read from strided heads too) and splits the keys."""
+    need = ctypes.c_size_t()
+    assert _lib.load().sk_attn_fwd_workspace(_lib.dtype_code(dtype), b, hq, hkv, sq, sk, d,
+                                             int(causal), ctypes.byref(need)) == 0
+    assert (need.value > 0) == (sk > 100)
+    q, k, v = make_qkv(b, hq, hkv, sq, sk, d, dtype, seed=sq + sk)
+    ref, ref_lse = oracle_fwd(q, k, v, causal)
+    for form in (q, q.transpose(1, 2).contiguous().transpose(1, 2)):
+        o, lse = flash_attn_fwd(form, k, v, is_causal=causal)
+        torch.cuda.synchronize()
+        assert_close_maxabs(o, ref, TOL[dtype], "O")
+        assert_lse_close(lse, ref_lse)
+
+
+def test_packed_heads_rotate_by_their_own_query(device):
+    """RoPE on packed rows: query i of every head at start + i, as rotated beforehand."""
+    from stackkernels_amd._core.attention._rope import rope_args, rope_rotate
+    from stackkernels_amd._reference.torch.rope import precompute_freqs
+
+    q, k, v = make_qkv(2, 8, 2, 37, 3000, 128, torch.bfloat16, seed=5)
+    cos, sin = precompute_freqs(128, 4096, device=device)
+    pos = torch.tensor([2963, 100], dtype=torch.int32, device=device)
+    fused, lse = flash_attn_fwd(q, k, v, True, None, cos, sin, pos)
+    plain, lse2 = flash_attn_fwd(rope_rotate(q, rope_args(cos, sin, pos, 2, 128, q.device)), k, v,
+                                 True)
+    assert torch.equal(fused, plain) and torch.equal(lse, lse2)
