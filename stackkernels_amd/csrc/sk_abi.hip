@@ -73,13 +73,23 @@ int check_ptr(const char* name, const void* p) {
 //   faster than two rounds), about two rounds with per-row lengths and over
 //   paged pools (per_row), whose rows spread their keys over their splits so
 //   a row shorter than the longest leaves a one-round grid uneven (8
-//   splits: 6.9% and 7.7% faster than 4 at the C4 shape with lengths U[1, Sk]);
+//   splits: 6.9% and 7.7% faster than 4 at the C4 shape with lengths U[1, Sk]).
+//   A uniform round is not overfilled: counts round down (368 rows and heads,
+//   S_k = 4,000 132.9 us at 6 splits, 120.7 at 5; 1,200, S_k = 1,000 114.5 at
+//   2, 98.2 at 1); with per-row lengths the one round rounds up (720, S_k <=
+//   1,500 59.3 us at 3 splits, 64.1 at 2);
+// * head dims above 128, groups of up to 16: four workgroups fit on a CU, so
+//   a uniform round is 1,024 (180, S_k = 5,357 209 us at 6 splits, 157 at 5;
+//   above 1,024 units two splits, 219 -> 191 us at 1,200), and per-row lengths
+//   take two such rounds at any length (368, S_k <= 976 53.4 us at 2 splits,
+//   42.1 at 5, 47.3 at 6; 800, S_k <= 1,500 121 at 2, 130 at 3);
 // * 32- and 64-head groups: exactly one round, so no split waits for a second
 //   round; a 64-head group writes 32 KB of partials per split, so fewer,
 //   longer splits also keep that traffic small (C5: 64 splits; 32 and 128
 //   splits measured 15% and 10% slower).
-// A split keeps at least 256 keys, 128 from 64 (batch, KV head) units on with
-// groups of up to 16 heads.  Small calls (at most 1,024 query heads in all,
+// A split keeps at least 256 keys, 128 with 64 to 384 (batch, KV head) units
+// of up to 16 heads (360 units, S_k <= 500, D = 128: 28.0 us whole, 20.9 at 3
+// splits; 800 units, S_k <= 700: 45.0 at 2, 47.9 at 3).  Small calls (at most 1,024 query heads in all,
 // whose partials cost the combine little) split further, because a split's
 // tiles follow one another: to 64 keys while that gives at most 512
 // workgroups (128 with the 64-key tiles of groups above 32), to one 32-key
@@ -90,13 +100,13 @@ int check_ptr(const char* name, const void* p) {
 // those limits more splits lose: B = 1, S_k = 32,768 31 us at 128, 36 at 256;
 // 64 x 64 heads, S_k = 500 16 us whole, 23 at 6.  Caches below 192 keys stay
 // whole.
-// Per-row lengths take their second round only where half of S_k gives each
-// split 256 keys (B = 32, U[1, 4,096]: 54.6 us with 16 splits, 53.1 with 8; B
-// = 64, U[1, 2,048]: 60.1 with 8, 56.5 with 4; 9 rows of 32 KV heads, U[1,
-// 8,664]: 118 with 15, 123 with 8).  The count is capped at 1024
+// Up to D = 128 per-row lengths take their second round only where the longest
+// row gives each split 512 keys, 352 up to 384 units (B = 32, U[1, 4,096], 256 keys: 54.6 us with 16
+// splits, 53.1 with 8; 720 units, U[1, 1,500], 300 keys: 64.6 with 5, 59.3 with
+// 3; 368 units, U[1, 4,000], 363 keys: 57.4 with 11, 64.6 with 6; 800 units,
+// U[1, 3,000], 600 keys: 113.6 with 5, 118.8 with 3).  The count is capped at 1024
 // (the combine kernel's LDS weight array).
 int plan_splits(int B, int Hq, int Hkv, int Sk, int D, bool per_row) {
-  (void)D;
   if (Sk < 192 || B <= 0 || Hkv <= 0) return 1;
   const int group = Hq / Hkv;
   const int waves = group <= 16 ? 1 : group <= 32 ? 2 : 4;
@@ -104,10 +114,14 @@ int plan_splits(int B, int Hq, int Hkv, int Sk, int D, bool per_row) {
   const int64_t units = (int64_t)B * Hkv;
   int64_t splits = (slots + units - 1) / units;
   if (group <= 16 && per_row) {
-    const int64_t two = (2 * slots + units - 1) / units;
-    if (Sk >= two * 512) splits = two;
+    const int64_t two = 2 * slots / units;
+    if (D > 128) splits = slots / units;
+    else if (Sk >= two * (units <= 384 ? 352 : 512)) splits = std::max(splits, two);
+  } else if (group <= 16) {
+    if (D <= 128) splits = slots / units;
+    else if (units <= slots / 2) splits = slots / 2 / units;
   }
-  int64_t most = Sk / (group <= 16 && units >= 64 ? 128 : 256);
+  int64_t most = Sk / (group <= 16 && units >= 64 && units <= 384 ? 128 : 256);
   if ((int64_t)B * Hq <= 1024) {
     most = std::max<int64_t>(most, std::min<int64_t>(512 / units, Sk / (group > 32 ? 128 : 64)));
     if (group <= 32)
