@@ -264,6 +264,12 @@ static int fwd_shape(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D, i
   return SK_OK;
 }
 
+// |sm_scale| as the kernels multiply by it.  A zero scale (every visible key
+// weighs the same) runs as 1e-30, which vanishes next to 1 for any ordinary
+// score but keeps a masked score, or a running maximum before its first key,
+// at -inf, where 0 * -inf would be NaN.
+static float softmax_scale(float sm_scale) { return std::max(std::fabs(sm_scale), 1e-30f); }
+
 // Bytes of the split forward's partials (per split and query row, D fp32
 // values and an LSE), 0 where it runs without.
 static size_t fwd_ws_bytes(int B, int Hq, int Sq, int D, const sk::FwdSplit& f) {
@@ -312,7 +318,7 @@ static int fwd_impl(int dtype, const void* q, const void* k, const void* v, void
   p.k_sb = k_strides[0], p.k_sh = k_strides[1], p.k_ss = k_strides[2];
   p.v_sb = v_strides[0], p.v_sh = v_strides[1], p.v_ss = v_strides[2];
   p.o_sb = o_strides[0], p.o_sh = o_strides[1], p.o_ss = o_strides[2];
-  p.scale = std::fabs(sm_scale);
+  p.scale = softmax_scale(sm_scale);
   p.scale_log2 = p.scale * 1.4426950408889634f;
   const bool neg = sm_scale < 0.f;
   if ((rc = fwd_shape(dtype, B, Hq, Hkv, Sq, Sk, D, is_causal, &p))) return rc;
@@ -506,9 +512,7 @@ int sk_attn_bwd(int dtype, const void* dout, const void* q, const void* k, const
   p.B = B, p.Hq = Hq, p.Hkv = Hkv, p.Sq = Sq, p.Sk = Sk, p.D = D, p.group = Hq / Hkv;
   p.scale = sm_scale;
   p.scale_log2 = sm_scale * 1.4426950408889634f;
-  // |s| * 1e-30 * log2(e) rounds to 0 next to any finite score, so a zero
-  // scale still gives P = exp2(-lse * log2 e) exactly while -inf stays -inf.
-  p.abs_scale_log2 = std::max(std::fabs(sm_scale), 1e-30f) * 1.4426950408889634f;
+  p.abs_scale_log2 = softmax_scale(sm_scale) * 1.4426950408889634f;
   p.op_sign = sm_scale < 0.f ? 0x80008000u : 0u;
   hipStream_t s = (hipStream_t)stream;
   hipError_t e = hipSuccess;
@@ -629,7 +633,7 @@ static int decode_impl(int dtype, const void* q, const void* k, const void* v, v
     p.v_sb = v_strides[0], p.v_sh = v_strides[1], p.v_ss = v_strides[2];
     p.o_sb = o_strides[0], p.o_sh = o_strides[1], p.o_ss = o_strides[2];
     p.B = B, p.Hq = Hq, p.Hkv = Hkv, p.Sq = 1, p.Sk = Sk, p.D = D, p.group = Hq / Hkv;
-    p.scale = std::fabs(sm_scale);
+    p.scale = softmax_scale(sm_scale);
     p.scale_log2 = p.scale * 1.4426950408889634f;
     p.q_sign = sm_scale < 0.f ? 1u : 0u;
     p.n_mblocks = 1;
@@ -652,7 +656,7 @@ static int decode_impl(int dtype, const void* q, const void* k, const void* v, v
   p.num_splits = num_splits;
   p.keys_per_split = kps;
   p.dpad = (int)decode_dpad(dtype, D);
-  p.scale = std::fabs(sm_scale);
+  p.scale = softmax_scale(sm_scale);
   p.scale_log2 = p.scale * 1.4426950408889634f;
   p.q_sign = sm_scale < 0.f ? 0x80008000u : 0u;
   p.seqlens = seqlens;
