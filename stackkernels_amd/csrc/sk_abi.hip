@@ -80,7 +80,10 @@ int check_ptr(const char* name, const void* p) {
 //   1,500 59.3 us at 3 splits, 64.1 at 2);
 // * head dims above 128, groups of up to 16: four workgroups fit on a CU, so
 //   a uniform round is 1,024 (180, S_k = 5,357 209 us at 6 splits, 157 at 5;
-//   above 1,024 units two splits, 219 -> 191 us at 1,200), and per-row lengths
+//   above 1,024 units two splits, 219 -> 191 us at 1,200; one whole round
+//   against two and three, 64 units, S_k = 16,384: 174, 191 and 205 us with
+//   16-head groups, 168, 176 and 186 with 4; 16 units, S_k = 32,768: 94, 112
+//   and 120), and per-row lengths
 //   take two such rounds at any length (368, S_k <= 976 53.4 us at 2 splits,
 //   42.1 at 5, 47.3 at 6; 800, S_k <= 1,500 121 at 2, 130 at 3);
 // * 32- and 64-head groups: exactly one round, so no split waits for a second

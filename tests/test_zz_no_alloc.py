@@ -74,13 +74,19 @@ def test_noalloc_decode_matches_workspace_decode():
     q, k, v = _inputs(4, 64, 1, 3000, 64, torch.float16, 1)
     o1, o2, _ = _both(lib, q, k, v, 7)
     assert torch.equal(o1, o2), "call 2 (fp16 MQA, 7 splits)"
-    # 3: the table's count lowered to fit the scratch
-    q, k, v = _inputs(8, 128, 8, 16384, 256, torch.bfloat16, 2)
+    # 3: the table's count lowered to fit the scratch (64 heads at D = 256: one round of
+    # four-wave workgroups writes 33.7 MB of partials)
+    q, k, v = _inputs(8, 64, 1, 16384, 256, torch.bfloat16, 2)
     o1, o2, used = _both(lib, q, k, v, 0)
-    per_split = 8 * 128 * 257 * 4
-    table = _plan(lib, _lib.SK_BF16, 8, 128, 8, 16384, 256)
+    per_split = 8 * 64 * 257 * 4
+    table = _plan(lib, _lib.SK_BF16, 8, 64, 1, 16384, 256)
     assert table * per_split > SCRATCH and used == SCRATCH // per_split < table
     assert torch.equal(o1, o2), "call 3 (split count lowered to fit)"
+    # 3b: 16-head groups at D = 256, whose partials fit whole
+    q, k, v = _inputs(8, 128, 8, 16384, 256, torch.bfloat16, 2)
+    o1, o2, used = _both(lib, q, k, v, 0)
+    assert used == _plan(lib, _lib.SK_BF16, 8, 128, 8, 16384, 256) > 1
+    assert torch.equal(o1, o2), "call 3b (16-head groups, the table's count)"
     # 4: fp32 (unsplit; LSE in the scratch)
     q, k, v = _inputs(2, 8, 2, 500, 64, torch.float32, 3)
     o1, o2, _ = _both(lib, q, k, v, 0)
