@@ -80,6 +80,14 @@ SK_API int sk_attn_fwd(int dtype, const void* q, const void* k, const void* v, v
                 int is_causal, float sm_scale, void* stream);
 
 /*
+ * Most bytes of fp32 partials the tables ask for in one call (256 MiB): the
+ * key splits of a forward (sk_attn_fwd_workspace) or the chunks of a
+ * backward's gradients (sk_attn_bwd_workspace_best).  Counts that would need
+ * more are not taken.
+ */
+#define SK_PARTIALS_CAP_BYTES 268435456LL
+
+/*
  * Forward attention with optional key splits and rotation.
  *
  * sk_attn_fwd_ws is sk_attn_fwd (rope_cos and rope_sin NULL) or
@@ -131,10 +139,11 @@ SK_API int sk_attn_bwd_workspace(int dtype, int B, int Hq, int Hkv, int Sq, int 
 
 /*
  * Most bytes of scratch sk_attn_bwd makes use of with these dims: the above
- * plus, for 16-bit calls whose dK/dV workgroups leave part of the chip idle,
- * the fp32 partial sums of a dK/dV split over the query tiles.  A call given
- * at least this many bytes sums dK and dV in that split's order; one given
- * less sums them in one pass per key block.
+ * plus, for calls whose workgroups leave part of the chip idle, the fp32
+ * partial sums (at most SK_PARTIALS_CAP_BYTES) of a dK/dV split over the query
+ * tiles and, for fp32, of a dQ split over the key tiles.  A call given at
+ * least this many bytes sums those gradients in the split's order; one given
+ * less sums them in one pass per block.
  */
 SK_API int sk_attn_bwd_workspace_best(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D,
                                int is_causal, size_t* bytes);

@@ -1591,9 +1591,10 @@ static double dkv_step_us(int d) { return d <= 64 ? 0.45 : d <= 128 ? 0.85 : 1.5
 // the blocks differ (causal), the mean load plus half a chunk, or whole
 // rounds; each with `fixed` steps of prologue and epilogue per workgroup, plus
 // chunk_us of partial sums written and read per chunk and 4 us for the merge.
-// Unsplit, heavy blocks first: the heaviest block or the mean load.
+// Unsplit, heavy blocks first: the heaviest block or the mean load.  At most
+// `most` chunks a block: what the cap on partial sums holds.
 int best_chunk(const int* steps, int n, double stands_for, bool causal, double step_us,
-               double fixed, double chunk_us) {
+               double fixed, double chunk_us, int64_t most) {
   double total = 0;
   int longest = 0;
   for (int i = 0; i < n; ++i) total += steps[i], longest = std::max(longest, steps[i]);
@@ -1607,6 +1608,7 @@ int best_chunk(const int* steps, int n, double stands_for, bool causal, double s
   for (int cut : kCuts) {
     const int len = (longest + cut - 1) / cut;
     if (len * step_us < 3) break;  // a chunk's fixed cost would be most of it
+    if (dkv_chunks(longest, len) > most) break;
     double m = 0, split = 0;  // workgroups; those that write partials
     for (int i = 0; i < n; ++i) {
       const int c = dkv_chunks(steps[i], len);
@@ -1653,7 +1655,8 @@ void bwd_dkv_split(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D, boo
     for (int i = 0; i < n; ++i) steps[i] = group * dkv_tiles((int)(i * nb / n), Sq, Sk, causal);
     const double stands_for = (double)pairs * parts * nb / n;
     const int best = best_chunk(steps, n, stands_for, causal, dkv_step_us(D), 4,
-                                128.0 * D * 8 * 2 / 5e6 / parts);
+                                128.0 * D * 8 * 2 / 5e6 / parts,
+                                SK_PARTIALS_CAP_BYTES / (pairs * Sk * D * 8));
     memo.iters = best;
     memo.chunks = best > 0 ? dkv_chunks(steps[0], best) : 1;
     std::copy(key, key + 7, memo.key);

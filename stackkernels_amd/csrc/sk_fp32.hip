@@ -632,9 +632,10 @@ int fwd_f32_key_splits(int d, int64_t bh, int sq, int sk) {
   const double tile_us = d <= 64 ? 8.4 : 16.5;
   const double tiles = sk / 64.0;
   const double merge_us = (double)bh * sq * d * 8 / 1.2e7;
+  const int most = fwd_most_splits(bh * sq, d);
   int best = 1;
   double best_us = 0, one_us = 0;
-  for (int ns = 1; ns <= 32; ++ns) {
+  for (int ns = 1; ns <= most; ++ns) {
     if (ns > 1 && sk < ns * 64) break;
     const int64_t load = (items * ns + 255) / 256;
     const double us = load * (tiles / ns + 0.5) * tile_us + (ns > 1 ? 8 + ns * merge_us : 0);
@@ -1138,12 +1139,18 @@ void bwd_f32_split(int B, int Hq, int Hkv, int Sq, int Sk, int D, bool causal, B
     const int group = Hq / Hkv;
     const int64_t nb = ((int64_t)Sk + 127) / 128, nm = ((int64_t)Sq + 127) / 128;
     for (int k = 0; k < 4; ++k) memo.it[k] = k & 1;
+    // Room for partial sums: dK and dV first, dQ in what they leave.
+    int64_t left = SK_PARTIALS_CAP_BYTES;
+    const int64_t kv_bytes = (int64_t)B * Hkv * Sk * D * 8;
     if (nb * B * Hkv < 1024) {
       const int n = (int)std::min<int64_t>(nb, 64);
       for (int i = 0; i < n; ++i) steps[i] = group * dkv_tiles((int)(i * nb / n), Sq, Sk, causal);
       memo.it[0] = best_chunk(steps, n, (double)B * Hkv * nb / n, causal, step_us * 1.3,
-                              0.5, 2 * chunk_us);
-      if (memo.it[0] > 0) memo.it[1] = dkv_chunks(steps[0], memo.it[0]);
+                              0.5, 2 * chunk_us, left / kv_bytes);
+      if (memo.it[0] > 0) {
+        memo.it[1] = dkv_chunks(steps[0], memo.it[0]);
+        left -= memo.it[1] * kv_bytes;
+      }
     }
     if (nm * B * Hq < 1024) {
       const int n = (int)std::min<int64_t>(nm, 64);
@@ -1151,7 +1158,8 @@ void bwd_f32_split(int B, int Hq, int Hkv, int Sq, int Sk, int D, bool causal, B
         const int64_t mb = i == n - 1 ? nm - 1 : i * nm / n;  // (the last is the longest)
         steps[i] = dq_tiles((int)mb, Sq, Sk, causal);
       }
-      memo.it[2] = best_chunk(steps, n, (double)B * Hq * nm / n, causal, step_us, 0.5, chunk_us);
+      memo.it[2] = best_chunk(steps, n, (double)B * Hq * nm / n, causal, step_us, 0.5, chunk_us,
+                              left / ((int64_t)B * Hq * Sq * D * 4));
       if (memo.it[2] > 0) memo.it[3] = dkv_chunks(steps[n - 1], memo.it[2]);
     }
     std::copy(key, key + 7, memo.key);

@@ -825,6 +825,12 @@ int fwd_pair_min(int dtype, int d, int64_t bh, int sq, int sk, bool causal) {
 // 106.
 int fwd_split_blocks(int64_t rows) { return (int)((rows + 127) / 128); }
 
+// Splits of that many query rows whose partials stay within the cap, at most 32.
+int fwd_most_splits(int64_t rows, int d) {
+  const int64_t fit = (int64_t)SK_PARTIALS_CAP_BYTES / (rows * (d + 1) * 4);
+  return (int)std::max<int64_t>(1, std::min<int64_t>(32, fit));
+}
+
 int fwd_split_keys(int sk, int splits) {
   const int per = (sk + splits - 1) / splits;
   return (per + 63) / 64 * 64;
@@ -852,13 +858,14 @@ FwdSplit fwd_key_splits(int dtype, int d, int B, int Hq, int Hkv, int sq, int sk
     return load * eff * (tiles / ns + 2) * tile_us + (merge ? 8 + ns * merge_us : 0);
   };
   const double one_us = us(whole, 1, false);
+  const int most = fwd_most_splits(bh * sq, d);
   int best = 1;
   bool pack = false;
   double best_us = one_us;
   for (int form = 0; form < 2; ++form) {
     const int64_t items = form ? packed : whole;
     if (items >= 384 || (form && packed >= whole)) continue;
-    for (int ns = form ? 1 : 2; ns <= 32 && (ns == 1 || sk >= ns * 256); ++ns) {
+    for (int ns = form ? 1 : 2; ns <= most && (ns == 1 || sk >= ns * 256); ++ns) {
       const double x = us(items, ns, true);
       if (x < best_us) best = ns, best_us = x, pack = form != 0;
     }

@@ -6,6 +6,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "sk_attn.h"
+
 // Causal forward: blocks j and n_mblocks-1-j run in one workgroup when the
 // paired workgroups still fill SK_FWD_PAIR_ROUNDS rounds of the 256 CUs at
 // the table entry's workgroups per CU (a tile-study build can raise it to
@@ -300,7 +302,7 @@ KernelPlan plan_bwd_dq(int dtype, BwdParams& p, bool causal);
 size_t bwd_ds_pair_bytes(int dtype, int Hq, int Hkv, int Sq, int Sk, int D, bool causal);
 // Chunk length for a grid of blocks of uneven steps (sk_bwd.hip), or 0.
 int best_chunk(const int* steps, int n, double stands_for, bool causal, double step_us,
-               double fixed, double chunk_us);
+               double fixed, double chunk_us, int64_t most);
 // Split of the dK/dV kernel the table takes for the shape: kv_iters and
 // kv_chunks of BwdParams (0 and 1: unsplit).
 void bwd_dkv_split(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D, bool causal,
@@ -337,6 +339,7 @@ struct FwdSplit {
 };
 FwdSplit fwd_key_splits(int dtype, int d, int B, int Hq, int Hkv, int sq, int sk, bool causal);
 int fwd_f32_key_splits(int d, int64_t bh, int sq, int sk);
+int fwd_most_splits(int64_t rows, int d);
 int fwd_split_keys(int sk, int splits);
 int fwd_split_blocks(int64_t rows);
 // Padded head dim the kernels are compiled for (64, 96, 128 or 256), or 0.
