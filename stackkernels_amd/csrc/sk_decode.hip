@@ -361,7 +361,13 @@ __global__ void __launch_bounds__(NWH * 64) decode_split_kernel(DecParams p) {
 // * S^T = K Q^T: k-step s contracts head-dim column DP/4 g + s in lane group g
 //   = lane / 16, on both operands, so one 16-byte LDS read gives a lane four
 //   k-steps of its key's row; the row padding of 4 floats puts the 16 rows of
-//   a lane group in distinct bank quads.
+//   a lane group in distinct bank quads.  Four accumulators take the k-steps in
+//   turn and are added in pairs, so a score is four chains of D / 4 products:
+//   one chain of D made short caches less exact than the four partial sums of
+//   the vector kernel (D = 256, 17 keys: 2-norm error 3.5e-7, 1.8e-7 with four;
+//   17 keys, D = 128: 2.7e-7 and 1.5e-7), at up to 2.5% of the time (64-head
+//   MQA, 8 x 32,768 keys: 106.3 us before, 109.1 now; 1% or less at 16 heads
+//   and below).
 // * O^T += V^T P^T: register r of a lane group is key 4 g + r, which is the B
 //   operand of k-step r as it stands; output block c holds columns DB m + c (m
 //   its row, DB = DP / 16), so a lane reads DB consecutive floats of a V row
@@ -485,9 +491,11 @@ __global__ void __launch_bounds__(NWH * 64) decode_split_f32_kernel(DecParams p)
     __syncthreads();
     if (t + 1 < n_tiles) ok_nxt = load_tile(t + 1);
     const int n0 = k_lo + t * BN;
-    f32x4 sc[NKB];
+    f32x4 part[NKB][4], sc[NKB];
 #pragma unroll
-    for (int kb = 0; kb < NKB; ++kb) sc[kb] = f32x4{};
+    for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) part[kb][e] = f32x4{};
 #pragma unroll
     for (int j = 0; j < KS / 4; ++j)
 #pragma unroll
@@ -495,8 +503,12 @@ __global__ void __launch_bounds__(NWH * 64) decode_split_f32_kernel(DecParams p)
         const f32x4 a = *reinterpret_cast<const f32x4*>(kq + 16 * kb * STR + 4 * j);
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          sc[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], qv[4 * j + e], sc[kb], 0, 0, 0);
+          part[kb][e] =
+              __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], qv[4 * j + e], part[kb][e], 0, 0, 0);
       }
+#pragma unroll
+    for (int kb = 0; kb < NKB; ++kb)
+      sc[kb] = (part[kb][0] + part[kb][1]) + (part[kb][2] + part[kb][3]);
     if (!ok_cur || n0 + BN > k_hi) {
 #pragma unroll
       for (int kb = 0; kb < NKB; ++kb)

@@ -2,6 +2,7 @@
 groups and head dims, against the float64 oracle at the fp32 bound; groups
 above 64 heads stay on the fp32 forward's one-row path, unsplit."""
 
+import numpy as np
 import pytest
 import torch
 
@@ -54,6 +55,39 @@ def test_paged_lengths_and_rope(device, d, page):
                                  start_pos=pos.to(device))
         assert_close_maxabs(out, ref, TOL[F32], f"O (splits={ns})")
         assert torch.all(out[0] == 0)
+
+
+def _fp32_in_quarters(q, k, v):
+    """Attention of q (H, D) over k, v (H, S, D) in float32: scores as four partial
+    sums of D / 4 products each, one running sum over the keys."""
+    f = np.float32
+    h, s, d = k.shape
+    prod = (q[:, None] * k).reshape(h, s, 4, d // 4)
+    acc = np.zeros((h, s, 4), f)
+    for i in range(d // 4):
+        acc += prod[..., i]
+    sc = ((acc[..., 0] + acc[..., 1]) + (acc[..., 2] + acc[..., 3])) * f(1 / np.sqrt(d))
+    w = np.exp(sc - sc.max(-1, keepdims=True))
+    o, den = np.zeros((h, d), f), np.zeros((h, 1), f)
+    for j in range(s):
+        o += w[:, j:j + 1] * v[:, j]
+        den += w[:, j:j + 1]
+    return o / den
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("sk", [17, 64, 200])
+def test_short_caches_keep_fp32_precision(device, d, sk):
+    """No further from 64 bits than fp32 sums in four quarters of the head dim, on
+    the same inputs.  (1.15: both are the rounding of as many operations, and its
+    2-norm over 8,192 or more outputs varies by a few percent.  One chain over the
+    head dim is 1.4 to 1.9 times as far.)"""
+    q, k, v = make_qkv(4, 32, 32, 1, sk, d, F32, seed=d + sk)
+    exact = oracle_fwd(q, k, v, False)[0].reshape(-1, d)
+    want = _fp32_in_quarters(*(t.cpu().numpy().reshape(128, -1, d) if t.shape[2] > 1
+                               else t.cpu().numpy().reshape(128, d) for t in (q, k, v)))
+    got = np64(core_decode(q, k, v)).reshape(-1, d)
+    assert np.linalg.norm(got - exact) <= 1.15 * np.linalg.norm(want - exact)
 
 
 def test_strided_cache(device):
