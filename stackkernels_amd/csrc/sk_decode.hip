@@ -194,6 +194,13 @@ __global__ void __launch_bounds__(NWH * 64) decode_split_kernel(DecParams p) {
   const uint16_t* kbase = (const uint16_t*)p.k + b * p.k_sb + hkv * p.k_sh;
   const uint16_t* vbase = (const uint16_t*)p.v + b * p.v_sb + hkv * p.v_sh;
 
+  // Four waves read q before the first tile: their splits are long, and q behind
+  // it has nothing to hide (64 heads, both kernels: 8 x 131,072 keys 98.5 us so,
+  // 99.6 behind; D = 64, 8 x 32,768 25.7 and 26.0; D = 256, 4 x 8,192 29.8 and 30.2).
+  constexpr bool kQFirst = NWH == 4;
+  u32x4 qreg[KD];
+  if constexpr (kQFirst) load_q<T>(p, b, hq, head_ok, g, qreg);
+
   // Paged: the page of tile t + 2 is read (vector load) while tile t runs,
   // and used when tile t + 2's loads are issued, one iteration later.
   PageTable ptab{};
@@ -252,10 +259,9 @@ __global__ void __launch_bounds__(NWH * 64) decode_split_kernel(DecParams p) {
     if (n_tiles > 1) pg_nxt = page_of(1);
     load_tile(0, pg_cur);
   }
-  // q (and its rotation's table rows) behind the first tile's loads: the two
-  // latencies overlap.
-  u32x4 qreg[KD];
-  load_q<T>(p, b, hq, head_ok, g, qreg);
+  // q (and its rotation's table rows): in workgroups of one or two waves behind
+  // the first tile's loads, so the two latencies overlap.
+  if constexpr (!kQFirst) load_q<T>(p, b, hq, head_ok, g, qreg);
   for (int t = 0; t < n_tiles; ++t) {
     store_tile();
     __syncthreads();
