@@ -443,8 +443,11 @@ SK_API int sk_kv_cache_update_paged_rope(int dtype, const void* k, const void* v
  * this library instead of a Triton heuristic.
  *
  *   op       SK_OP_FWD, SK_OP_BWD_DKV, SK_OP_BWD_DQ, SK_OP_DECODE (the split
- *            pass; fp32: the fp32 forward kernel with one query row) or
- *            SK_OP_DECODE_COMBINE (grid 0 when one split writes O directly);
+ *            pass; fp32 groups above 64 heads: the fp32 forward kernel with
+ *            one query row), SK_OP_DECODE_COMBINE, SK_OP_FWD_COMBINE or
+ *            SK_OP_BWD_REDUCE (the merges; grid 0 where nothing is split).
+ *            Forward and backward as run with the scratch that
+ *            sk_attn_fwd_workspace and sk_attn_bwd_workspace_best report;
  *   Sq       ignored for decode; num_splits: decode only (0 = the table's pick);
  *   variant  SK_VARIANT_* bits: the decode over a paged pool, the RoPE
  *            prologue (forward and decode), per-row cache lengths (decode:
@@ -461,6 +464,8 @@ SK_API int sk_kv_cache_update_paged_rope(int dtype, const void* k, const void* v
 #define SK_OP_BWD_DQ 2
 #define SK_OP_DECODE 3
 #define SK_OP_DECODE_COMBINE 4
+#define SK_OP_FWD_COMBINE 5
+#define SK_OP_BWD_REDUCE 6
 
 #define SK_VARIANT_PAGED 1
 #define SK_VARIANT_ROPE 2
@@ -472,7 +477,8 @@ SK_API int sk_kv_cache_update_paged_rope(int dtype, const void* k, const void* v
 #define SK_CFG_BLOCK_N 3        /* keys per tile (dK/dV: keys per workgroup)    */
 #define SK_CFG_STAGES 4         /* tile ring depth; 0 = staged in registers     */
 #define SK_CFG_HEAD_DIM 5       /* padded head dim the kernel is compiled for   */
-#define SK_CFG_SPLITS 6         /* decode, forward: key splits (1 otherwise)    */
+#define SK_CFG_SPLITS 6         /* decode, forward: key splits; backward: chunks of the
+                                 * longest block's tiles, one workgroup each (1: unsplit) */
 #define SK_CFG_PAIRED 7         /* forward: causal query blocks paired per workgroup */
 #define SK_CFG_WORKSPACE 8      /* scratch bytes the call needs                 */
 #define SK_CFG_KEYS_PER_SPLIT 9 /* decode, split forward                        */
@@ -480,6 +486,8 @@ SK_API int sk_kv_cache_update_paged_rope(int dtype, const void* k, const void* v
 #define SK_CFG_VGPRS 11         /* device-reported registers per lane, or -1    */
 #define SK_CFG_WG_PER_CU 12     /* device-reported resident workgroups per CU, or -1 */
 #define SK_CFG_CHUNKS 13        /* backward: launches of the kernel per call (chunks of pairs) */
+#define SK_CFG_SIDE_STREAM 14   /* dQ: 1 where it runs beside dK/dV on the side stream */
+#define SK_CFG_PACKED_HEADS 15  /* forward: heads of a group that share blocks of rows (1) */
 #define SK_CFG_LEN 16
 
 SK_API int sk_kernel_config(int op, int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D,

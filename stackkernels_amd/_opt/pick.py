@@ -38,9 +38,11 @@ _DTYPE_CODES = {"float32": 0, "fp32": 0, "float": 0, "float16": 1, "fp16": 1, "h
 
 # sk_kernel_config ops and cfg slots (include/sk_attn.h).
 _OP_FWD, _OP_BWD_DKV, _OP_BWD_DQ, _OP_DECODE, _OP_DECODE_COMBINE = 0, 1, 2, 3, 4
+_OP_FWD_COMBINE, _OP_BWD_REDUCE = 5, 6
 _VARIANT_PAGED, _VARIANT_ROPE, _VARIANT_VARLEN = 1, 2, 4
 _SLOTS = ("grid", "threads", "block_m", "block_n", "stages", "head_dim", "splits", "paired",
-          "workspace_bytes", "keys_per_split", "lds_bytes", "vgprs", "wg_per_cu", "chunks")
+          "workspace_bytes", "keys_per_split", "lds_bytes", "vgprs", "wg_per_cu", "chunks",
+          "side_stream", "packed_heads")
 
 
 def _dtype_code(dtype: Any) -> int:
@@ -157,9 +159,16 @@ def pick(
         kernels.append(k)
         config = _public(k)
         config["paired_causal_blocks"] = bool(k["paired"])
-        # key splits of a small grid, each with a grid of its own; its scratch
+        # key splits of a small grid, each with a grid of its own (and heads of a group in
+        # shared blocks), the scratch of their partials and the pass that merges them
         config["SPLIT_KV"] = k["splits"]
+        config["packed_heads"] = k["packed_heads"]
         config["workspace_bytes"] = k["workspace_bytes"]
+        if k["workspace_bytes"]:
+            comb = kernel_config(_OP_FWD_COMBINE, code, prob, 0, 0, query)
+            kernels.append(comb)
+            config["keys_per_split"] = k["keys_per_split"]
+            config["combine"] = _public(comb)
     elif op_name in _BWD_OPS:
         dkv = kernel_config(_OP_BWD_DKV, code, prob, 0, 0, query)
         dq = kernel_config(_OP_BWD_DQ, code, prob, 0, 0, query)
@@ -167,6 +176,13 @@ def pick(
         config = _public(dkv)
         config["kernel_variant"] = f"{config['kernel_variant']}+{dq['kernel'].split('<')[0]}"
         config["dq"] = _public(dq)
+        # chunks of the longest block's tiles, one workgroup each, and their merge
+        config["splits"], config["dq"]["splits"] = dkv["splits"], dq["splits"]
+        config["dq"]["side_stream"] = bool(dq["side_stream"])
+        if max(dkv["splits"], dq["splits"]) > 1:
+            red = kernel_config(_OP_BWD_REDUCE, code, prob, 0, 0, query)
+            kernels.append(red)
+            config["reduce"] = _public(red)
         config["workspace_bytes"] = dkv["workspace_bytes"]
         # launches of each kernel per call: chunks of (batch, KV head) pairs
         # whose dS tiles fit the workspace (1 for the seven-GEMM backward)
@@ -212,16 +228,21 @@ def pick(
         "Kernels & Wave Math:",
     ]
     for k in kernels:
-        line = (f"  - {k['kernel']}: grid {k['grid']} workgroups x {k['threads']} threads"
+        grid = k["grid"] * (k["splits"] if op_name in _FWD_OPS and k is kernels[0] else 1)
+        line = (f"  - {k['kernel']}: grid {grid} workgroups x {k['threads']} threads"
                 f" ({k['threads'] // 64} wavefronts)")
         if k["wg_per_cu"] > 0:
-            rounds = k["grid"] / (table_prof.sm_count * k["wg_per_cu"])
+            rounds = grid / (table_prof.sm_count * k["wg_per_cu"])
             line += (f"; {k['wg_per_cu']} resident per CU (LDS {k['lds_bytes']} B, "
                      f"{k['vgprs']} registers per lane) -> {rounds:.2f} rounds over "
                      f"{table_prof.sm_count} CUs")
         else:
-            line += f"; {k['grid'] / table_prof.sm_count:.2f} workgroups per CU"
+            line += f"; {grid / table_prof.sm_count:.2f} workgroups per CU"
         lines.append(line)
+    if op_name in _FWD_OPS and config["workspace_bytes"]:
+        lines.append(f"  - split-KV: {config['SPLIT_KV']} splits of {config['keys_per_split']} keys, "
+                     f"{config['packed_heads']} head(s) per row block, "
+                     f"{config['workspace_bytes']} bytes of partials")
     if op_name in _DECODE_OPS:
         lines.append(f"  - split-KV: {config['SPLIT_KV']} splits of {config['keys_per_split']} keys, "
                      f"{config['workspace_bytes']} bytes of partials")

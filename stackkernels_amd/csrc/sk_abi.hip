@@ -279,6 +279,19 @@ static size_t fwd_ws_bytes(int B, int Hq, int Sq, int D, const sk::FwdSplit& f) 
   return f.on() ? (size_t)f.splits * B * Hq * Sq * (D + 1) * sizeof(float) : 0;
 }
 
+// Makes p the split forward f: one query block per workgroup and split
+// (pairing evens out the causal triangle on full grids only), partials at part.
+static void fwd_apply_split(int dtype, const sk::FwdSplit& f, void* part, sk::FwdParams* p) {
+  p->pair_items = 0;
+  p->pack_heads = f.pack;
+  if (dtype != SK_F32) p->n_mblocks = sk::fwd_split_blocks((int64_t)f.pack * p->Sq);
+  p->n_items = p->n_mblocks;
+  p->n_splits = f.splits;
+  p->split_keys = sk::fwd_split_keys(p->Sk, f.splits);
+  p->part_o = (float*)part;
+  p->part_lse = p->part_o + (size_t)f.splits * p->B * p->Hq * p->Sq * p->D;
+}
+
 // Split count and keys per split of a decode call (num_splits 0: the gfx950
 // table's pick; for fp32 one split, and always one for fp32 groups above 64).
 static int decode_splits(int dtype, int B, int Hq, int Hkv, int Sk, int D, bool per_row, int num_splits,
@@ -342,16 +355,7 @@ static int fwd_impl(int dtype, const void* q, const void* k, const void* v, void
   }
   p.pack_heads = 1;
   if (f.on()) {
-    // One query block per workgroup and split (pairing evens out the causal
-    // triangle on full grids only).
-    p.pair_items = 0;
-    p.pack_heads = f.pack;
-    if (dtype != SK_F32) p.n_mblocks = sk::fwd_split_blocks((int64_t)f.pack * Sq);
-    p.n_items = p.n_mblocks;
-    p.n_splits = f.splits;
-    p.split_keys = sk::fwd_split_keys(Sk, f.splits);
-    p.part_o = (float*)workspace;
-    p.part_lse = p.part_o + (size_t)f.splits * B * Hq * Sq * D;
+    fwd_apply_split(dtype, f, workspace, &p);
     if ((int64_t)p.n_items * B * Hq * f.splits > 0x7fffffffLL)
       return fail(SK_EINVAL, "grid too large");
   }
@@ -1043,9 +1047,9 @@ int sk_kernel_config(int op, int dtype, int B, int Hq, int Hkv, int Sq, int Sk, 
   const bool rope = (variant & SK_VARIANT_ROPE) != 0;
   const bool paged = (variant & SK_VARIANT_PAGED) != 0;
   sk::KernelPlan k;
-  int64_t splits = 1, kps = 0, paired = 0, chunks = 1;
+  int64_t splits = 1, kps = 0, paired = 0, chunks = 1, packed = 1, side = 0;
   size_t ws = 0;
-  if (op == SK_OP_FWD || (decode && dtype == SK_F32 && Hq / Hkv > 64)) {
+  if (op == SK_OP_FWD || op == SK_OP_FWD_COMBINE || (decode && dtype == SK_F32 && Hq / Hkv > 64)) {
     if (op == SK_OP_DECODE_COMBINE) {  // (unsplit: no combine pass)
       cfg[SK_CFG_SPLITS] = 1;
       return SK_OK;
@@ -1055,21 +1059,29 @@ int sk_kernel_config(int op, int dtype, int B, int Hq, int Hkv, int Sq, int Sk, 
       return rc;
     if (rope) p.rope.cos = &kStandIn;
     if (paged && decode) p.block_table = &kStandIn;
-    k = dtype == SK_F32 ? sk::plan_fwd_f32(p, !decode && is_causal)
-                        : sk::plan_fwd_mfma(dtype, p, is_causal != 0);
-    paired = p.pair_items;
     if (decode) {
       ws = decode_ws_bytes(dtype, B, Hq, D, 1);
     } else {
+      // The call with the scratch sk_attn_fwd_workspace reports.
       const sk::FwdSplit f = sk::fwd_key_splits(dtype, D, B, Hq, Hkv, Sq, Sk, is_causal != 0);
-      splits = f.splits;
-      if (f.on()) kps = sk::fwd_split_keys(Sk, f.splits);
       ws = fwd_ws_bytes(B, Hq, Sq, D, f);
+      splits = f.splits, packed = f.pack;
+      if (f.on()) {
+        fwd_apply_split(dtype, f, const_cast<int*>(&kStandIn), &p);
+        kps = p.split_keys;
+      } else if (op == SK_OP_FWD_COMBINE) {
+        cfg[SK_CFG_SPLITS] = 1;
+        return SK_OK;
+      }
     }
-  } else if (op == SK_OP_BWD_DKV || op == SK_OP_BWD_DQ) {
+    k = op == SK_OP_FWD_COMBINE ? sk::plan_fwd_combine(dtype, p)
+        : dtype == SK_F32       ? sk::plan_fwd_f32(p, !decode && is_causal)
+                                : sk::plan_fwd_mfma(dtype, p, is_causal != 0);
+    paired = p.pair_items;
+  } else if (op == SK_OP_BWD_DKV || op == SK_OP_BWD_DQ || op == SK_OP_BWD_REDUCE) {
     sk::BwdParams p{};
     p.B = B, p.Hq = Hq, p.Hkv = Hkv, p.Sq = Sq, p.Sk = Sk, p.D = D, p.group = Hq / Hkv;
-    // The plan of one chunk at the workspace size sk_attn_bwd_workspace reports.
+    // The plan of one chunk of pairs at the size sk_attn_bwd_workspace_best reports.
     const int64_t pairs = (int64_t)B * Hkv;
     const int64_t chunk = bwd_chunk_pairs(
         pairs, sk::bwd_ds_pair_bytes(dtype, Hq, Hkv, Sq, Sk, D, is_causal != 0),
@@ -1079,9 +1091,25 @@ int sk_kernel_config(int op, int dtype, int B, int Hq, int Hkv, int Sq, int Sk, 
       p.n_pairs = (int)chunk;
       chunks = (pairs + chunk - 1) / chunk;
     }
-    k = op == SK_OP_BWD_DKV ? sk::plan_bwd_dkv(dtype, p, is_causal != 0)
-                            : sk::plan_bwd_dq(dtype, p, is_causal != 0);
-    ws = bwd_ws_bytes(dtype, B, Hq, Hkv, Sq, Sk, D, is_causal != 0);
+    const BwdParts parts = bwd_parts(dtype, B, Hq, Hkv, Sq, Sk, D, is_causal != 0);
+    ws = parts.bytes > 0 ? parts.offset + parts.bytes
+                         : bwd_ws_bytes(dtype, B, Hq, Hkv, Sq, Sk, D, is_causal != 0);
+    if (parts.bytes > 0) {
+      p.kv_iters = parts.p.kv_iters, p.kv_chunks = parts.p.kv_chunks;
+      p.dq_iters = parts.p.dq_iters, p.dq_chunks = parts.p.dq_chunks;
+    }
+    if (op == SK_OP_BWD_REDUCE && parts.bytes == 0) {
+      cfg[SK_CFG_SPLITS] = 1;
+      return SK_OK;
+    }
+    if (op == SK_OP_BWD_DKV && p.kv_iters > 0) splits = p.kv_chunks;
+    if (op == SK_OP_BWD_DQ && p.dq_iters > 0) splits = p.dq_chunks;
+    if (op == SK_OP_BWD_REDUCE)
+      splits = std::max(p.kv_iters > 0 ? p.kv_chunks : 1, p.dq_iters > 0 ? p.dq_chunks : 1);
+    if (op == SK_OP_BWD_DQ) side = sk::bwd_forks(dtype, p, is_causal != 0);
+    k = op == SK_OP_BWD_DKV  ? sk::plan_bwd_dkv(dtype, p, is_causal != 0)
+        : op == SK_OP_BWD_DQ ? sk::plan_bwd_dq(dtype, p, is_causal != 0)
+                             : sk::plan_bwd_reduce(dtype, p);
   } else if (decode) {
     int ns = 0, per = 0;
     const bool per_row = (variant & (SK_VARIANT_PAGED | SK_VARIANT_VARLEN)) != 0;
@@ -1102,7 +1130,7 @@ int sk_kernel_config(int op, int dtype, int B, int Hq, int Hkv, int Sq, int Sk, 
     return fail(SK_EINVAL, "unknown op %d", op);
   }
   if (!k.fn) return fail(SK_EUNSUPPORTED, "no kernel for op %d with these arguments", op);
-  cfg[SK_CFG_GRID] = (int64_t)k.grid.x * k.grid.y * k.grid.z;
+  cfg[SK_CFG_GRID] = (int64_t)k.grid.x * k.grid.y * k.grid.z / (op == SK_OP_FWD ? splits : 1);
   cfg[SK_CFG_THREADS] = (int64_t)k.block.x * k.block.y * k.block.z;
   cfg[SK_CFG_BLOCK_M] = k.block_m;
   cfg[SK_CFG_BLOCK_N] = k.block_n;
@@ -1113,6 +1141,8 @@ int sk_kernel_config(int op, int dtype, int B, int Hq, int Hkv, int Sq, int Sk, 
   cfg[SK_CFG_WORKSPACE] = (int64_t)ws;
   cfg[SK_CFG_KEYS_PER_SPLIT] = kps;
   cfg[SK_CFG_CHUNKS] = chunks;
+  cfg[SK_CFG_SIDE_STREAM] = side;
+  cfg[SK_CFG_PACKED_HEADS] = packed;
   cfg[SK_CFG_LDS_BYTES] = cfg[SK_CFG_VGPRS] = cfg[SK_CFG_WG_PER_CU] = -1;
   if (kernel_name && name_len)
     snprintf(kernel_name, name_len, "%s<%s, D=%d, BM=%d, BN=%d, stages=%d, causal=%d, paged=%d, rope=%d>",

@@ -1695,16 +1695,26 @@ KernelPlan plan_bwd_dq(int dtype, BwdParams& p, bool causal) {
   return KernelPlan{};
 }
 
-// Merge of a split dK/dV (nothing where it is unsplit).
-static hipError_t launch_dkv_reduce(int dtype, const BwdParams& p, bool causal, hipStream_t s) {
-  if (p.kv_iters <= 0) return hipSuccess;
+KernelPlan plan_bwd_reduce(int dtype, const BwdParams& p) {
+  if (dtype == 0) return plan_bwd_reduce_f32(p);
+  KernelPlan k;
+  if (p.kv_iters <= 0) return k;
   const int64_t n = (int64_t)p.B * p.Hkv * p.Sk * (p.D / 4);
-  const dim3 grid((unsigned)((n + 255) / 256), 2);
-  if (dtype == BF16::code)
-    hipLaunchKernelGGL(bwd_dkv_reduce_kernel<BF16>, grid, dim3(256), 0, s, p, causal);
-  else
-    hipLaunchKernelGGL(bwd_dkv_reduce_kernel<F16>, grid, dim3(256), 0, s, p, causal);
-  return hipGetLastError();
+  k.fn = dtype == BF16::code ? (const void*)bwd_dkv_reduce_kernel<BF16>
+                             : (const void*)bwd_dkv_reduce_kernel<F16>;
+  k.grid = dim3((unsigned)((n + 255) / 256), 2);
+  k.block = dim3(256);
+  k.kernel = "bwd_dkv_reduce_kernel";
+  k.elem = dtype;
+  k.head_dim = padded_head_dim(p.D);
+  return k;
+}
+
+hipError_t launch_bwd_reduce(int dtype, const BwdParams& p, bool causal, hipStream_t s) {
+  const KernelPlan k = plan_bwd_reduce(dtype, p);
+  if (!k.fn) return hipSuccess;
+  void* args[] = {const_cast<BwdParams*>(&p), &causal};
+  return hipLaunchKernel(k.fn, k.grid, k.block, args, 0, s);
 }
 
 // Side streams for the dQ kernel, one per (device, caller stream), each with
@@ -1764,6 +1774,15 @@ static const SideEntry* side_entry(hipStream_t s) {
   return &g_side[g_n_side++];
 }
 
+// Heavy blocks first where most blocks differ in work (S_k < 2 S_q); with
+// longer keys the order costs L2 hits and gains nothing (S_q = 2,048, S_k =
+// 8,192 0.6% slower).  B = 4, H = 32, S = 4,096 MHA: 1,930 us head-major,
+// 1,797 with dQ's blocks so, 1,778 with dK/dV's as well; H_kv = 8, S = 2,048:
+// 611, 559 and 462.
+static bool heavy_first(const BwdParams& p, bool causal) {
+  return causal && p.Sk < 2 * (int64_t)p.Sq;
+}
+
 // dK/dV and dQ only read what the preprocess pass and the caller wrote, and
 // write disjoint outputs.  Where that pays, dQ runs on the caller stream's
 // side stream, forked from the caller's stream after the preprocess pass and
@@ -1782,8 +1801,10 @@ static const SideEntry* side_entry(hipStream_t s) {
 // 879 us, non-causal S = 1,500, D = 256 609 and 535; causal S = 4,096, D = 256
 // 2,620 and 2,996, fp16 S = 1,024, D = 64 (48 heads) 57 and 60 with the host
 // 45 us longer.
-static bool fork_pays(const BwdParams& p, bool causal, int64_t dkv_wgs) {
-  if (dkv_wgs <= 256 || p.dkv_heavy_first) return false;
+bool bwd_forks(int dtype, const BwdParams& p, bool causal) {
+  const int64_t dkv_wgs = ((int64_t)p.Sk + 127) / 128 * p.B * p.Hkv * (p.D > 128 ? 2 : 1);
+  if ((dtype != BF16::code && dtype != F16::code) || p.ds != nullptr || p.Sq <= 0) return false;
+  if (dkv_wgs <= 256 || heavy_first(p, causal)) return false;
   const double seen = causal ? (double)p.Sq * (p.Sk - p.Sq / 2) : (double)p.Sq * p.Sk;
   const double steps = (double)p.B * p.Hq * (p.D > 128 ? 2 : 1) * seen / (32 * 128);
   return steps / 256 * dkv_step_us(p.D) >= 200;
@@ -1794,12 +1815,7 @@ static bool fork_pays(const BwdParams& p, bool causal, int64_t dkv_wgs) {
 // chunk's dS tiles and the dQ kernel reads them, both on the caller's stream.
 hipError_t launch_bwd_mfma(int dtype, const BwdParams& params, bool causal, hipStream_t s) {
   BwdParams p = params;
-  // Heavy blocks first where most blocks differ in work (S_k < 2 S_q); with
-  // longer keys the order costs L2 hits and gains nothing (S_q = 2,048, S_k =
-  // 8,192 0.6% slower).  B = 4, H = 32, S = 4,096 MHA: 1,930 us head-major,
-  // 1,797 with dQ's blocks so, 1,778 with dK/dV's as well; H_kv = 8, S = 2,048:
-  // 611, 559 and 462.
-  p.dkv_heavy_first = p.dq_heavy_first = causal && p.Sk < 2 * (int64_t)p.Sq;
+  p.dkv_heavy_first = p.dq_heavy_first = heavy_first(p, causal);
   if (dtype != BF16::code && dtype != F16::code) return hipErrorInvalidValue;
   const int64_t pairs = (int64_t)p.B * p.Hkv;
   if (p.ds != nullptr) {
@@ -1819,7 +1835,7 @@ hipError_t launch_bwd_mfma(int dtype, const BwdParams& params, bool causal, hipS
       if (e != hipSuccess) return e;
       if ((e = run_plan(dq, &q, s)) != hipSuccess) return e;
     }
-    return launch_dkv_reduce(dtype, p, causal, s);
+    return launch_bwd_reduce(dtype, p, causal, s);
   }
   BwdParams q = p;
   q.bk0 = 0;
@@ -1830,12 +1846,12 @@ hipError_t launch_bwd_mfma(int dtype, const BwdParams& params, bool causal, hipS
   const int64_t g_kv = (int64_t)q.n_nblocks * p.B * p.Hkv * (kv.head_dim == 256 ? 2 : 1);
   const int64_t g_q = (int64_t)q.n_mblocks * p.B * p.Hq;
   if (g_kv > 0x7fffffffLL || g_q > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-  const SideEntry* se = fork_pays(q, causal, g_kv) && g_q > 0 ? side_entry(s) : nullptr;
+  const SideEntry* se = bwd_forks(dtype, q, causal) ? side_entry(s) : nullptr;
   if (!se) {
     hipError_t e = run_plan(kv, &q, s);
     if (e != hipSuccess) return e;
     if ((e = run_plan(dq, &q, s)) != hipSuccess) return e;
-    return launch_dkv_reduce(dtype, q, causal, s);
+    return launch_bwd_reduce(dtype, q, causal, s);
   }
   hipError_t e = hipEventRecord(se->fork, s);
   if (e == hipSuccess) e = hipStreamWaitEvent(se->side, se->fork, 0);
@@ -1844,7 +1860,7 @@ hipError_t launch_bwd_mfma(int dtype, const BwdParams& params, bool causal, hipS
   // s's capture), so it is joined back whatever fails.
   const hipError_t e_dq = run_plan(dq, &q, se->side);
   hipError_t e_kv = e_dq == hipSuccess ? run_plan(kv, &q, s) : hipSuccess;
-  if (e_dq == hipSuccess && e_kv == hipSuccess) e_kv = launch_dkv_reduce(dtype, q, causal, s);
+  if (e_dq == hipSuccess && e_kv == hipSuccess) e_kv = launch_bwd_reduce(dtype, q, causal, s);
   hipError_t e_join = hipEventRecord(se->join, se->side);
   if (e_join == hipSuccess) e_join = hipStreamWaitEvent(s, se->join, 0);
   if (e_dq != hipSuccess) return e_dq;

@@ -1217,11 +1217,20 @@ hipError_t launch_bwd_f32(const BwdParams& p, bool causal, hipStream_t s) {
   hipError_t e = run_plan(dq, &q, s);
   if (e != hipSuccess) return e;
   if ((e = run_plan(kv, &q, s)) != hipSuccess) return e;
-  if (q.dq_iters <= 0 && q.kv_iters <= 0) return hipSuccess;
-  const int64_t rows = std::max((int64_t)q.B * q.Hq * q.Sq, (int64_t)q.B * q.Hkv * q.Sk);
-  const dim3 grid((unsigned)((rows * (q.D / 4) + 255) / 256), 3);
-  hipLaunchKernelGGL(bwd_f32_reduce_kernel, grid, dim3(256), 0, s, q, causal);
-  return hipGetLastError();
+  return launch_bwd_reduce(0, q, causal, s);
+}
+
+KernelPlan plan_bwd_reduce_f32(const BwdParams& p) {
+  KernelPlan k;
+  if (p.dq_iters <= 0 && p.kv_iters <= 0) return k;
+  const int64_t rows = std::max((int64_t)p.B * p.Hq * p.Sq, (int64_t)p.B * p.Hkv * p.Sk);
+  k.fn = (const void*)bwd_f32_reduce_kernel;
+  k.grid = dim3((unsigned)((rows * (p.D / 4) + 255) / 256), 3);
+  k.block = dim3(256);
+  k.kernel = "bwd_f32_reduce_kernel";
+  k.elem = 0;
+  k.head_dim = padded_head_dim(p.D);
+  return k;
 }
 
 }  // namespace sk

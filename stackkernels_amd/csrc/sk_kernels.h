@@ -296,6 +296,11 @@ KernelPlan plan_decode_combine(int dtype, const DecParams& p);
 // The backward plans fill the block counts of p they derive.
 KernelPlan plan_bwd_dkv(int dtype, BwdParams& p, bool causal);
 KernelPlan plan_bwd_dq(int dtype, BwdParams& p, bool causal);
+// Merge of the split gradients' partials (none where p is unsplit).
+KernelPlan plan_bwd_reduce(int dtype, const BwdParams& p);
+hipError_t launch_bwd_reduce(int dtype, const BwdParams& p, bool causal, hipStream_t s);
+// Whether dQ runs on the side stream, beside dK/dV (p.ds null: seven GEMMs).
+bool bwd_forks(int dtype, const BwdParams& p, bool causal);
 // Bytes of dS tiles the five-GEMM backward needs per (batch, KV head) pair
 // (its query heads' tiles), or 0 where the seven-GEMM backward runs (head
 // dims other than 65-128, fp32).
@@ -311,6 +316,7 @@ void bwd_dkv_split(int dtype, int B, int Hq, int Hkv, int Sq, int Sk, int D, boo
 void bwd_f32_split(int B, int Hq, int Hkv, int Sq, int Sk, int D, bool causal, BwdParams* p);
 KernelPlan plan_bwd_dkv_f32(BwdParams& p, bool causal);
 KernelPlan plan_bwd_dq_f32(BwdParams& p, bool causal);
+KernelPlan plan_bwd_reduce_f32(const BwdParams& p);
 
 // Launchers: return hipSuccess or the launch error.  dtype is SK_F32/F16/BF16.
 hipError_t launch_fwd_mfma(int dtype, const FwdParams& p, bool causal, hipStream_t s);
