@@ -1,12 +1,13 @@
 """The backward's two launch shapes, eagerly and under HIP graph capture.
 
-Seven GEMMs (head dims other than 65-128): when the dK/dV grid runs more than
-one round of workgroups, ``sk_attn_bwd`` forks the dQ kernel onto the side
-stream the library keeps for the caller's stream, after the preprocess pass,
-and joins it back with events.  Five GEMMs (D = 128): the dK/dV kernel stores
-dS in the workspace and the dQ kernel reads it after it, on the caller's
-stream.  The kernels use no atomics, so the result does not depend on how
-they overlap: every replay of a captured backward (fork and join become graph
+Seven GEMMs (head dims other than 65-128): for long calls in head-major order
+(dK/dV of 200 us or more, no mask or S_k >= 2 S_q) ``sk_attn_bwd`` forks the
+dQ kernel onto the side stream the library keeps for the caller's stream,
+after the preprocess pass, and joins it back with events; shorter calls run it
+on the caller's stream.  ``pick`` says which of the two a shape takes.  Five
+GEMMs (D = 128): the dK/dV kernel stores dS in the workspace and the dQ kernel
+reads it after it, on the caller's stream.  The kernels use no atomics, so the
+result does not depend on how they overlap: every replay of a captured backward (fork and join become graph
 edges) must equal, bit for bit, the eager call on the same inputs, and the
 eager call must match the oracle-checked fp32 reference within the bf16
 tolerance.
@@ -17,20 +18,30 @@ import torch
 
 from stackkernels_amd._core.attention.flash_bwd import flash_attn_bwd
 from stackkernels_amd._core.attention.flash_fwd import flash_attn_fwd
+from stackkernels_amd._opt.pick import pick
 from stackkernels_amd._reference.torch.attention import attention_reference
 
 from _gpu_util import TOL, assert_close_maxabs, native_loaded
 
 pytestmark = pytest.mark.gpu
 
-# B=2, H_kv=8, S_k=4096: 32 key blocks x 16 = 512 dK/dV workgroups, two rounds.
-SHAPE = dict(b=2, hq=16, hkv=8, sq=512, sk=4096)
-DIMS = {"seven_gemm_fork": 64, "five_gemm": 128}
+# B=2, H_kv=8, S_k=4096: 32 key blocks x 16 = 512 dK/dV workgroups, two rounds;
+# S_k=8192: 1,024 of them, about 400 us, with dQ forked.
+SHAPE = {}
+SHAPES = {
+    "seven_gemm_fork": dict(b=2, hq=32, hkv=8, sq=2048, sk=8192, d=64),
+    "seven_gemm": dict(b=2, hq=16, hkv=8, sq=512, sk=4096, d=64),
+    "five_gemm": dict(b=2, hq=16, hkv=8, sq=512, sk=4096, d=128),
+}
 
 
-@pytest.fixture(params=sorted(DIMS), autouse=True)
-def _head_dim(request):
-    SHAPE["d"] = DIMS[request.param]
+@pytest.fixture(params=sorted(SHAPES), autouse=True)
+def _shape(request):
+    SHAPE.update(SHAPES[request.param])
+    s = SHAPE
+    plan = pick("flash_bwd", (s["b"], s["hq"], s["sq"], s["d"]), dtype="bfloat16",
+                num_kv_heads=s["hkv"], kv_len=s["sk"], is_causal=True)
+    assert plan["dq"]["side_stream"] == (request.param == "seven_gemm_fork")
     yield
 
 

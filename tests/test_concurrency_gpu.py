@@ -3,10 +3,14 @@
 The library keeps per-process state that concurrent callers share: the table
 of side streams (one per caller stream, made on first use under a mutex) that
 the seven-GEMM backward forks its dQ kernel onto, and the thread-local error
-text; every call takes its scratch from the caller's workspace.  Four jobs run
-at once, on four host threads and four streams, three times each:
-* a D = 64 causal backward large enough to fork (512 dK/dV workgroups);
+text and last split plans; every call takes its scratch from the caller's
+workspace.  Eight jobs run at once, on as many host threads and streams, three
+times each:
+* a D = 64 backward that forks (``pick`` says so: no mask, 512 dK/dV
+  workgroups of about 230 us), beside a causal one of that size that does not;
 * a D = 128 five-GEMM backward (its dS tiles in the call's own workspace);
+* a D = 96 backward and an fp32 one whose gradients are summed in chunks;
+* a forward whose keys are split;
 * a per-row-length decode;
 * a paged decode.
 
@@ -23,6 +27,7 @@ import torch
 
 from stackkernels_amd._core.attention.flash_bwd import flash_attn_bwd
 from stackkernels_amd._core.attention.flash_fwd import flash_attn_fwd
+from stackkernels_amd._opt.pick import pick
 from stackkernels_amd.torch import flash_decode
 
 from _gpu_util import native_loaded
@@ -48,6 +53,12 @@ def _train_job(b, hq, hkv, s, d, dtype, causal, seed):
     return run
 
 
+def _split_job(seed):
+    q, k, v = (_rand((1, h, s, 128), torch.bfloat16, seed + i)
+               for i, (h, s) in enumerate(((32, 512), (8, 16000), (8, 16000))))
+    return lambda: flash_attn_fwd(q, k, v, is_causal=True)
+
+
 def _decode_job(paged, seed):
     dtype = torch.float16 if paged else torch.bfloat16
     b, hq, hkv, d = 8, 32, 8, 128
@@ -66,11 +77,23 @@ def _decode_job(paged, seed):
 
 def test_concurrent_threads_and_streams_match_serial_results(device):
     jobs = {
-        "bwd_d64_forked": _train_job(2, 8, 8, 4096, 64, torch.bfloat16, True, 10),
+        "bwd_d64_forked": _train_job(2, 16, 8, 4096, 64, torch.bfloat16, False, 10),
+        "bwd_d64_heavy_first": _train_job(2, 8, 8, 4096, 64, torch.bfloat16, True, 15),
+        "bwd_d96_chunks": _train_job(1, 32, 8, 2000, 96, torch.bfloat16, True, 50),
+        "bwd_f32_chunks": _train_job(2, 8, 8, 1024, 64, torch.float32, False, 60),
+        "fwd_key_splits": _split_job(70),
         "bwd_d128_five_gemm": _train_job(1, 8, 2, 1024, 128, torch.float16, False, 20),
         "decode_varlen": _decode_job(False, 30),
         "decode_paged": _decode_job(True, 40),
     }
+    def plan(op, b, h, s, d, **kw):
+        return pick(op, (b, h, s, d), dtype=kw.pop("dtype", "bfloat16"), **kw)
+
+    assert plan("flash_bwd", 2, 16, 4096, 64, num_kv_heads=8)["dq"]["side_stream"]
+    assert plan("flash_bwd", 1, 32, 2000, 96, num_kv_heads=8, is_causal=True)["splits"] > 1
+    assert plan("flash_bwd", 2, 8, 1024, 64, dtype="float32")["dq"]["splits"] > 1
+    assert plan("flash_attn", 1, 32, 512, 128, num_kv_heads=8, kv_len=16000,
+                is_causal=True)["SPLIT_KV"] > 1
     expect = {name: job() for name, job in jobs.items()}
     torch.cuda.synchronize()
     assert native_loaded()
