@@ -84,51 +84,73 @@ int check_ptr(const char* name, const void* p) {
 //   against two and three, 64 units, S_k = 16,384: 174, 191 and 205 us with
 //   16-head groups, 168, 176 and 186 with 4; 16 units, S_k = 32,768: 94, 112
 //   and 120), and per-row lengths
-//   take two such rounds at any length (368, S_k <= 976 53.4 us at 2 splits,
-//   42.1 at 5, 47.3 at 6; 800, S_k <= 1,500 121 at 2, 130 at 3);
+//   take two such rounds that fit (368, S_k <= 976 53.4 us at 2 splits, 42.1 at
+//   5, 47.3 at 6; 800, S_k <= 1,500 121 at 2, 130 at 3), two splits above
+//   1,024 units (1,120, S_k <= 1,572 179 us whole, 155 at 2, 163 at 4; 147
+//   shapes up to 2,047 units 1% below three or four splits on average);
 // * 32- and 64-head groups: exactly one round, so no split waits for a second
 //   round; a 64-head group writes 32 KB of partials per split, so fewer,
 //   longer splits also keep that traffic small (C5: 64 splits; 32 and 128
 //   splits measured 15% and 10% slower).
 // A split keeps at least 256 keys, 128 with 64 to 384 (batch, KV head) units
 // of up to 16 heads (360 units, S_k <= 500, D = 128: 28.0 us whole, 20.9 at 3
-// splits; 800 units, S_k <= 700: 45.0 at 2, 47.9 at 3).  Small calls (at most 1,024 query heads in all,
-// whose partials cost the combine little) split further, because a split's
-// tiles follow one another: to 64 keys while that gives at most 512
-// workgroups (128 with the 64-key tiles of groups above 32), to one 32-key
-// tile while at most 256.  Microseconds of both kernels (graph replays), H_q =
-// 32, H_kv = 8, D = 128 bf16, 256 keys a split -> now: B = 1, S_k = 1,000 19.2
-// -> 8.4 (32 splits), S_k = 4,096 16.2 -> 10.8 (64); B = 16, S_k = 1,000 22.4
-// -> 19.3 (7); MQA, 64 heads, B = 1, S_k = 8,192 13.8 -> 11.6 (64).  Past
-// those limits more splits lose: B = 1, S_k = 32,768 31 us at 128, 36 at 256;
-// 64 x 64 heads, S_k = 500 16 us whole, 23 at 6.  Caches below 192 keys stay
-// whole.
+// splits; 800 units, S_k <= 700: 45.0 at 2, 47.9 at 3).  Small calls (at most
+// 1,024 query heads in all, whose partials cost the combine little) split
+// further, because a split's tiles follow one another:
+// * up to 32 heads a group, to 64 keys while that gives at most 512 workgroups
+//   and to one 32-key tile while at most 256.  Microseconds of both kernels
+//   (graph replays), H_q = 32, H_kv = 8, D = 128 bf16, 256 keys a split -> so: B
+//   = 1, S_k = 1,000 19.2 -> 8.4 (32 splits), S_k = 4,096 16.2 -> 10.8 (64); B
+//   = 16, S_k = 1,000 22.4 -> 19.3 (7).  Past those limits more splits lose: B =
+//   1, S_k = 32,768 31 us at 128, 36 at 256; 64 x 64 heads, S_k = 500 16 us
+//   whole, 23 at 6;
+// * above 32, to 128 keys while at most 256 workgroups of the 64-key tiles up to
+//   D = 128 (16 units, S_k = 3,356 19.6 us at 13 splits, 19.2 at 16, 21.2 at
+//   21), and there from three splits on (2 units, S_k = 263 8.2 us whole, 10.1
+//   at 2), or 512 above (15 units, S_k = 6,286 17% faster with 33 than with 22);
+// * above 16, to at most 64 splits, whose partials are read by one workgroup
+//   per head: 64 heads, 2 units, S_k = 27,491 19.7 us at 107 splits of 256
+//   keys, 22.5 at 215 of 128; 32 heads, 1 unit, S_k = 34,585 22.8 and 28.4.
+// Caches below 192 keys stay whole, below 256 at head dims up to 64 and, up to
+// 128, in groups above 16 (16 units, S_k = 211, D = 64 7.6 us whole, 8.4 at 7).
 // Up to D = 128 per-row lengths take their second round only where the longest
-// row gives each split 512 keys, 352 up to 384 units (B = 32, U[1, 4,096], 256 keys: 54.6 us with 16
-// splits, 53.1 with 8; 720 units, U[1, 1,500], 300 keys: 64.6 with 5, 59.3 with
-// 3; 368 units, U[1, 4,000], 363 keys: 57.4 with 11, 64.6 with 6; 800 units,
-// U[1, 3,000], 600 keys: 113.6 with 5, 118.8 with 3).  The count is capped at 1024
-// (the combine kernel's LDS weight array).
+// row gives each split 512 keys, 352 up to 384 units (B = 32, U[1, 4,096], 256
+// keys: 54.6 us with 16 splits, 53.1 with 8; 720 units, U[1, 1,500], 300 keys:
+// 64.6 with 5, 59.3 with 3; 368 units, U[1, 4,000], 363 keys: 57.4 with 11,
+// 64.6 with 6; 800 units, U[1, 3,000], 600 keys: 113.6 with 5, 118.8 with 3).
+// Groups of one or two heads write few partials, and take it from 256 keys on
+// and shorter rounds that fit 256 (14 x 32 heads, U[1, 4,467], D = 96 53.5 us
+// with 5, 49.4 with 10; 9 x 12, U[1, 10,680] 54.8 with 19, 51.6 with 38; 16 x
+// 8, U[1, 5,263] 38.8 with 15, 37.1 with 20).  Over 436 shapes of 90 to 1,300
+// units (S_k 800 to 16,384) that is 3.2% below two rounds of 256 keys for all.
+// The count is capped at 1024 (the combine kernel's LDS weight array).
 int plan_splits(int B, int Hq, int Hkv, int Sk, int D, bool per_row) {
-  if (Sk < 192 || B <= 0 || Hkv <= 0) return 1;
+  if (B <= 0 || Hkv <= 0) return 1;
   const int group = Hq / Hkv;
+  if (Sk < (D <= 64 || (D <= 128 && group > 16) ? 256 : 192)) return 1;
   const int waves = group <= 16 ? 1 : group <= 32 ? 2 : 4;
   const int64_t slots = 256LL * 8 / waves;
   const int64_t units = (int64_t)B * Hkv;
   int64_t splits = (slots + units - 1) / units;
   if (group <= 16 && per_row) {
     const int64_t two = 2 * slots / units;
-    if (D > 128) splits = slots / units;
-    else if (Sk >= two * (units <= 384 ? 352 : 512)) splits = std::max(splits, two);
+    if (D > 128) {
+      if (units <= slots / 2) splits = slots / units;
+    } else if (group <= 2 && units <= slots / 2) {
+      splits = std::max(splits, std::min<int64_t>((2 * slots + units - 1) / units, Sk / 256));
+    } else if (Sk >= two * (units <= 384 ? 352 : 512)) {
+      splits = std::max(splits, two);
+    }
   } else if (group <= 16) {
     if (D <= 128) splits = slots / units;
     else if (units <= slots / 2) splits = slots / 2 / units;
   }
   int64_t most = Sk / (group <= 16 && units >= 64 && units <= 384 ? 128 : 256);
-  if ((int64_t)B * Hq <= 1024) {
-    most = std::max<int64_t>(most, std::min<int64_t>(512 / units, Sk / (group > 32 ? 128 : 64)));
-    if (group <= 32)
-      most = std::max<int64_t>(most, std::min<int64_t>(256 / units, (Sk + 31) / 32));
+  if ((int64_t)B * Hq <= 1024 && (group <= 32 || D > 128 || Sk >= 384)) {
+    const int fits = group > 32 && D <= 128 ? 256 : 512;
+    int64_t fine = std::min<int64_t>(fits / units, Sk / (group > 32 ? 128 : 64));
+    if (group <= 32) fine = std::max(fine, std::min<int64_t>(256 / units, (Sk + 31) / 32));
+    most = std::max(most, group > 16 ? std::min<int64_t>(fine, 64) : fine);
   }
   splits = std::min(splits, most);
   return (int)std::max<int64_t>(1, std::min<int64_t>(splits, 1024));
