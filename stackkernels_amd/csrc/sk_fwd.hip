@@ -53,9 +53,10 @@
 //   long rows do not trail at the end of the grid.  Under the causal mask a
 //   workgroup runs query blocks j and n-1-j back to back when the grid
 //   stays at two or more workgroups per CU, which evens out the work per
-//   workgroup and halves the per-item fixed cost; smaller causal grids start
-//   every head's heavy blocks before any light one (bf16, H_q = 32, H_kv = 8,
-//   D = 128, B = 2, S = 1,337, 704 workgroups: 54 us head-major, 43 so).
+//   workgroup and halves the per-item fixed cost; causal grids of half a round
+//   to two rounds of the chip start every head's heavy blocks before any light
+//   one (bf16, H_q = 32, H_kv = 8, D = 128, B = 2, S = 1,337, 704 workgroups: 54
+//   us head-major, 43 so).
 #include <algorithm>
 #include <type_traits>
 
@@ -150,6 +151,10 @@ __global__ void __launch_bounds__(NW * 64, OCC) fwd_mfma_kernel(FwdParams p) {
   int bh = iw / p.n_items;
   int item = iw - bh * p.n_items;
   if (CAUSAL && !SPLIT && p.heavy_first) heavy_first_order(blockIdx.x, p.B * p.Hq, bh, item);
+  if constexpr (CAUSAL && !SPLIT) {  // (else the join's copies lie in VGPRs, q's resource too)
+    bh = __builtin_amdgcn_readfirstlane(bh);
+    item = __builtin_amdgcn_readfirstlane(item);
+  }
   // Packed rows (split kernels): the unit is a (batch, KV head) and its rows
   // are the group's heads one after the other, row r query r % Sq of head
   // r / Sq; hq is the first head.  Else the rows are one head's queries.
@@ -945,10 +950,16 @@ KernelPlan plan_fwd_mfma(int dtype, const FwdParams& p, bool causal) {
 
 hipError_t launch_fwd_mfma(int dtype, const FwdParams& params, bool causal, hipStream_t s) {
   FwdParams p = params;
-  // Unpaired causal grids only: paired blocks carry equal work, and head-major
-  // order then keeps each head's K/V in one L2 (B * H = 128, S = 4,096 527 us,
-  // 575 with the blocks outermost).
-  p.heavy_first = causal && !p.pair_items && !p.part_o;
+  // Unpaired causal grids between half a round and two rounds of the chip:
+  // 4-21% on average over 80 shapes there.  Below, every block starts at once;
+  // above, later blocks fill in behind long ones anyway and head-major order
+  // keeps a head's K/V in one L2 (over 100 shapes from 2.5 rounds on neutral on
+  // average, up to 6% slower heavy first: 24 heads on 2, B = 10, S = 1,011, D =
+  // 64 63.9 us, 67.7).  Paired blocks carry equal work (B * H = 128, S = 4,096
+  // 527 us, 575 with the blocks outermost).
+  const int64_t wgs = (int64_t)p.n_items * p.B * p.Hq;
+  const int slots = 256 * fwd_config(p.D, (int64_t)p.B * p.Hq, p.Sq, p.Sk, causal).occ;
+  p.heavy_first = causal && !p.pair_items && !p.part_o && 2 * wgs > slots && wgs <= 2 * slots;
   const KernelPlan k = plan_fwd_mfma(dtype, p, causal);
   if (!k.fn) return hipErrorInvalidValue;
   return run_plan(k, &p, s);
