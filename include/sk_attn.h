@@ -174,12 +174,14 @@ SK_API int sk_attn_bwd_workspace_min(int dtype, int B, int Hq, int Hkv, int Sq, 
  * the workspace and the dQ kernel reads it, both on `stream`.  The results
  * are the same bit for bit for every chunking and equal the seven-GEMM
  * backward's.  Seven-GEMM backward (other head dims, fp32, or a workspace
- * too small for one pair's tiles): where the dK/dV kernel runs more than one round of workgroups
- * (more than 256) in head-major order (no mask, or S_k >= 2 S_q) for about
- * 200 us or more, the dQ kernel runs on the library's side stream for `stream`, forked from `stream` after the preprocess pass and joined back
- * into it (also when a launch fails); under graph capture the fork and the
- * join are recorded as graph edges.  A call under capture on a stream that
- * has never run an eager backward keeps the one-stream order.
+ * too small for one pair's tiles): where the dK/dV kernel runs more than one
+ * round of workgroups (more than 256) in head-major order (no mask, S_k >= 2
+ * S_q, or many rounds) and both kernels take about 140 us or more, the dQ
+ * kernel runs on the library's side stream for `stream`, forked from `stream`
+ * after the preprocess pass and joined back into it (also when a launch
+ * fails); under graph capture, and there whatever the kernels take, the fork
+ * and the join are recorded as graph edges.  A call under capture on a stream
+ * that has never run such a backward eagerly keeps the one-stream order.
  */
 SK_API int sk_attn_bwd(int dtype, const void* dout, const void* q, const void* k, const void* v,
                 const void* o, const float* lse, void* dq, void* dk, void* dv,
@@ -486,7 +488,7 @@ SK_API int sk_kv_cache_update_paged_rope(int dtype, const void* k, const void* v
 #define SK_CFG_VGPRS 11         /* device-reported registers per lane, or -1    */
 #define SK_CFG_WG_PER_CU 12     /* device-reported resident workgroups per CU, or -1 */
 #define SK_CFG_CHUNKS 13        /* backward: launches of the kernel per call (chunks of pairs) */
-#define SK_CFG_SIDE_STREAM 14   /* dQ: 1 where it runs beside dK/dV on the side stream */
+#define SK_CFG_SIDE_STREAM 14   /* dQ: 1 where an eager call runs it beside dK/dV on the side stream */
 #define SK_CFG_PACKED_HEADS 15  /* forward: heads of a group that share blocks of rows (1) */
 #define SK_CFG_LEN 16
 

@@ -1774,13 +1774,31 @@ static const SideEntry* side_entry(hipStream_t s) {
   return &g_side[g_n_side++];
 }
 
-// Heavy blocks first where most blocks differ in work (S_k < 2 S_q); with
-// longer keys the order costs L2 hits and gains nothing (S_q = 2,048, S_k =
-// 8,192 0.6% slower).  B = 4, H = 32, S = 4,096 MHA: 1,930 us head-major,
-// 1,797 with dQ's blocks so, 1,778 with dK/dV's as well; H_kv = 8, S = 2,048:
-// 611, 559 and 462.
-static bool heavy_first(const BwdParams& p, bool causal) {
-  return causal && p.Sk < 2 * (int64_t)p.Sq;
+// Workgroups of an unsplit dK/dV launch.
+static int64_t dkv_workgroups(const BwdParams& p) {
+  return ((int64_t)p.Sk + 127) / 128 * launch_pairs(p) * (p.D > 128 ? 2 : 1);
+}
+
+// Heavy blocks first, for a kernel of that many workgroups, where most blocks
+// differ in work (S_k < 2 S_q); with longer keys the order costs L2 hits and
+// gains nothing (S_q = 2,048, S_k = 8,192 0.6% slower).  B = 4, H = 32, S = 4,096
+// MHA: 1,930 us head-major, 1,797 with dQ's blocks so, 1,778 with dK/dV's as
+// well; H_kv = 8, S = 2,048: 611, 559 and 462.  Grids of up to 256 workgroups
+// start at once and stay head-major (fp16, 2 x 12 heads, S = 1,113, D = 64, 216
+// of each: 54.5 us heavy first, 51.8 so), and so do both kernels where dK/dV
+// runs many rounds, whose end weighs little beside the L2 hits (90 causal
+// squares; D = 64 gains 2-9% below 2,400 workgroups, loses 1-6% above 2,600; D
+// = 128 gains 2-12% up to 4,640, neutral at 5,000; D = 256 loses 1-5% from
+// 1,400 on and 20% at 9,000: 10 x 32 heads, S = 1,744 3,597 us, 2,998 so).
+// Where the fork is the alternative (head dims up to 64 and above 128) and the
+// keys are read by one or two heads, that is the better one from S_k = 1.5 S_q
+// on (2 x 8 heads, 1,598 x 2,603, D = 64 86.4 us heavy first, 71.9 forked; 2 x
+// 12, 1,103 x 1,697, D = 256 246 and 226).
+static bool heavy_first(const BwdParams& p, bool causal, int64_t wgs) {
+  const int64_t most = p.D <= 64 ? 2560 : p.D <= 128 ? 4608 : 1280;
+  const bool few = p.group <= 2 && (p.D <= 64 || p.D > 128);
+  return causal && (few ? 2 * (int64_t)p.Sk < 3 * (int64_t)p.Sq : p.Sk < 2 * (int64_t)p.Sq) &&
+         wgs > 256 && dkv_workgroups(p) <= most;
 }
 
 // dK/dV and dQ only read what the preprocess pass and the caller wrote, and
@@ -1796,18 +1814,35 @@ static bool heavy_first(const BwdParams& p, bool causal) {
 // call without, 65 with), and two kernels that mix on the chip evict each
 // other's tiles, so it is kept for calls of more than one round, in
 // head-major order (heavy-first grids end evenly by themselves) and long
-// enough to hide it: dK/dV of 200 us or more by its step count.  bf16, one
-// stream against the fork: H_q = 32, H_kv = 8, 2,048 x 8,192, D = 64 922 and
-// 879 us, non-causal S = 1,500, D = 256 609 and 535; causal S = 4,096, D = 256
-// 2,620 and 2,996, fp16 S = 1,024, D = 64 (48 heads) 57 and 60 with the host
-// 45 us longer.
-bool bwd_forks(int dtype, const BwdParams& p, bool causal) {
-  const int64_t dkv_wgs = ((int64_t)p.Sk + 127) / 128 * p.B * p.Hkv * (p.D > 128 ? 2 : 1);
+// enough to hide it: 140 us or more of kernels, by a sum of both kernels' steps
+// fitted to 90 shapes (5% off at the median).  It gains most where the queries
+// are few and dQ's grid leaves CUs idle.  bf16, one stream against the fork:
+// H_q = 32, H_kv = 8, 2,048 x 8,192, D = 64 922 and 879 us, non-causal S =
+// 1,500, D = 256 609 and 535, 2 x 12 heads, 320 x 7,125, D = 64 184 and 140, 3
+// x 16, 109 x 3,968, D = 256 416 and 256; fp16 S = 1,024, D = 64 (48 heads) 57
+// and 60 with the host 45 us longer.  A replayed graph has no host calls to
+// hide, so under capture every such call forks, whatever its length (2 x 16
+// heads, 348 x 3,219, D = 64 102 us on one stream, 71 forked).
+static bool may_fork(int dtype, const BwdParams& p, bool causal) {
+  const int64_t wgs = dkv_workgroups(p);
   if ((dtype != BF16::code && dtype != F16::code) || p.ds != nullptr || p.Sq <= 0) return false;
-  if (dkv_wgs <= 256 || heavy_first(p, causal)) return false;
-  const double seen = causal ? (double)p.Sq * (p.Sk - p.Sq / 2) : (double)p.Sq * p.Sk;
-  const double steps = (double)p.B * p.Hq * (p.D > 128 ? 2 : 1) * seen / (32 * 128);
-  return steps / 256 * dkv_step_us(p.D) >= 200;
+  return wgs > 256 && !heavy_first(p, causal, wgs);
+}
+bool bwd_forks(int dtype, const BwdParams& p, bool causal) {
+  if (!may_fork(dtype, p, causal)) return false;
+  const int64_t wgs = dkv_workgroups(p);
+  // Microseconds of a dK/dV step (32 queries x 128 keys) and workgroup, of a dQ
+  // step (128 x 32) and workgroup, and dQ's slots.
+  const double kStep = p.D <= 64 ? 0.81 : p.D <= 128 ? 1.1 : 1.53;
+  const double kWg = p.D <= 64 ? 4.6 : p.D <= 128 ? 6.5 : 8.9;
+  const double qStep = p.D <= 64 ? 0.43 : p.D <= 128 ? 0.8 : 1.65;
+  const double qWg = p.D <= 64 ? 6.2 : p.D <= 128 ? 10 : 22.4;
+  const double slots = p.D <= 128 ? 512 : 256;
+  const double keys = causal ? std::max(0.0, p.Sk - p.Sq / 2.0) : p.Sk;  // per query, mean
+  const double steps = (double)p.B * p.Hq * (p.D > 128 ? 2 : 1) * p.Sq * keys / (32 * 128);
+  const double rounds = std::max(1.0, (double)((p.Sq + 127) / 128) * p.B * p.Hq / slots);
+  const double us = 13 + (kStep * steps + kWg * wgs) / 256 + rounds * (qStep * keys / 32 + qWg);
+  return us >= 140;
 }
 
 // Five-GEMM backward (p.ds set, p.n_pairs the pairs per chunk): for each
@@ -1815,7 +1850,6 @@ bool bwd_forks(int dtype, const BwdParams& p, bool causal) {
 // chunk's dS tiles and the dQ kernel reads them, both on the caller's stream.
 hipError_t launch_bwd_mfma(int dtype, const BwdParams& params, bool causal, hipStream_t s) {
   BwdParams p = params;
-  p.dkv_heavy_first = p.dq_heavy_first = heavy_first(p, causal);
   if (dtype != BF16::code && dtype != F16::code) return hipErrorInvalidValue;
   const int64_t pairs = (int64_t)p.B * p.Hkv;
   if (p.ds != nullptr) {
@@ -1831,6 +1865,8 @@ hipError_t launch_bwd_mfma(int dtype, const BwdParams& params, bool causal, hipS
       const KernelPlan kv = plan_bwd_dkv(dtype, q, causal);
       const KernelPlan dq = plan_bwd_dq(dtype, q, causal);
       if (!kv.fn || !dq.fn) return hipErrorInvalidValue;
+      q.dkv_heavy_first = heavy_first(q, causal, kv.grid.x);
+      q.dq_heavy_first = heavy_first(q, causal, dq.grid.x);
       hipError_t e = run_plan(kv, &q, s);
       if (e != hipSuccess) return e;
       if ((e = run_plan(dq, &q, s)) != hipSuccess) return e;
@@ -1846,7 +1882,18 @@ hipError_t launch_bwd_mfma(int dtype, const BwdParams& params, bool causal, hipS
   const int64_t g_kv = (int64_t)q.n_nblocks * p.B * p.Hkv * (kv.head_dim == 256 ? 2 : 1);
   const int64_t g_q = (int64_t)q.n_mblocks * p.B * p.Hq;
   if (g_kv > 0x7fffffffLL || g_q > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-  const SideEntry* se = bwd_forks(dtype, q, causal) ? side_entry(s) : nullptr;
+  q.dkv_heavy_first = heavy_first(q, causal, kv.grid.x);
+  q.dq_heavy_first = heavy_first(q, causal, dq.grid.x);
+  // (The entry is made by eager calls that do not fork as well: a capture can't.)
+  const SideEntry* se = may_fork(dtype, q, causal) ? side_entry(s) : nullptr;
+  if (se && !bwd_forks(dtype, q, causal)) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
+      (void)hipGetLastError();
+      cap = hipStreamCaptureStatusNone;
+    }
+    if (cap == hipStreamCaptureStatusNone) se = nullptr;
+  }
   if (!se) {
     hipError_t e = run_plan(kv, &q, s);
     if (e != hipSuccess) return e;

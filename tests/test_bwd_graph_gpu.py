@@ -1,10 +1,10 @@
 """The backward's two launch shapes, eagerly and under HIP graph capture.
 
 Seven GEMMs (head dims other than 65-128): for long calls in head-major order
-(dK/dV of 200 us or more, no mask or S_k >= 2 S_q) ``sk_attn_bwd`` forks the
+(140 us or more of kernels, no mask or S_k >= 2 S_q) ``sk_attn_bwd`` forks the
 dQ kernel onto the side stream the library keeps for the caller's stream,
 after the preprocess pass, and joins it back with events; shorter calls run it
-on the caller's stream.  ``pick`` says which of the two a shape takes.  Five
+on the caller's stream, except under capture.  ``pick`` says which of the two a shape takes.  Five
 GEMMs (D = 128): the dK/dV kernel stores dS in the workspace and the dQ kernel
 reads it after it, on the caller's stream.  The kernels use no atomics, so the
 result does not depend on how they overlap: every replay of a captured backward (fork and join become graph
@@ -30,6 +30,7 @@ pytestmark = pytest.mark.gpu
 SHAPE = {}
 SHAPES = {
     "seven_gemm_fork": dict(b=2, hq=32, hkv=8, sq=2048, sk=8192, d=64),
+    # eagerly on one stream, forked under capture
     "seven_gemm": dict(b=2, hq=16, hkv=8, sq=512, sk=4096, d=64),
     "five_gemm": dict(b=2, hq=16, hkv=8, sq=512, sk=4096, d=128),
 }

@@ -86,8 +86,11 @@ def test_split_backward(dtype, b, hq, hkv, sq, sk, d, causal, dq_split):
     (("bfloat16", 2, 32, 8, 2048, 8192, 64, True), True),     # long, keys 4 x queries
     (("bfloat16", 4, 32, 8, 1500, 1500, 256, False), True),
     (("bfloat16", 2, 8, 8, 4096, 4096, 64, True), False),     # heavy blocks first
-    (("bfloat16", 2, 16, 8, 512, 4096, 64, True), False),     # 27 us of dK/dV
+    (("bfloat16", 2, 16, 8, 512, 4096, 64, True), False),     # too short
     (("bfloat16", 2, 32, 8, 2048, 8192, 128, True), False),   # five GEMMs
+    (("bfloat16", 2, 12, 12, 320, 7125, 64, False), True),    # few queries: dQ's grid is small
+    (("float16", 10, 32, 32, 1744, 1744, 256, True), True),   # 35 rounds: head-major again
+    (("bfloat16", 5, 16, 16, 1008, 1008, 64, False), False),  # 130 us: the host would show
     (("float32", 2, 32, 8, 2048, 8192, 64, True), False),
 ])
 def test_side_stream(dims, forks):
