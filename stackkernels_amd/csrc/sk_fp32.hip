@@ -625,10 +625,20 @@ static bool fwd_f32_on_mfma(int d, int sq) {
 // 16.5 at 128; half a tile of prologue).  B * H = 16, S = 1,024, D = 64: 64
 // workgroups 135 us, 4 splits 58 with the merge (MQA, 8 heads, 300 x 3,000, D =
 // 96: 703 and 72).
-int fwd_f32_key_splits(int d, int64_t bh, int sq, int sk) {
+// The model takes every block for a full one.  Under the causal mask two kinds
+// of calls run so much shorter whole that splitting them lost, and stay whole:
+// grids just over a round of three to six blocks a head, whose light blocks
+// fill in (288 blocks, S = 647, D = 64 119 us whole, 153 in 4; 320, S = 1,194,
+// D = 96 341 and 444); and, by their own times, squares whose second and last
+// block has up to 128 rows, one wave per SIMD (96 blocks, S = 344, D = 64 34
+// and 37.5).
+int fwd_f32_key_splits(int d, int64_t bh, int sq, int sk, bool causal) {
   if (!fwd_f32_on_mfma(d, sq) || sk <= 0 || bh <= 0) return 1;
   const int64_t items = (int64_t)((sq + kF32MmaRows - 1) / kF32MmaRows) * bh;
   if (items >= 384) return 1;
+  const int nb = (sq + kF32MmaRows - 1) / kF32MmaRows;
+  if (causal && items > 256 && nb >= 3 && nb <= 6) return 1;
+  const bool thin = causal && nb == 2 && sq <= 384 && sk < sq + 128;
   const double tile_us = d <= 64 ? 8.4 : 16.5;
   const double tiles = sk / 64.0;
   const double merge_us = (double)bh * sq * d * 8 / 1.2e7;
@@ -638,7 +648,9 @@ int fwd_f32_key_splits(int d, int64_t bh, int sq, int sk) {
   for (int ns = 1; ns <= most; ++ns) {
     if (ns > 1 && sk < ns * 64) break;
     const int64_t load = (items * ns + 255) / 256;
-    const double us = load * (tiles / ns + 0.5) * tile_us + (ns > 1 ? 8 + ns * merge_us : 0);
+    double t = tiles / ns;
+    if (thin) t = ns == 1 ? std::max((256 + sk - sq) / 64.0, 0.55 * tiles) : fwd_split_keys(sk, ns) / 64;
+    const double us = load * (t + 0.5) * tile_us + (ns > 1 ? 8 + ns * merge_us : 0);
     if (ns == 1) one_us = us;
     if (ns == 1 || us < best_us) best = ns, best_us = us;
   }

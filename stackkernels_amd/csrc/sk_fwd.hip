@@ -846,7 +846,7 @@ FwdSplit fwd_key_splits(int dtype, int d, int B, int Hq, int Hkv, int sq, int sk
   FwdSplit out;
   if (sq <= 0 || sk <= 0 || bh <= 0 || Hkv <= 0) return out;
   if (dtype == 0) {
-    out.splits = fwd_f32_key_splits(d, bh, sq, sk);
+    out.splits = fwd_f32_key_splits(d, bh, sq, sk, causal);
     return out;
   }
   if (dtype != BF16::code && dtype != F16::code) return out;

@@ -344,7 +344,7 @@ struct FwdSplit {
   bool on() const { return splits > 1 || pack > 1; }
 };
 FwdSplit fwd_key_splits(int dtype, int d, int B, int Hq, int Hkv, int sq, int sk, bool causal);
-int fwd_f32_key_splits(int d, int64_t bh, int sq, int sk);
+int fwd_f32_key_splits(int d, int64_t bh, int sq, int sk, bool causal);
 int fwd_most_splits(int64_t rows, int d);
 int fwd_split_keys(int sk, int splits);
 int fwd_split_blocks(int64_t rows);

@@ -54,6 +54,19 @@ def test_split_forward_f32():
     assert f["workspace_bytes"] == _bytes("sk_attn_fwd_workspace", *dims)
 
 
+@pytest.mark.parametrize("b,hq,hkv,s,d,split", [
+    (3, 32, 32, 647, 64, False),   # 288 blocks, three a head
+    (2, 32, 1, 1194, 96, False),
+    (3, 16, 4, 344, 64, False),    # a thin second block
+    (1, 8, 8, 390, 64, True),
+    (3, 16, 4, 490, 128, True),
+    (2, 16, 4, 2139, 80, True),    # nine blocks a head
+])
+def test_f32_causal_squares(b, hq, hkv, s, d, split):
+    f = _pick("flash_attn", "float32", b, hq, hkv, s, s, d, True)
+    assert (f["SPLIT_KV"] > 1) == split
+
+
 def test_whole_forward_has_no_merge():
     f = _pick("flash_attn", "bfloat16", 4, 32, 32, 4096, 4096, 128, True)
     assert f["SPLIT_KV"] == f["packed_heads"] == 1 and f["workspace_bytes"] == 0
