@@ -87,19 +87,19 @@ PEAK_NOTE = {
 # so these are recorded figures.  TRAFFIC_SOURCES_SHA256 is the digest of the
 # kernel sources (kernel_sources_digest) the counters were measured on; when
 # the sources differ, the line reports traffic null rather than a stale figure.
-TRAFFIC_SOURCES_SHA256 = "caabc7557ffd45bbbc639c87567a7368ad6532d52283fbb03d5e3d5445c1d131"
+TRAFFIC_SOURCES_SHA256 = "380e706a9f9ff00cc6737510addb9f5c4a9dcb38b77195f4b5061a0dbe89fb8d"
 HBM_TRAFFIC_BYTES = {
-    "fwd": 681_165_750,
-    "fwd_long": 838_971_108,
-    "fwdbwd": 4_535_370_302,
-    "decode": 8_601_597_260,
-    "decode_mqa": 573_053_237,
-    "decode_varlen": 4_305_224_903,
-    "kv_update": 67_240_127,
-    "decode_paged": 4_305_376_554,
-    "decode_rope": 8_601_618_835,
-    "kv_update_rope": 75_523_377,
-    "decode_step": 4_306_761_979,
+    "fwd": 681_380_439,
+    "fwd_long": 843_569_282,
+    "fwdbwd": 4_537_210_787,
+    "decode": 8_601_609_521,
+    "decode_mqa": 573_052_296,
+    "decode_varlen": 4_305_237_050,
+    "kv_update": 67_240_131,
+    "decode_paged": 4_305_384_404,
+    "decode_rope": 8_601_623_901,
+    "kv_update_rope": 75_523_328,
+    "decode_step": 4_306_766_830,
 }
 
 
