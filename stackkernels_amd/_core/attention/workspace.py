@@ -64,11 +64,12 @@ def bwd_workspace(dtype: torch.dtype, B: int, Hq: int, Hkv: int, Sq: int, Sk: in
 
     The most the call makes use of (``sk_attn_bwd_workspace_best``: row
     statistics, one chunk of the five-GEMM backward's dS tiles, at most
-    ``SK_BWD_DS_CAP_BYTES`` of them, and the partial sums of a split dK/dV);
-    if torch cannot allocate that, the size without the partial sums, then
-    the minimum (row statistics only), with which the call runs the
-    seven-GEMM backward: slower, and dK/dV summed in another order than a
-    split one sums them.
+    ``SK_BWD_DS_CAP_BYTES`` of them, and the partial sums of gradients split
+    over several workgroups, dK/dV and for fp32 dQ, at most
+    ``SK_PARTIALS_CAP_BYTES``); if torch cannot allocate that, the size
+    without the partial sums, then the minimum (row statistics only), with
+    which the call runs the seven-GEMM backward: slower, and those gradients
+    summed in one pass, another order than a split one's.
     """
     code = _lib.dtype_code(dtype)
     sizes = _bwd_workspace_bytes(code, B, Hq, Hkv, Sq, Sk, D, bool(is_causal))

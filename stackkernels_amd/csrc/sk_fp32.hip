@@ -723,9 +723,10 @@ hipError_t launch_bwd_prep(int dtype, const BwdParams& p, hipStream_t s) {
 // output block c holds head-dim columns DB*m + c.  Streamed tiles (32 rows)
 // keep 16-byte chunk c of row r at c ^ (r % 16), so the row-wise operand
 // reads (16 rows, one chunk each) and the column-piece reads (one row, 32
-// chunks) both hit distinct bank quads.  A workgroup is 4 waves, one per SIMD
-// (the resident operands and two accumulator sets exceed 256 registers), and
-// its tiles go through a 2-deep ring written by buffer_load ... lds, one
+// chunks) both hit distinct bank quads.  A workgroup is 4 waves: at DP = 128
+// one per SIMD (the resident operands and two accumulator sets exceed 256
+// registers), at DP = 64 two (dQ 202 registers, dK/dV 233, no spills).  Its
+// tiles go through a 2-deep ring written by buffer_load ... lds, one
 // barrier per step; a step is 192 (dQ) or 256 (dK/dV) MFMAs of 64 cycles per
 // wave, so one step of load look-ahead is ample.  P = exp2(S * scale * log2 e
 // - lse * log2 e) is set to 0 where the key is masked, past S_k, or the query
