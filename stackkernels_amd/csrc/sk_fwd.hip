@@ -53,9 +53,9 @@
 //   long rows do not trail at the end of the grid.  Under the causal mask a
 //   workgroup runs query blocks j and n-1-j back to back when the grid
 //   stays at two or more workgroups per CU, which evens out the work per
-//   workgroup and halves the per-item fixed cost; causal grids of half a round
-//   to two rounds of the chip start every head's heavy blocks before any light
-//   one (bf16, H_q = 32, H_kv = 8, D = 128, B = 2, S = 1,337, 704 workgroups: 54
+//   workgroup and halves the per-item fixed cost; causal grids of more than one
+//   workgroup per CU, up to two rounds, start every head's heavy blocks before
+//   any light one (bf16, H_q = 32, H_kv = 8, D = 128, B = 2, S = 1,337, 704 workgroups: 54
 //   us head-major, 43 so).
 #include <algorithm>
 #include <type_traits>
@@ -822,7 +822,10 @@ int fwd_pair_min(int dtype, int d, int64_t bh, int sq, int sk, bool causal) {
 // 8,000 (138 us, 132 with 2), where the grid or the merge leaves no gain.
 // A predicted gain under 15% is left alone (causal squares, whose blocks
 // differ: 1,000 x 1,000 at 8 heads 20 us either way), and from 384 query
-// blocks on (1.5 per CU) nothing is split.
+// blocks on (1.5 per CU) nothing is split.  Nor are, at D = 256 (one workgroup
+// per CU), causal grids of more than one round whose blocks differ (S_k < 2
+// S_q): the light ones fill in behind the heavy (264 blocks, 2,801 x 2,891 127
+// us whole, 186 in 4; 372, 3,879 x 4,223 247 and 275).
 // Where the group's heads share blocks of 128 rows to a gain (few queries per
 // head), a (batch, KV head)'s rows are packed, which also reads the keys once
 // per group: 8 rows of 35 queries, H_q = 64, H_kv = 8, 19,392 keys 532 us
@@ -854,6 +857,7 @@ FwdSplit fwd_key_splits(int dtype, int d, int B, int Hq, int Hkv, int sq, int sk
   const int group = Hq / Hkv;
   const int64_t whole = (int64_t)fwd_split_blocks(sq) * bh;
   const int64_t packed = (int64_t)fwd_split_blocks((int64_t)group * sq) * B * Hkv;
+  if (causal && d > 128 && whole > 256 && sk < 2 * (int64_t)sq) return out;
   const double tile_us = d <= 64 ? 0.5 : d <= 128 ? 1.0 : 1.15;
   const double tiles = (double)sk / (d <= 128 ? 64 : 32);
   const double merge_us = (double)bh * sq * d * 8 / 1.2e7 + 0.5;  // per split
@@ -950,16 +954,16 @@ KernelPlan plan_fwd_mfma(int dtype, const FwdParams& p, bool causal) {
 
 hipError_t launch_fwd_mfma(int dtype, const FwdParams& params, bool causal, hipStream_t s) {
   FwdParams p = params;
-  // Unpaired causal grids between half a round and two rounds of the chip:
-  // 4-21% on average over 80 shapes there.  Below, every block starts at once;
-  // above, later blocks fill in behind long ones anyway and head-major order
+  // Unpaired causal grids of more than one workgroup per CU, up to two rounds of
+  // the chip: 4-21% on average over 80 shapes there.  Below, no block waits or
+  // shares a CU (D = 256, 208 workgroups 3% slower heavy first); above, later blocks fill in behind long ones anyway and head-major order
   // keeps a head's K/V in one L2 (over 100 shapes from 2.5 rounds on neutral on
   // average, up to 6% slower heavy first: 24 heads on 2, B = 10, S = 1,011, D =
   // 64 63.9 us, 67.7).  Paired blocks carry equal work (B * H = 128, S = 4,096
   // 527 us, 575 with the blocks outermost).
   const int64_t wgs = (int64_t)p.n_items * p.B * p.Hq;
   const int slots = 256 * fwd_config(p.D, (int64_t)p.B * p.Hq, p.Sq, p.Sk, causal).occ;
-  p.heavy_first = causal && !p.pair_items && !p.part_o && 2 * wgs > slots && wgs <= 2 * slots;
+  p.heavy_first = causal && !p.pair_items && !p.part_o && wgs > 256 && wgs <= 2 * slots;
   const KernelPlan k = plan_fwd_mfma(dtype, p, causal);
   if (!k.fn) return hipErrorInvalidValue;
   return run_plan(k, &p, s);

@@ -45,6 +45,17 @@ def test_split_forward(dtype, b, hq, hkv, sq, sk, d, causal, packed):
     assert f["combine"]["grid"] == -(-b * hq * sq // f["combine"]["BLOCK_M"])
 
 
+@pytest.mark.parametrize("b,hq,hkv,sq,sk,split", [
+    (1, 12, 12, 2801, 2891, False),  # 264 blocks, just over a round
+    (1, 24, 2, 1330, 1330, False),
+    (1, 4, 4, 2048, 2048, True),     # 64 blocks
+    (1, 12, 12, 2801, 9000, True),   # blocks alike
+])
+def test_split_forward_d256_causal(b, hq, hkv, sq, sk, split):
+    f = _pick("flash_attn", "bfloat16", b, hq, hkv, sq, sk, 256, True)
+    assert (f["workspace_bytes"] > 0) == split
+
+
 def test_split_forward_f32():
     dims = ("float32", 2, 8, 8, 1024, 1024, 64, False)
     f = _pick("flash_attn", *dims)
