@@ -87,19 +87,19 @@ PEAK_NOTE = {
 # so these are recorded figures.  TRAFFIC_SOURCES_SHA256 is the digest of the
 # kernel sources (kernel_sources_digest) the counters were measured on; when
 # the sources differ, the line reports traffic null rather than a stale figure.
-TRAFFIC_SOURCES_SHA256 = "380e706a9f9ff00cc6737510addb9f5c4a9dcb38b77195f4b5061a0dbe89fb8d"
+TRAFFIC_SOURCES_SHA256 = "caf67ddc427234fcfa34719631437866058f68af6a620cbe94e3947be4e70ea7"
 HBM_TRAFFIC_BYTES = {
-    "fwd": 681_380_439,
-    "fwd_long": 843_569_282,
-    "fwdbwd": 4_537_210_787,
-    "decode": 8_601_609_521,
-    "decode_mqa": 573_052_296,
-    "decode_varlen": 4_305_237_050,
-    "kv_update": 67_240_131,
-    "decode_paged": 4_305_384_404,
-    "decode_rope": 8_601_623_901,
-    "kv_update_rope": 75_523_328,
-    "decode_step": 4_306_766_830,
+    "fwd": 680_866_517,
+    "fwd_long": 844_129_003,
+    "fwdbwd": 4_537_413_755,
+    "decode": 8_601_609_571,
+    "decode_mqa": 573_052_245,
+    "decode_varlen": 4_305_237_180,
+    "kv_update": 67_240_132,
+    "decode_paged": 4_305_384_459,
+    "decode_rope": 8_601_623_879,
+    "kv_update_rope": 75_523_343,
+    "decode_step": 4_306_766_909,
 }
 
 
